@@ -10,8 +10,8 @@
 // grid): a static split with no device work counter, no atomics and no
 // barrier inside the item loop, so every workgroup's loop ends after a fixed
 // number of items.
-// Under the wave-coherent schedule, -m 0 to -m 5 views without lighting run
-// kernels_wave.hip's render_views_wave and render_views_wave_persistent
+// Under the wave-coherent schedule, -m 0 to -m 5 views run wave_paths.hpp's
+// render_views_wave and (without shading) render_views_wave_persistent
 // instead, with the same items and ids.
 // No reference counterpart: the reference renders one camera per owlLaunch2D
 // (renderer.cpp:949).
@@ -224,7 +224,7 @@ RenderFn select_views(int mode, int dtype, bool count, bool lit, bool wide) {
 
 // the extended kernel: shadow rays, gradient shading or denoiser inputs
 bool is_lit(const RenderParams& p) {
-  return p.fr.sh.shadows != 0 || p.fr.sh.gradient != 0 || p.fr.aov != nullptr;
+  return is_shaded(p) || p.fr.aov != nullptr;
 }
 
 hipError_t prepare(RenderFn f, size_t lds) {
@@ -239,14 +239,18 @@ namespace {
 bool wide_views(const RenderParams& p, int dtype) {
   return p.vol.channels <= 4 && (dtype == MDWT_DT_U8 || dtype == MDWT_DT_U16);
 }
-// batched views on the wave-coherent kernels (schedule 1 where it applies)
+// batched views on the wave-coherent kernels (schedule 1 where it applies; the
+// persistent form has no shaded instance)
 bool wave_views(const RenderParams& p, int mode, bool count) {
-  return p.fr.schedule == 1 && wave_schedule_applies(p, mode, count, is_lit(p));
+  return p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
+}
+bool wave_persistent(const RenderParams& p, int mode) {
+  return wave_views(p, mode, false) && !is_shaded(p);
 }
 }  // namespace
 
 hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int dtype, int* out) {
-  const bool wave = wave_views(p, mode, false);
+  const bool wave = wave_persistent(p, mode);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
   const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 2)
                           : select_persistent(mode, dtype, is_lit(p), wide_views(p, dtype));
@@ -258,7 +262,7 @@ hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int d
 hipError_t launch_views_persistent(const RenderParams& p, int mode, int dtype, int grid,
                                    hipStream_t s) {
   if (p.fr.n_items <= 0 || grid <= 0 || !p.fr.work) return hipErrorInvalidValue;
-  const bool wave = wave_views(p, mode, false);
+  const bool wave = wave_persistent(p, mode);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
   const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 2)
                           : select_persistent(mode, dtype, is_lit(p), wide_views(p, dtype));

@@ -265,7 +265,7 @@ size_t render_lds_bytes(const RenderParams& p) {
 namespace {
 // the extended kernel: shadow rays, gradient shading or denoiser inputs
 bool is_lit(const RenderParams& p) {
-  return p.fr.sh.shadows != 0 || p.fr.sh.gradient != 0 || p.fr.aov != nullptr;
+  return is_shaded(p) || p.fr.aov != nullptr;
 }
 // Six waves per SIMD (with scratch spills) pay on at most four channels of
 // 1- or 2-byte voxels: -m 2 0.334 -> 0.317 ms on four 256^3 u8 channels. On
@@ -287,7 +287,7 @@ hipError_t prepare(RenderFn f, size_t lds) {
 
 hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s) {
   const bool lit = is_lit(p);
-  const bool wave = p.fr.schedule == 1 && wave_schedule_applies(p, mode, count, lit);
+  const bool wave = p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
   const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 0)
                           : select_render(mode, dtype, count, lit, six_waves(p, dtype));

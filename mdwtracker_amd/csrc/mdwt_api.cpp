@@ -559,13 +559,9 @@ int make_bricks(mdwt_renderer* h) {
 }
 
 // The wave-coherent schedule covers the tracking modes -m 0 to -m 5; the ray
-// marchers, shadow rays, gradient shading and the
-// frames that write auxiliary outputs (the first aov_frames of an
-// accumulation) run the thread-per-pixel kernel (the launcher checks the same
-// conditions). Both give the same image bits, so an accumulation may switch.
+// marchers run the thread-per-pixel kernel (the launcher checks the same
+// conditions). Both give the same image bits.
 int eff_schedule(const mdwt_renderer* h) {
-  if (h->sh.shadows || h->sh.gradient) return 0;
-  if (h->aov_on && (h->aov_frames == 0 || h->accum_id < uint32_t(h->aov_frames))) return 0;
   return (h->mode >= 0 && h->mode <= 5) ? h->schedule : 0;
 }
 

@@ -9,11 +9,15 @@ namespace mdwt {
 
 // host stub of a frame kernel
 using RenderFn = void (*)(RenderParams);
-// wave-coherent frame kernels (kernels_wave.hip, schedule 1): -m 0 to -m 5 on
-// at most twelve channels, no lighting, not the counting pass; form 0 one view,
-// 1 batched views in one launch, 2 batched views in a persistent launch
-bool wave_schedule_applies(const RenderParams& p, int mode, bool count, bool lit);
+// gradient shading or shadow rays
+inline bool is_shaded(const RenderParams& p) { return p.fr.sh.shadows != 0 || p.fr.sh.gradient != 0; }
+// wave-coherent frame kernels (kernels_wave.hip, and kernels_wave_lit.hip with
+// shading; schedule 1): -m 0 to -m 5 on at most twelve channels, not the
+// counting pass; form 0 one view, 1 batched views in one launch, 2 batched
+// views in a persistent launch (not with shading)
+bool wave_schedule_applies(const RenderParams& p, int mode, bool count);
 RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form);
+RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int form);
 // dynamic LDS of a wave-coherent launch (transfer-function opacities)
 size_t wave_lds_bytes(const RenderParams& p);
 

@@ -84,7 +84,7 @@ struct FrameParams {
   unsigned long long* counters;  // samples, visits, rejections, rays
   const uint32_t* block_order;   // (bx | by << 16) per 16x16 pixel block, Hilbert order
   int n_blocks;
-  int schedule;  // 0: one thread per pixel, 1: wave-coherent (-m 0 to -m 5, no lighting)
+  int schedule;  // 0: one thread per pixel, 1: wave-coherent (-m 0 to -m 5)
   // cost-sorted order: wall-clock ticks (100 MHz) of each wave, indexed by
   // waves_per_block * (position in block_order) + wave; nullptr = not recorded
   uint32_t* wave_cost;

@@ -584,16 +584,18 @@ __device__ __forceinline__ void trace_mode(const Ctx<DT>& X, const GridRay& g, f
 }
 
 // Gradient (Blinn-Phong) shading of a Woodcock hit, deviceCode.cu:326-381,
-// with the hit channel's material. pow is exp(y log x) (ppowf).
-template <int DT>
+// with the hit channel's material. pow is exp(y log x) (ppowf). gradient(tex,
+// step, channel) is Ctx::gradient or the same values from another table.
+template <int DT, class Gradient>
 __device__ void shade_gradient(const RenderParams& P, const Ctx<DT>& X, V3 org, V3 dir,
-                               const HitRec& h, float& diffuse, float& specular) {
+                               const HitRec& h, float& diffuse, float& specular,
+                               const Gradient& gradient) {
   if (!(sqrtf(h.r * h.r + h.g * h.g + h.b * h.b) > 0.001f)) return;
   const int m = h.channel;
   const V3 blo = load3(P.vol.blo), bhi = load3(P.vol.bhi);
   const V3 w2u = v3(1.f / (bhi.x - blo.x), 1.f / (bhi.y - blo.y), 1.f / (bhi.z - blo.z));
   const V3 tex = (org + h.tHit * dir) * w2u;
-  const V3 grad = X.gradient(tex, P.fr.sh.grad_step[m], m);
+  const V3 grad = gradient(tex, P.fr.sh.grad_step[m], m);
   if (sqrtf(dot3(grad, grad)) > 1e-6f) {
     const V3 N = normalize3(v3(-grad.x, -grad.y, -grad.z));
     const V3 L = normalize3(load3(P.fr.sh.light_dir));
@@ -690,7 +692,9 @@ __device__ __forceinline__ void render_block(const RenderParams& P, const Ctx<DT
         rd = v3(-P.fr.sh.light_dir[0], -P.fr.sh.light_dir[1], -P.fr.sh.light_dir[2]);
         rng.init(V.seed, pixel, V.frame_id, uint32_t(s), 1u);
       }
-      if (LIT && !h.missed && P.fr.sh.gradient) shade_gradient(P, X, org, dir, h, diffuse, specular);
+      if (LIT && !h.missed && P.fr.sh.gradient)
+        shade_gradient(P, X, org, dir, h, diffuse, specular,
+                       [&](V3 tex, float eps, int m) { return X.gradient(tex, eps, m); });
     } else {
       float t0, t1;
       if (clip_root(org, dir, blo, bhi, t0, t1)) {

@@ -1,0 +1,66 @@
+"""The default frame kernels against the thread-per-pixel schedule (itself
+bit-exact against the oracle, test_gpu_parity.py): identical images, second
+moments and auxiliary buffers at the sizes and options where the paths differ."""
+import numpy as np
+import pytest
+
+from mdwtracker_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def capi():
+    from mdwtracker_amd import capi
+    return capi
+
+
+def volume(channels, dtype, dims=(37, 29, 42), seed=5):
+    """(channel volumes (nz, ny, nx), transfer functions) of a small ragged scene."""
+    rng = np.random.default_rng(seed)
+    vols, tfs = [], []
+    for c in range(channels):
+        v = scenes.normalise(scenes.noise_blob_volume(dims[::-1], 6, rng))
+        vols.append(scenes.quantize_u8(v) if dtype == np.uint8 else
+                    np.rint(v * 65535).astype(np.uint16) if dtype == np.uint16 else v.astype(dtype))
+        tfs.append(scenes.piecewise_tf(6, rng, c / channels, x_lo=0.2, clear_first=True))
+    return vols, tfs
+
+
+def renderer(capi, vols, tfs, mode, size, spp, schedule, mc=(5, 4, 6), opacity=0.08):
+    r = capi.MdwtRenderer(0)
+    for v in vols:
+        r.push_channel(v)
+    r.init(mode, mc, False)
+    r.set_schedule(schedule)
+    for c, t in enumerate(tfs):
+        r.set_tf(c, t, opacity, (0.0, 1.0))
+    r.set_frame(size[0], size[1], spp, True, (0.1, 0.2, 0.3))
+    r.set_camera(*scenes.orbit_camera(1.6))
+    r.set_seed(11)
+    return r
+
+
+@pytest.mark.parametrize("channels,dtype", [(1, np.uint16), (3, np.uint8), (10, np.float32)])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4, 5])
+def test_shading_and_aov_on_both_schedules(capi, mode, channels, dtype):
+    """Gradient shading, shadow rays and the denoiser's buffers, alone and
+    together, on a frame whose sides are not multiples of 8."""
+    vols, tfs = volume(channels, dtype)
+    for shadows, gradient, aov in ((1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)):
+        out = []
+        for schedule in (0, 1):
+            print(f"[paths] mode {mode} channels {channels} shadows {shadows} gradient {gradient} "
+                  f"aov {aov} schedule {schedule}", flush=True)
+            r = renderer(capi, vols, tfs, mode, (75, 51), 2, schedule)
+            r.set_light((0.3, -1.0, 0.2), bool(shadows), bool(gradient))
+            r.set_moments(True)
+            r.set_aov(bool(aov))
+            r.set_aov_frames(2)
+            r.render(3)
+            got = list(r.read_accum(with_m2=True)) + ([r.read_aov()] if aov else [])
+            assert got[0][..., :3].std() > 0.01
+            out.append([g.view(np.uint32) for g in got])
+            r.close()
+        for a, b in zip(*out):
+            np.testing.assert_array_equal(a, b)
