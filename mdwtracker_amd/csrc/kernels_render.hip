@@ -289,10 +289,16 @@ hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count,
   const bool lit = is_lit(p);
   const bool wave = p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
-  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 0)
+  if (p.fr.team_frames > 0 && !wave) return hipErrorInvalidValue;
+  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, p.fr.team_frames > 0 ? 3 : 0)
                           : select_render(mode, dtype, count, lit, six_waves(p, dtype));
   const hipError_t e = prepare(f, lds);
   if (e != hipSuccess) return e;
+  if (p.fr.team_frames > 0) {  // one workgroup per 8x8 quad
+    hipLaunchKernelGGL(f, dim3(unsigned(p.fr.n_blocks) * unsigned(p.fr.bw * p.fr.bh / 64)),
+                       dim3(kThreads), lds, s, p);
+    return hipGetLastError();
+  }
   // one workgroup per pixel block
   hipLaunchKernelGGL(f, dim3(unsigned(p.fr.n_blocks)), dim3(unsigned(p.fr.bw * p.fr.bh)), lds, s, p);
   return hipGetLastError();

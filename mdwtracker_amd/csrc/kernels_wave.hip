@@ -5,12 +5,16 @@
 namespace mdwt {
 namespace {
 
-// form: 0 one view, 1 batched views (one launch), 2 batched views (persistent)
+// form: 0 one view, 1 batched views (one launch), 2 batched views (persistent),
+// 3 one view, several frames
 template <int MODE, int DT, bool WIDE>
 RenderFn wave_fn_form(int form) {
-  return form == 0 ? render_wave<MODE, DT, WIDE, false>
-                   : (form == 1 ? render_views_wave<MODE, DT, WIDE, false>
-                                : render_views_wave_persistent<MODE, DT, WIDE>);
+  switch (form) {
+    case 0: return render_wave<MODE, DT, WIDE, false>;
+    case 1: return render_views_wave<MODE, DT, WIDE, false>;
+    case 2: return render_views_wave_persistent<MODE, DT, WIDE>;
+    default: return render_wave_team<MODE, DT, WIDE, false>;
+  }
 }
 template <int MODE, bool WIDE>
 RenderFn wave_fn(int dtype, int form) {

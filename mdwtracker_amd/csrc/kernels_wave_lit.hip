@@ -16,7 +16,11 @@ namespace {
 
 template <int MODE, int DT, bool WIDE>
 RenderFn lit_fn_form(int form) {
-  return form == 0 ? render_wave<MODE, DT, WIDE, true> : render_views_wave<MODE, DT, WIDE, true>;
+  switch (form) {
+    case 0: return render_wave<MODE, DT, WIDE, true>;
+    case 1: return render_views_wave<MODE, DT, WIDE, true>;
+    default: return render_wave_team<MODE, DT, WIDE, true>;
+  }
 }
 template <int MODE, bool WIDE>
 RenderFn lit_fn(int dtype, int form) {

@@ -605,10 +605,27 @@ mdwt::RenderParams render_params(const mdwt_renderer* h) {
   return p;
 }
 
-// One frame launch (the counting pass always runs the thread-per-pixel kernel).
-int launch_frame(mdwt_renderer* h, bool count) {
+// Frames of the next launch when `left` are to be rendered: several by the
+// team kernel (see team_quad in wave_paths.hpp), whose four waves take four
+// draws (samples) at a time, or 0 for one frame by the one-frame kernels. Only
+// whole rounds of four draws: in a partial one, waves hold their workgroup's
+// LDS and do nothing. About 32 draws: longer launches gained under 1 %.
+constexpr int kTeamDraws = 32;
+int team_frames(const mdwt_renderer* h, const mdwt::RenderParams& p, int left) {
+  if (p.fr.schedule != 1 || !mdwt::wave_schedule_applies(p, h->mode, false)) return 0;
+  // the auxiliary buffers stop at their own frame count
+  if (p.fr.aov && h->aov_frames) left = std::min(left, int(uint32_t(h->aov_frames) - h->accum_id));
+  const int step = h->spp % 4 == 0 ? 1 : (h->spp % 2 == 0 ? 2 : 4);
+  return std::min(left, std::max(step, kTeamDraws / h->spp)) / step * step;
+}
+
+// One frame launch (the counting pass always runs the thread-per-pixel kernel),
+// or of several (*frames, at most `left`) by the team kernel.
+int launch_frame(mdwt_renderer* h, bool count, int left = 1, int* frames = nullptr) {
   mdwt::RenderParams p = render_params(h);
   if (count) p.fr.wave_cost = nullptr;
+  p.fr.team_frames = count ? 0 : team_frames(h, p, left);
+  if (frames) *frames = std::max(p.fr.team_frames, 1);
   HIPCHK(h, mdwt::launch_render(p, h->mode, h->dtype, count, h->stream));
   if (p.fr.wave_cost) h->cost_ready = true;
   return MDWT_OK;
@@ -1072,11 +1089,13 @@ int mdwt_render(mdwt_renderer* h, int n_frames, float* ms_out) {
     h->need_resort = false;
   }
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
-  for (int f = 0; f < n_frames; ++f) {
-    rc = launch_frame(h, false);
+  for (int f = 0; f < n_frames;) {
+    int n = 1;
+    rc = launch_frame(h, false, n_frames - f, &n);
     if (rc != MDWT_OK) return rc;
-    h->accum_id++;
-    h->frame_id++;
+    h->accum_id += uint32_t(n);
+    h->frame_id += uint32_t(n);
+    f += n;
   }
   HIPCHK(h, hipEventRecord(h->ev1, h->stream));
   HIPCHK(h, hipEventSynchronize(h->ev1));

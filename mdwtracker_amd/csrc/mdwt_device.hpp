@@ -264,23 +264,18 @@ __device__ __forceinline__ float tf_lerp_alpha(const float4* tab, int n, float u
 }
 
 // --------------------------------------------------------- voxel fetch -----
+// a voxel's stored bits, and their value
 template <int DT>
-__device__ __forceinline__ float fetch_raw(const uint8_t* base, uint32_t i);
-template <>
-__device__ __forceinline__ float fetch_raw<MDWT_DT_U8>(const uint8_t* base, uint32_t i) {
-  return float(base[i]);
+__device__ __forceinline__ uint32_t fetch_bits(const uint8_t* base, uint32_t i) {
+  if (DT == MDWT_DT_U8) return base[i];
+  if (DT == MDWT_DT_F32) return reinterpret_cast<const uint32_t*>(base)[i];
+  return reinterpret_cast<const uint16_t*>(base)[i];
 }
-template <>
-__device__ __forceinline__ float fetch_raw<MDWT_DT_U16>(const uint8_t* base, uint32_t i) {
-  return float(reinterpret_cast<const uint16_t*>(base)[i]);
-}
-template <>
-__device__ __forceinline__ float fetch_raw<MDWT_DT_F16>(const uint8_t* base, uint32_t i) {
-  return float(reinterpret_cast<const _Float16*>(base)[i]);
-}
-template <>
-__device__ __forceinline__ float fetch_raw<MDWT_DT_F32>(const uint8_t* base, uint32_t i) {
-  return reinterpret_cast<const float*>(base)[i];
+template <int DT>
+__device__ __forceinline__ float voxel_value(uint32_t bits) {
+  if (DT == MDWT_DT_F32) return __uint_as_float(bits);
+  if (DT == MDWT_DT_F16) return float(__builtin_bit_cast(_Float16, uint16_t(bits)));
+  return float(bits);
 }
 
 // ------------------------------------------------------------- DDA ---------

@@ -14,7 +14,8 @@ inline bool is_shaded(const RenderParams& p) { return p.fr.sh.shadows != 0 || p.
 // wave-coherent frame kernels (kernels_wave.hip, and kernels_wave_lit.hip with
 // shading; schedule 1): -m 0 to -m 5 on at most twelve channels, not the
 // counting pass; form 0 one view, 1 batched views in one launch, 2 batched
-// views in a persistent launch (not with shading)
+// views in a persistent launch (not with shading), 3 p.fr.team_frames frames of
+// one view in one launch
 bool wave_schedule_applies(const RenderParams& p, int mode, bool count);
 RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form);
 RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int form);

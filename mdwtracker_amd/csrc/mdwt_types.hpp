@@ -88,6 +88,7 @@ struct FrameParams {
   // cost-sorted order: wall-clock ticks (100 MHz) of each wave, indexed by
   // waves_per_block * (position in block_order) + wave; nullptr = not recorded
   uint32_t* wave_cost;
+  int team_frames;  // 0: one frame; n: the frames a launch of the team kernel renders
   int bw, bh;  // pixel block of a workgroup: 8x8, 16x8 or 16x16 (bw*bh/64 waves of 8x8 pixels)
   // batched views (views == nullptr: the single view described above). An
   // item is one pixel block of one view (view << 20 | by << 10 | bx); launch

@@ -64,15 +64,30 @@ struct Ctx {
   }
 
   // sampleVolumeTexture (deviceCode.cu:122-132): NaN outside [0,1]^3, else
-  // clamp-to-edge trilinear at texel coordinate p*N - 0.5.
-  __device__ __forceinline__ float sample(V3 p, int c) const {
-    if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
-      return qnan();
+  // clamp-to-edge trilinear at texel coordinate p*N - 0.5. In two parts, so
+  // that a caller can do other work while the voxels are on their way:
+  // corners() issues the eight loads (indices are clamped, so they are in
+  // bounds for every p, NaN included), trilinear() waits for them.
+  struct Corners {
+    uint32_t b000, b100, b010, b110, b001, b101, b011, b111;  // stored bits
+    float fx, fy, fz;
+    bool inside;
+    // the point up to which other work may run while the loads are in flight
+    __device__ __forceinline__ void arrived() {
+      asm volatile("" : "+v"(b000), "+v"(b100), "+v"(b010), "+v"(b110), "+v"(b001), "+v"(b101),
+                        "+v"(b011), "+v"(b111));
+    }
+  };
+  __device__ __forceinline__ Corners corners(V3 p, int c) const {
+    Corners k;
+    k.inside = !(p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f);
     const float x = p.x * float(nx) - 0.5f;
     const float y = p.y * float(ny) - 0.5f;
     const float z = p.z * float(nz) - 0.5f;
     const float flx = floorf(x), fly = floorf(y), flz = floorf(z);
-    const float fx = x - flx, fy = y - fly, fz = z - flz;
+    k.fx = x - flx;
+    k.fy = y - fly;
+    k.fz = z - flz;
     const uint32_t x0 = uint32_t(clamp_index(flx, nx)), x1 = uint32_t(clamp_index_plus1(flx, nx));
     const uint32_t y0 = uint32_t(clamp_index(fly, ny)), y1 = uint32_t(clamp_index_plus1(fly, ny));
     const uint32_t z0 = uint32_t(clamp_index(flz, nz)), z1 = uint32_t(clamp_index_plus1(flz, nz));
@@ -88,18 +103,43 @@ struct Ctx {
     const uint32_t az0 = (__umul24(z0 >> 2, nbxy) << 6) | ((z0 & 3u) << 4);
     const uint32_t az1 = (__umul24(z1 >> 2, nbxy) << 6) | ((z1 & 3u) << 4);
     const uint32_t r00 = ay0 + az0, r10 = ay1 + az0, r01 = ay0 + az1, r11 = ay1 + az1;
-    const float v000 = fetch_raw<DT>(base, r00 + ax0), v100 = fetch_raw<DT>(base, r00 + ax1);
-    const float v010 = fetch_raw<DT>(base, r10 + ax0), v110 = fetch_raw<DT>(base, r10 + ax1);
-    const float v001 = fetch_raw<DT>(base, r01 + ax0), v101 = fetch_raw<DT>(base, r01 + ax1);
-    const float v011 = fetch_raw<DT>(base, r11 + ax0), v111 = fetch_raw<DT>(base, r11 + ax1);
-    const float c00 = v000 + fx * (v100 - v000);
-    const float c10 = v010 + fx * (v110 - v010);
-    const float c01 = v001 + fx * (v101 - v001);
-    const float c11 = v011 + fx * (v111 - v011);
-    const float c0 = c00 + fy * (c10 - c00);
-    const float c1 = c01 + fy * (c11 - c01);
-    const float r = c0 + fz * (c1 - c0);
-    return r * scale + offset;
+    k.b000 = fetch_bits<DT>(base, r00 + ax0);
+    k.b100 = fetch_bits<DT>(base, r00 + ax1);
+    k.b010 = fetch_bits<DT>(base, r10 + ax0);
+    k.b110 = fetch_bits<DT>(base, r10 + ax1);
+    k.b001 = fetch_bits<DT>(base, r01 + ax0);
+    k.b101 = fetch_bits<DT>(base, r01 + ax1);
+    k.b011 = fetch_bits<DT>(base, r11 + ax0);
+    k.b111 = fetch_bits<DT>(base, r11 + ax1);
+    return k;
+  }
+  // TOGETHER false: for callers with several channels in flight.
+  template <bool TOGETHER = true>
+  __device__ __forceinline__ float trilinear(Corners k) const {
+    // All eight loads in flight before the first value is used: left to itself
+    // the scheduler saves address registers by issuing one load, waiting for it
+    // and reusing its address pair, in some instances and not in others.
+    if (TOGETHER)
+      asm("" : "+v"(k.b000), "+v"(k.b100), "+v"(k.b010), "+v"(k.b110), "+v"(k.b001), "+v"(k.b101),
+               "+v"(k.b011), "+v"(k.b111));
+    const float v000 = voxel_value<DT>(k.b000), v100 = voxel_value<DT>(k.b100);
+    const float v010 = voxel_value<DT>(k.b010), v110 = voxel_value<DT>(k.b110);
+    const float v001 = voxel_value<DT>(k.b001), v101 = voxel_value<DT>(k.b101);
+    const float v011 = voxel_value<DT>(k.b011), v111 = voxel_value<DT>(k.b111);
+    const float c00 = v000 + k.fx * (v100 - v000);
+    const float c10 = v010 + k.fx * (v110 - v010);
+    const float c01 = v001 + k.fx * (v101 - v001);
+    const float c11 = v011 + k.fx * (v111 - v011);
+    const float c0 = c00 + k.fy * (c10 - c00);
+    const float c1 = c01 + k.fy * (c11 - c01);
+    const float r = c0 + k.fz * (c1 - c0);
+    return k.inside ? r * scale + offset : qnan();
+  }
+  template <bool TOGETHER = true>
+  __device__ __forceinline__ float sample(V3 p, int c) const {
+    if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
+      return qnan();
+    return trilinear<TOGETHER>(corners(p, c));
   }
 
   // transferFunction (deviceCode.cu:27-42), opacity only; colour is looked

@@ -350,10 +350,10 @@ __device__ float4 blend_channels(const Ctx<DT>& X, V3 p) {
   const bool pre = MODE >= 6 && X.C <= 4;
   float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
   if (pre) {
-    v4.x = X.sample(p, 0);
-    if (X.C > 1) v4.y = X.sample(p, 1);
-    if (X.C > 2) v4.z = X.sample(p, 2);
-    if (X.C > 3) v4.w = X.sample(p, 3);
+    v4.x = X.template sample<false>(p, 0);
+    if (X.C > 1) v4.y = X.template sample<false>(p, 1);
+    if (X.C > 2) v4.z = X.template sample<false>(p, 2);
+    if (X.C > 3) v4.w = X.template sample<false>(p, 3);
   }
   auto value = [&](int c) { return pre ? pick(v4, c) : X.sample(p, c); };
   if (MODE == 6) {

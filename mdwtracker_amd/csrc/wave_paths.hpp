@@ -228,13 +228,25 @@ __device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& 
                                           const Record& R, const WaveRay& Y, uint32_t j, float t,
                                           float m, float& tn) {
   const float4 ow = Y.org_w2g, dg = Y.dir_g2w;
+  const float tWorld = t * dg.w;
+  const V3 xT = (v3(ow.x, ow.y, ow.z) + tWorld * v3(dg.x, dg.y, dg.z)) * w2u;
+  // the (first) channel's voxels are requested before the pair is drawn: its
+  // Philox block runs while they are on their way (1 to 2 % of a frame; the
+  // compiler otherwise moves the block behind the wait)
+  [[maybe_unused]] typename Ctx<DT>::Corners k0;
+  if constexpr (MODE <= 3) {
+    k0 = X.corners(xT, MODE == 3 ? 0 : c);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   uint32_t w[4];
   philox(D.frame, D.sample, 1u + (((R.vl & kVisitMask) << 4) | uint32_t(c)), D.stream | ((j >> 1) << 1),
          D.seed, Y.pixel, w);
+  if constexpr (MODE <= 3) {  // in this order: loads, block, values
+    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+    k0.arrived();
+  }
   const float thr = to_unit((j & 1u) ? w[2] : w[0]) * m;
   const float un = to_unit((j & 1u) ? w[3] : w[1]);
-  const float tWorld = t * dg.w;
-  const V3 xT = (v3(ow.x, ow.y, ow.z) + tWorld * v3(dg.x, dg.y, dg.z)) * w2u;
   if (MODE == 4 || MODE == 5) {
     // blendDTCH (deviceCode.cu:972-1065): one blended sample of all channels
     const float4 sb = blend_channels<MODE, DT>(X, xT);
@@ -247,7 +259,7 @@ __device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& 
     // their opacity off the threshold until one exceeds what is left
     float th = thr;
     for (int k = 0; k < X.C; ++k) {
-      const float value = X.sample(xT, k);
+      const float value = k == 0 ? X.trilinear(k0) : X.sample(xT, k);
       if (value != value) continue;
       const float a = alpha_lookup(s_a, X.chtf[k], value);
       if (a > 0.0f && th < a) {
@@ -257,7 +269,7 @@ __device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& 
       th -= a;
     }
   } else {
-    const float value = X.sample(xT, c);
+    const float value = X.trilinear(k0);
     bool hit = false;
     if (!(value != value)) {
       const float a = alpha_lookup(s_a, X.chtf[c], value);
@@ -621,13 +633,117 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
   return hit;
 }
 
-// The 8x8 pixel quad of this wave in pixel block (bx, by) of view V (a
-// workgroup's bw x bh block has one quad per wave). WIDE: more than four
-// channels (-m 2), drawn in groups of four; a separate instantiation, since
-// the group loop's code in the four-channel kernel cost it 3%. LIT: gradient
-// shading and shadow rays, as render_block (render_paths.hpp) does them: the
-// shadow ray of every lane that hit runs through the same tracking rounds
+// One sample of the wave's 8x8 pixels (lane: pixel (px, py), index pixel, of
+// view V): the camera ray tracked to its first event, shaded. The lane's
+// contribution to its pixel's sums is returned (composite_sample on empty
+// sums); h is the hit for the auxiliary buffers. WIDE: more than four channels
+// (-m 2), drawn in groups of four; a separate instantiation, since the group
+// loop's code in the four-channel kernel cost it 3%. LIT: gradient shading and
+// shadow rays, as render_block (render_paths.hpp) does them: the shadow ray of
+// every lane that hit runs through the same tracking rounds
 // (deviceCode.cu:383-403), on stream 1.
+template <int MODE, int DT, bool WIDE, bool LIT>
+__device__ __forceinline__ float4 trace_sample(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+                                               const float* s_alpha, const ViewCtx& V,
+                                               uint32_t frame_id, int s, int px, int py, bool valid,
+                                               uint32_t pixel, V3 w2u, HitRec& h) {
+  const int lane = threadIdx.x & 63;
+  const V3 blo = load3(P.vol.blo), bhi = load3(P.vol.bhi);
+  Draw D = {frame_id, uint32_t(s), V.seed, 0u};
+  // ---- the camera ray (mainRG, deviceCode.cu:293-321)
+  V3 org, dir;
+  {
+    Rng rng;
+    rng.init(V.seed, pixel, frame_id, uint32_t(s), 0u);
+    float jx, jy;
+    rng.jitter2(P.fr.jitter2d != 0, jx, jy);
+    camera_ray(*V.cam, px, py, V.W, V.H, jx, jy, org, dir);
+  }
+  h.missed = true;
+  h.a = 1.f;
+  h.channel = 0;
+  h.tHit = 0.f;
+  h.r = h.g = h.b = 0.f;
+  float diffuse = 1.0f, specular = 0.0f, shadow = 1.0f;
+  V3 ro = org, rd = dir;
+  bool want = valid;
+  for (int pass = 0; pass < (LIT ? 2 : 1); ++pass) {
+    // the program's grid ray
+    Dda d;
+    bool alive = false;
+    {
+      float c0, c1;
+      WaveRay Y;
+      Y.org_w2g = make_float4(ro.x, ro.y, ro.z, 0.f);
+      Y.dir_g2w = make_float4(rd.x, rd.y, rd.z, 0.f);
+      Y.tend = 0.f;
+      Y.idw = 0.f;
+      if (want && clip_root(ro, rd, blo, bhi, c0, c1)) {
+        const GridRay g = make_grid_ray(ro, rd, blo, bhi, X.mx, X.my, X.mz);
+        alive = d.begin(g.org, g.dir, 1e20f, X.mx, X.my, X.mz);
+        Y.org_w2g.w = g.worldToGridT;
+        Y.dir_g2w.w = g.gridToWorldT;
+        Y.tend = c1;
+        Y.idw = 1.0f / (X.dt * g.worldToGridT);
+      }
+      Y.pixel = pixel;
+      Y.mask = (1u << X.C) - 1u;
+      L.ray[lane] = Y;
+    }
+    int hit_c = 0;
+    float hit_t = 0.f;
+    const bool hit = track_rays<MODE, DT, WIDE>(P, X, L, s_alpha, w2u, D, d, alive, hit_c, hit_t);
+    if (LIT && pass == 1) {
+      if (want) shadow = (1.f - P.fr.ambient) * (1.f - (hit ? 1.0f : 0.0f));
+      break;
+    }
+    // ---- the hit's colour
+    h.missed = !hit;
+    if (hit) {
+      const WaveRay& Y = L.ray[lane];
+      const float tWorld = hit_t * Y.dir_g2w.w;
+      const V3 xT = (v3(Y.org_w2g.x, Y.org_w2g.y, Y.org_w2g.z) +
+                     tWorld * v3(Y.dir_g2w.x, Y.dir_g2w.y, Y.dir_g2w.z)) * w2u;
+      if (MODE == 4 || MODE == 5) {
+        // the blended sample's colour; the hit keeps channel 0
+        const float4 sb = blend_channels<MODE, DT>(X, xT);
+        h.r = sb.x;
+        h.g = sb.y;
+        h.b = sb.z;
+      } else {
+        float r2;
+        (void)X.tf_alpha(X.sample(xT, hit_c), hit_c, r2);
+        X.tf_rgb(r2, hit_c, h);
+        h.channel = hit_c;
+      }
+      h.tHit = tWorld;
+    }
+    if (!LIT) break;
+    if (hit && P.fr.sh.gradient)
+      shade_gradient(P, X, org, dir, h, diffuse, specular, [&](V3 tex, float eps, int m) {
+        return opacity_gradient(X, s_alpha, tex, eps, m);
+      });
+    if (!P.fr.sh.shadows || __ballot(hit) == 0ull) break;
+    wave_sync();
+    want = hit;
+    ro = org + h.tHit * dir;
+    rd = v3(-P.fr.sh.light_dir[0], -P.fr.sh.light_dir[1], -P.fr.sh.light_dir[2]);
+    D.stream = 1u;
+  }
+  // ---- shade and composite the sample (deviceCode.cu:411-433)
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  composite_sample(P, !h.missed, h.r, h.g, h.b, h.a, diffuse, specular, shadow, h.channel, o.x, o.y,
+                   o.z, o.w);
+  return o;
+}
+
+__device__ __forceinline__ V3 world_to_unit(const RenderParams& P) {
+  const V3 ext = load3(P.vol.bhi) - load3(P.vol.blo);
+  return v3(1.f / ext.x, 1.f / ext.y, 1.f / ext.z);
+}
+
+// The 8x8 pixel quad of this wave in pixel block (bx, by) of view V (a
+// workgroup's bw x bh block has one quad per wave), one frame.
 template <int MODE, int DT, bool WIDE, bool LIT>
 __device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
                                            const float* s_alpha, const ViewCtx& V, int bx, int by) {
@@ -637,104 +753,133 @@ __device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>&
   const int py = by * P.fr.bh + (wave >> qs) * 8 + (lane >> 3);
   const bool valid = px < V.W && py < V.H;
   const uint32_t pixel = valid ? uint32_t(px) + uint32_t(V.W) * uint32_t(py) : 0u;
-  const V3 blo = load3(P.vol.blo), bhi = load3(P.vol.bhi);
-  const V3 ext = bhi - blo;
-  const V3 w2u = v3(1.f / ext.x, 1.f / ext.y, 1.f / ext.z);
-  const uint32_t all_ch = (1u << X.C) - 1u;
-
+  const V3 w2u = world_to_unit(P);
   float fr = 0.f, fg = 0.f, fb = 0.f, fa = 1.f;
   for (int s = 0; s < V.spp; ++s) {
-    Draw D = {V.frame_id, uint32_t(s), V.seed, 0u};
-    // ---- the camera ray (mainRG, deviceCode.cu:293-321)
-    V3 org, dir;
-    {
-      Rng rng;
-      rng.init(V.seed, pixel, V.frame_id, uint32_t(s), 0u);
-      float jx, jy;
-      rng.jitter2(P.fr.jitter2d != 0, jx, jy);
-      camera_ray(*V.cam, px, py, V.W, V.H, jx, jy, org, dir);
-    }
     HitRec h;
-    h.missed = true;
-    h.a = 1.f;
-    h.channel = 0;
-    h.tHit = 0.f;
-    h.r = h.g = h.b = 0.f;
-    float diffuse = 1.0f, specular = 0.0f, shadow = 1.0f;
-    V3 ro = org, rd = dir;
-    bool want = valid;
-    for (int pass = 0; pass < (LIT ? 2 : 1); ++pass) {
-      // the program's grid ray
-      Dda d;
-      bool alive = false;
-      {
-        float c0, c1;
-        WaveRay Y;
-        Y.org_w2g = make_float4(ro.x, ro.y, ro.z, 0.f);
-        Y.dir_g2w = make_float4(rd.x, rd.y, rd.z, 0.f);
-        Y.tend = 0.f;
-        Y.idw = 0.f;
-        if (want && clip_root(ro, rd, blo, bhi, c0, c1)) {
-          const GridRay g = make_grid_ray(ro, rd, blo, bhi, X.mx, X.my, X.mz);
-          alive = d.begin(g.org, g.dir, 1e20f, X.mx, X.my, X.mz);
-          Y.org_w2g.w = g.worldToGridT;
-          Y.dir_g2w.w = g.gridToWorldT;
-          Y.tend = c1;
-          Y.idw = 1.0f / (X.dt * g.worldToGridT);
-        }
-        Y.pixel = pixel;
-        Y.mask = all_ch;
-        L.ray[lane] = Y;
-      }
-      int hit_c = 0;
-      float hit_t = 0.f;
-      const bool hit =
-          track_rays<MODE, DT, WIDE>(P, X, L, s_alpha, w2u, D, d, alive, hit_c, hit_t);
-      if (LIT && pass == 1) {
-        if (want) shadow = (1.f - P.fr.ambient) * (1.f - (hit ? 1.0f : 0.0f));
-        break;
-      }
-      // ---- the hit's colour
-      h.missed = !hit;
-      if (hit) {
-        const WaveRay& Y = L.ray[lane];
-        const float tWorld = hit_t * Y.dir_g2w.w;
-        const V3 xT = (v3(Y.org_w2g.x, Y.org_w2g.y, Y.org_w2g.z) +
-                       tWorld * v3(Y.dir_g2w.x, Y.dir_g2w.y, Y.dir_g2w.z)) * w2u;
-        if (MODE == 4 || MODE == 5) {
-          // the blended sample's colour; the hit keeps channel 0
-          const float4 sb = blend_channels<MODE, DT>(X, xT);
-          h.r = sb.x;
-          h.g = sb.y;
-          h.b = sb.z;
-        } else {
-          float r2;
-          (void)X.tf_alpha(X.sample(xT, hit_c), hit_c, r2);
-          X.tf_rgb(r2, hit_c, h);
-          h.channel = hit_c;
-        }
-        h.tHit = tWorld;
-      }
-      if (!LIT) break;
-      if (hit && P.fr.sh.gradient)
-        shade_gradient(P, X, org, dir, h, diffuse, specular, [&](V3 tex, float eps, int m) {
-          return opacity_gradient(X, s_alpha, tex, eps, m);
-        });
-      if (!P.fr.sh.shadows || __ballot(hit) == 0ull) break;
-      wave_sync();
-      want = hit;
-      ro = org + h.tHit * dir;
-      rd = v3(-P.fr.sh.light_dir[0], -P.fr.sh.light_dir[1], -P.fr.sh.light_dir[2]);
-      D.stream = 1u;
-    }
-    // ---- shade and composite the sample (deviceCode.cu:411-433)
-    composite_sample(P, !h.missed, h.r, h.g, h.b, h.a, diffuse, specular, shadow, h.channel, fr,
-                     fg, fb, fa);
+    const float4 o = trace_sample<MODE, DT, WIDE, LIT>(P, X, L, s_alpha, V, V.frame_id, s, px, py,
+                                                       valid, pixel, w2u, h);
+    fr = fr + o.x;
+    fg = fg + o.y;
+    fb = fb + o.z;
+    fa = fa + o.w;
     if (P.fr.aov && valid) aov_sample(P, V, pixel, s, h);
     wave_sync();
   }
   if (valid) finish_pixel(P, V.accum, V.m2, V.accum_id, V.spp, pixel, fr, fg, fb, fa);
 }
+
+// One 8x8 pixel quad, `frames` frames: the workgroup's four waves trace four
+// consecutive draws (frame, sample) of the quad at a time and the workgroup
+// folds their contributions into the running means in draw order, so the image
+// is the one that frame after frame gives, bit for bit. The frame kernel issues
+// VALU instructions over 80% of its cycles, so what can go is the rest: the
+// accumulator moves once per launch instead of once per frame, the waves of a
+// workgroup read the same cells and voxels (one L1), and the launch's tail,
+// its set-up and its tables are shared by the frames. 64 frames of 1024^2
+// (-m 2, 4 x 256^3 u8): 137 us a frame one by one, 130 / 121 / 118 us at 4 / 8 /
+// 32 draws per launch. Each wave looping over the frames of its own quad
+// without the fold gave 124 us (and nothing on 640 x 480, where the quads alone
+// do not fill the chip: 8 frames of 4 samples 2180 -> 2090 us against 1630).
+// Folding: lane l of wave w owns component l % 4 of the quad's pixel
+// 16 w + l / 4. The contributions pass through the waves' record lists, which
+// are free after a draw.
+struct FoldLds {
+  float4 add[64];
+  float2 hit[64];  // first-hit distance, hit channel (bits; ~0: a miss)
+};
+static_assert(sizeof(FoldLds) <= sizeof(Record) * kRecords, "folded through the record list");
+
+template <int MODE, int DT, bool WIDE, bool LIT>
+__device__ __forceinline__ void team_quad(const RenderParams& P, const Ctx<DT>& X, WaveLds* s_wave,
+                                          const float* s_alpha, const ViewCtx& V, int bx, int by,
+                                          int quad, int frames) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int qs = P.fr.bw == 16 ? 1 : 0;
+  const int qx = bx * P.fr.bw + (quad & qs) * 8, qy = by * P.fr.bh + (quad >> qs) * 8;
+  if (qx >= V.W || qy >= V.H) return;  // the whole workgroup
+  const int px = qx + (lane & 7), py = qy + (lane >> 3);
+  const bool valid = px < V.W && py < V.H;
+  const uint32_t pixel = valid ? uint32_t(px) + uint32_t(V.W) * uint32_t(py) : 0u;
+  const V3 w2u = world_to_unit(P);
+  const int draws = frames * V.spp;
+  // this lane's component of the fold
+  const int fp = 16 * wave + (lane >> 2), comp_i = lane & 3;
+  const int fx = qx + (fp & 7), fy = qy + (fp >> 3);
+  const bool fold = fx < V.W && fy < V.H;
+  const size_t fi = fold ? 4 * (size_t(fx) + size_t(V.W) * fy) + comp_i : 0;
+  const size_t fpix = fi >> 2;
+  float* accum = reinterpret_cast<float*>(V.accum) + fi;
+  float* m2 = V.m2 ? reinterpret_cast<float*>(V.m2) + fi : nullptr;
+  const int ng = aov_groups(P.vol.channels);
+  float* aov = P.fr.aov ? reinterpret_cast<float*>(P.fr.aov) + 4 * size_t(ng) * fpix + comp_i : nullptr;
+  const float sum0 = comp_i == 3 ? 1.f : 0.f, spp = float(V.spp);
+  float mean = 0.f, sq = 0.f, sum = sum0;
+  int sample = 0;
+  uint32_t accum_id = V.accum_id;
+  for (int d0 = 0; d0 < draws; d0 += 4) {
+    const int dr = d0 + wave;
+    if (dr < draws) {
+      WaveLds& L = s_wave[wave];
+      const int f = dr / V.spp, s = dr - f * V.spp;
+      HitRec h;
+      const float4 o = trace_sample<MODE, DT, WIDE, LIT>(P, X, L, s_alpha, V, V.frame_id + uint32_t(f),
+                                                         s, px, py, valid, pixel, w2u, h);
+      wave_sync();
+      FoldLds& F = *reinterpret_cast<FoldLds*>(L.rec);
+      F.add[lane] = o;
+      if (P.fr.aov)
+        F.hit[lane] = make_float2(h.tHit, __uint_as_float(h.missed ? ~0u : uint32_t(h.channel)));
+    }
+    if (d0 == 0 && fold && P.fr.accumulate) {
+      mean = *accum;
+      if (m2) sq = *m2;
+    }
+    __syncthreads();
+    if (fold) {
+      for (int k = 0; k < 4 && d0 + k < draws; ++k) {
+        const FoldLds& F = *reinterpret_cast<const FoldLds*>(s_wave[k].rec);
+        sum = sum + reinterpret_cast<const float*>(&F.add[fp])[comp_i];
+        if (aov) {  // aov_sample
+          const float2 hh = F.hit[fp];
+          const uint32_t code = __float_as_uint(hh.y);
+          const bool hit = code != ~0u;
+          const uint32_t n = (P.fr.accumulate ? accum_id * uint32_t(V.spp) : 0u) + uint32_t(sample);
+          const float kf = float(n), k1 = float(n + 1u);
+          for (int g = 0; g < ng; ++g) {
+            const int slot = 4 * g + comp_i;
+            const float v = slot == 0 ? (hit ? hh.x : 0.f)
+                            : slot == 1 ? (hit ? 0.f : 1.f)
+                                        : (hit && int(code) == slot - 2 ? 1.f : 0.f);
+            const float old = n ? aov[4 * g] : 0.f;
+            aov[4 * g] = (v + kf * old) / k1;
+          }
+        }
+        if (++sample == V.spp) {  // finish_pixel
+          const float v = sum / spp;
+          const float kf = float(accum_id), k1 = float(accum_id + 1u);
+          mean = P.fr.accumulate ? (v + kf * mean) / k1 : v;
+          if (m2) sq = P.fr.accumulate ? (v * v + kf * sq) / k1 : v * v;
+          sample = 0;
+          sum = sum0;
+          ++accum_id;
+        }
+      }
+    }
+    if (d0 + 4 < draws) __syncthreads();
+  }
+  if (fold) {
+    *accum = mean;
+    if (m2) *m2 = sq;
+  }
+}
+
+// Three waves per SIMD is what the LDS allows; stated, so that the register
+// budget is 168 (the shaded several-frame kernels took 172 and ran at two
+// waves: 3.29 -> 2.71 ms for eight 1024^2 frames) and no instance is squeezed
+// towards four waves.
+#define MDWT_WAVE_KERNEL \
+  __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 
 // Per-workgroup set-up: the opacity table and channel parameters in LDS (the
 // only workgroup barrier: the waves run independently from here) and the
@@ -750,16 +895,9 @@ __device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>&
   Ctx<DT> X;                                                                      \
   /* colours of a hit are looked up in the HBM copy of the tables */            \
   X.init(P, reinterpret_cast<const float4*>(P.tf.tab), s_ch);                     \
-  WaveLds& L = s_wave[threadIdx.x >> 6];
+  [[maybe_unused]] WaveLds& L = s_wave[threadIdx.x >> 6];
 
-// One view: workgroup i renders the pixel block at position block_slot(i) of
-// the frame's block order.
-template <int MODE, int DT, bool WIDE, bool LIT>
-__global__ __launch_bounds__(256) void render_wave(RenderParams P) {
-  const uint64_t t_begin = P.fr.wave_cost ? wall_clock64() : 0ull;
-  MDWT_WAVE_PROLOGUE
-  const uint32_t slot_b = block_slot(blockIdx.x, uint32_t(P.fr.n_blocks));
-  const uint32_t bxy = P.fr.block_order[slot_b];
+__device__ __forceinline__ ViewCtx frame_view(const RenderParams& P) {
   ViewCtx V;
   V.cam = &P.cam;
   V.W = P.fr.width;
@@ -770,10 +908,38 @@ __global__ __launch_bounds__(256) void render_wave(RenderParams P) {
   V.accum_id = P.fr.accum_id;
   V.accum = P.fr.accum;
   V.m2 = P.fr.m2;
+  return V;
+}
+
+// One view: workgroup i renders the pixel block at position block_slot(i) of
+// the frame's block order.
+template <int MODE, int DT, bool WIDE, bool LIT>
+MDWT_WAVE_KERNEL void render_wave(RenderParams P) {
+  const uint64_t t_begin = P.fr.wave_cost ? wall_clock64() : 0ull;
+  MDWT_WAVE_PROLOGUE
+  const uint32_t slot_b = block_slot(blockIdx.x, uint32_t(P.fr.n_blocks));
+  const uint32_t bxy = P.fr.block_order[slot_b];
+  const ViewCtx V = frame_view(P);
   wave_block<MODE, DT, WIDE, LIT>(P, X, L, s_alpha, V, int(bxy & 0xffffu), int(bxy >> 16));
   if (P.fr.wave_cost && (threadIdx.x & 63) == 0)
     P.fr.wave_cost[(blockDim.x >> 6) * slot_b + (threadIdx.x >> 6)] =
         uint32_t(wall_clock64() - t_begin);
+}
+
+// One view, P.fr.team_frames frames: workgroup i renders quad i % q of the
+// pixel block at position i / q of the block order (q quads per block).
+template <int MODE, int DT, bool WIDE, bool LIT>
+MDWT_WAVE_KERNEL void render_wave_team(RenderParams P) {
+  const uint64_t t_begin = P.fr.wave_cost ? wall_clock64() : 0ull;
+  MDWT_WAVE_PROLOGUE
+  const uint32_t q = uint32_t(P.fr.bw * P.fr.bh) / 64u;
+  const uint32_t slot_b = blockIdx.x / q, quad = blockIdx.x - slot_b * q;
+  const uint32_t bxy = P.fr.block_order[slot_b];
+  const ViewCtx V = frame_view(P);
+  team_quad<MODE, DT, WIDE, LIT>(P, X, s_wave, s_alpha, V, int(bxy & 0xffffu), int(bxy >> 16),
+                                 int(quad), P.fr.team_frames);
+  if (P.fr.wave_cost && threadIdx.x == 0)
+    P.fr.wave_cost[blockIdx.x] = uint32_t(wall_clock64() - t_begin);
 }
 
 __device__ __forceinline__ ViewCtx batch_view(const RenderParams& P, uint32_t code,
@@ -796,7 +962,7 @@ __device__ __forceinline__ ViewCtx batch_view(const RenderParams& P, uint32_t co
 // by << 10 | bx) at the launch's frame and accumulation ids; with item_ticks
 // set it records its start and end wall clock.
 template <int MODE, int DT, bool WIDE, bool LIT>
-__global__ __launch_bounds__(256) void render_views_wave(RenderParams P) {
+MDWT_WAVE_KERNEL void render_views_wave(RenderParams P) {
   const uint64_t t_begin = P.fr.item_ticks ? wall_clock64() : 0ull;
   MDWT_WAVE_PROLOGUE
   const uint32_t code = P.fr.items[blockIdx.x];
@@ -816,7 +982,7 @@ __global__ __launch_bounds__(256) void render_views_wave(RenderParams P) {
 // moves to its next item as soon as its quad is done. Wave 0 records each
 // item's start and end wall clock.
 template <int MODE, int DT, bool WIDE>
-__global__ __launch_bounds__(256) void render_views_wave_persistent(RenderParams P) {
+MDWT_WAVE_KERNEL void render_views_wave_persistent(RenderParams P) {
   MDWT_WAVE_PROLOGUE
   const uint32_t fid = P.fr.work[1], aid = P.fr.work[2];
   const uint32_t n = uint32_t(P.fr.n_items);

@@ -64,3 +64,39 @@ def test_shading_and_aov_on_both_schedules(capi, mode, channels, dtype):
             r.close()
         for a, b in zip(*out):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("mode,channels,dtype,shaded", [
+    (0, 3, np.uint8, False), (0, 5, np.uint16, False), (1, 4, np.float16, False),
+    (2, 4, np.uint8, False), (2, 10, np.float32, True), (3, 2, np.uint16, True),
+    (4, 4, np.uint8, False), (5, 1, np.float32, True)])
+def test_several_frames_in_one_launch(capi, mode, channels, dtype, shaded):
+    """n frames in one call against n calls of one frame: around the launch's
+    rounds of four draws and its 32 draws, with the auxiliary buffers ending
+    inside the call, with and without accumulation, small workgroups."""
+    vols, tfs = volume(channels, dtype)
+    for size, spp, frames, accumulate, aov, block in (
+            ((9, 7), 1, 4, True, 0, 256), ((75, 51), 1, 39, True, 5, 256), ((40, 64), 2, 3, True, 0, 64),
+            ((33, 24), 3, 9, False, 0, 128), ((17, 16), 4, 1, True, 1, 256), ((8, 8), 33, 5, True, 3, 64)):
+        out = []
+        for split in (False, True):
+            print(f"[paths] mode {mode} channels {channels} {size} spp {spp} frames {frames} "
+                  f"split {split}", flush=True)
+            r = renderer(capi, vols, tfs, mode, size, spp, 0 if split else 1)
+            r.set_frame(size[0], size[1], spp, accumulate, (0.1, 0.2, 0.3))
+            r.set_block(block)
+            r.set_moments(True)
+            if shaded:
+                r.set_light((0.3, -1.0, 0.2), True, True)
+            if aov:
+                r.set_aov(True)
+                r.set_aov_frames(aov)
+            for _ in range(2):  # the second accumulation runs in cost order
+                r.reset_accumulation()
+                for _ in range(frames if split else 1):
+                    r.render(1 if split else frames)
+            got = list(r.read_accum(with_m2=True)) + ([r.read_aov()] if aov else [])
+            out.append([g.view(np.uint32) for g in got] + [np.array(list(r.info().values())[3:])])
+            r.close()
+        for a, b in zip(*out):
+            np.testing.assert_array_equal(a, b)
