@@ -397,6 +397,35 @@ __global__ __launch_bounds__(256) void brick_kernel(const uint8_t* __restrict__ 
                : T(0);
 }
 
+// Joint copy (VolumeParams::joint): output voxel o of group blockIdx.y holds
+// channels 4 g .. 4 g + 3 of brick_kernel's voxel o side by side (zero past the
+// last channel). One thread per output voxel: the reads of a channel are the
+// brick copy's, the write is one 4-, 8- or 16-byte store.
+template <typename T>
+__global__ __launch_bounds__(256) void joint_kernel(const uint8_t* __restrict__ vol, uint64_t chan_stride,
+                                                    int channels, int nx, int ny, int nz, int nbx,
+                                                    int nby, uint64_t per, uint8_t* __restrict__ joint,
+                                                    uint64_t joint_stride) {
+  struct alignas(4 * sizeof(T)) T4 {
+    T v[4];
+  };
+  const uint64_t o = uint64_t(blockIdx.x) * 256u + threadIdx.x;
+  if (o >= per) return;
+  const uint32_t b = uint32_t(o >> 6), w = uint32_t(o & 63u);
+  const uint32_t bx = b % uint32_t(nbx), r = b / uint32_t(nbx);
+  const uint32_t by = r % uint32_t(nby), bz = r / uint32_t(nby);
+  const uint32_t x = bx * 4u + (w & 3u), y = by * 4u + ((w >> 2) & 3u), z = bz * 4u + (w >> 4);
+  const bool in = x < uint32_t(nx) && y < uint32_t(ny) && z < uint32_t(nz);
+  const size_t at = in ? (size_t(z) * uint32_t(ny) + y) * uint32_t(nx) + x : 0;
+  T4 q;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = 4 * int(blockIdx.y) + k;
+    q.v[k] = in && c < channels ? reinterpret_cast<const T*>(vol + size_t(c) * chan_stride)[at] : T(0);
+  }
+  reinterpret_cast<T4*>(joint + size_t(blockIdx.y) * joint_stride)[o] = q;
+}
+
 template <int DT>
 void launch_pencils(const RangeParams& p, hipStream_t s) {
   const dim3 grid(unsigned(p.mc[1]), unsigned(p.mc[2]), unsigned(p.channels));
@@ -447,6 +476,27 @@ hipError_t launch_bricks(const VolumeParams& v, int dtype, hipStream_t s) {
     default:
       hipLaunchKernelGGL(brick_kernel<uint32_t>, grid, dim3(256), 0, s, v.vol, v.chan_stride, v.nx, v.ny,
                          v.nz, v.nbx, v.nby, per, const_cast<uint8_t*>(v.bricks), v.brick_stride);
+      break;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_joint(const VolumeParams& v, int dtype, hipStream_t s) {
+  const uint64_t per = uint64_t(v.nbx) * uint64_t(v.nby) * uint64_t((v.nz + 3) / 4) * 64u;
+  const dim3 grid(unsigned((per + 255) / 256), unsigned((v.channels + 3) / 4));
+  uint8_t* out = const_cast<uint8_t*>(v.joint);
+  switch (dtype_bytes(dtype)) {
+    case 1:
+      hipLaunchKernelGGL(joint_kernel<uint8_t>, grid, dim3(256), 0, s, v.vol, v.chan_stride, v.channels,
+                         v.nx, v.ny, v.nz, v.nbx, v.nby, per, out, v.joint_stride);
+      break;
+    case 2:
+      hipLaunchKernelGGL(joint_kernel<uint16_t>, grid, dim3(256), 0, s, v.vol, v.chan_stride, v.channels,
+                         v.nx, v.ny, v.nz, v.nbx, v.nby, per, out, v.joint_stride);
+      break;
+    default:
+      hipLaunchKernelGGL(joint_kernel<uint32_t>, grid, dim3(256), 0, s, v.vol, v.chan_stride, v.channels,
+                         v.nx, v.ny, v.nz, v.nbx, v.nby, per, out, v.joint_stride);
       break;
   }
   return hipGetLastError();

@@ -111,6 +111,9 @@ struct mdwt_renderer {
   uint64_t chan_stride = 0;
   uint8_t* d_bricks = nullptr;  // brick copy of d_vol, read by the samplers
   uint64_t brick_stride = 0;
+  uint8_t* d_joint = nullptr;  // channels side by side, made when a mode first needs it
+  uint64_t joint_stride = 0;
+  bool joint_tried = false;
   float* d_ranges = nullptr;
   float* d_maj = nullptr;
   Float4* d_tf = nullptr;
@@ -527,6 +530,8 @@ mdwt::VolumeParams volume_params(const mdwt_renderer* h) {
   v.chan_stride = h->chan_stride;
   v.bricks = h->d_bricks;
   v.brick_stride = h->brick_stride;
+  v.joint = h->d_joint;
+  v.joint_stride = h->joint_stride;
   v.nbx = (h->dims[0] + 3) / 4;
   v.nby = (h->dims[1] + 3) / 4;
   v.nx = h->dims[0];
@@ -555,6 +560,24 @@ int make_bricks(mdwt_renderer* h) {
   mdwt::VolumeParams v = volume_params(h);
   v.bricks = h->d_bricks;
   HIPCHK(h, mdwt::launch_bricks(v, h->dtype, h->stream));
+  return MDWT_OK;
+}
+
+// Make the joint copy for -m 3 to -m 8 (which read every channel at a
+// position) on two channels or more. Where the memory for it is not there, the
+// kernels read the channels' own bricks.
+int make_joint(mdwt_renderer* h) {
+  if (h->joint_tried || h->mode < 3 || h->mode > 8 || h->C < 2) return MDWT_OK;
+  h->joint_tried = true;
+  const size_t per = size_t((h->dims[0] + 3) / 4) * size_t((h->dims[1] + 3) / 4) *
+                     size_t((h->dims[2] + 3) / 4) * 64u * 4u * bytes_per_voxel(h->dtype);
+  h->joint_stride = (per + 255) & ~size_t(255);
+  if (hipMalloc(&h->d_joint, h->joint_stride * size_t((h->C + 3) / 4)) != hipSuccess) {
+    (void)hipGetLastError();
+    h->d_joint = nullptr;
+    return MDWT_OK;
+  }
+  HIPCHK(h, mdwt::launch_joint(volume_params(h), h->dtype, h->stream));
   return MDWT_OK;
 }
 
@@ -717,7 +740,7 @@ int mdwt_destroy(mdwt_renderer* h) {
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     free_frame(h);
     free_batch(h);
-    void* ptrs[] = {h->d_vol, h->d_bricks, h->d_ranges, h->d_maj, h->d_tf, h->d_counters, h->d_win};
+    void* ptrs[] = {h->d_vol, h->d_bricks, h->d_joint, h->d_ranges, h->d_maj, h->d_tf, h->d_counters, h->d_win};
     for (void* p : ptrs)
       if (p) (void)hipFree(p);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
@@ -855,7 +878,7 @@ int mdwt_init(mdwt_renderer* h, int mode, const int mc[3], int auto_camera) {
                              hipMemcpyHostToDevice, h->stream));
   int rc0 = build_range_grid(h, wx, wy, wz);
   if (rc0 != MDWT_OK) return rc0;
-  if ((rc0 = make_bricks(h)) != MDWT_OK) return rc0;
+  if ((rc0 = make_bricks(h)) != MDWT_OK || (rc0 = make_joint(h)) != MDWT_OK) return rc0;
   HIPCHK(h, hipMalloc(&h->d_counters, 4 * sizeof(unsigned long long)));
   HIPCHK(h, hipDeviceGetAttribute(&h->cu_count, hipDeviceAttributeMultiprocessorCount, h->device));
   // this device's copy of the allocation-free read's staging array
@@ -885,7 +908,8 @@ int mdwt_set_mode(mdwt_renderer* h, int mode) {
   HIPCHK(h, hipSetDevice(h->device));
   h->mode = mode;
   reset_acc(h);
-  return rebuild_majorants(h);
+  const int rc = make_joint(h);
+  return rc != MDWT_OK ? rc : rebuild_majorants(h);
 }
 
 int mdwt_set_xf_colormap(mdwt_renderer* h, int ch, const float* rgba, int n_texels) {

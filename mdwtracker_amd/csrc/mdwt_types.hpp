@@ -31,6 +31,11 @@ struct VolumeParams {
   uint64_t chan_stride;
   const uint8_t* bricks;
   uint64_t brick_stride;
+  // the channels of a voxel side by side, in groups of four (zero past the last
+  // channel), in the same brick order: group g at joint + g * joint_stride. For
+  // the modes that read every channel at a position; nullptr: not there
+  const uint8_t* joint;
+  uint64_t joint_stride;
   int nbx, nby;
   int nx, ny, nz;
   int channels;

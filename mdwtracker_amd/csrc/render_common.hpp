@@ -32,6 +32,8 @@ template <int DT>
 struct Ctx {
   const uint8_t* bricks;
   uint64_t brick_stride;
+  const uint8_t* joint;
+  uint64_t joint_stride;
   uint32_t nbx, nbxy;  // bricks per row and per slab (both below 2^24)
   int nx, ny, nz;
   float scale, offset;
@@ -46,6 +48,8 @@ struct Ctx {
                                        const ChanTf* ch_lds) {
     bricks = P.vol.bricks;
     brick_stride = P.vol.brick_stride;
+    joint = P.vol.joint;
+    joint_stride = P.vol.joint_stride;
     nbx = uint32_t(P.vol.nbx);
     nbxy = nbx * uint32_t(P.vol.nby);
     nx = P.vol.nx;
@@ -78,8 +82,15 @@ struct Ctx {
                         "+v"(b011), "+v"(b111));
     }
   };
-  __device__ __forceinline__ Corners corners(V3 p, int c) const {
-    Corners k;
+  // The footprint of a position: the voxel indices of its eight corners
+  // (x fastest), the lerp weights, and whether it is in the unit cube.
+  struct Foot {
+    uint32_t i[8];
+    float fx, fy, fz;
+    bool inside;
+  };
+  __device__ __forceinline__ Foot foot(V3 p) const {
+    Foot k;
     k.inside = !(p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f);
     const float x = p.x * float(nx) - 0.5f;
     const float y = p.y * float(ny) - 0.5f;
@@ -91,10 +102,9 @@ struct Ctx {
     const uint32_t x0 = uint32_t(clamp_index(flx, nx)), x1 = uint32_t(clamp_index_plus1(flx, nx));
     const uint32_t y0 = uint32_t(clamp_index(fly, ny)), y1 = uint32_t(clamp_index_plus1(fly, ny));
     const uint32_t z0 = uint32_t(clamp_index(flz, nz)), z1 = uint32_t(clamp_index_plus1(flz, nz));
-    // the voxels are read from the 4 x 4 x 4 brick copy: index = X(x) +
+    // the voxels are read from the 4 x 4 x 4 brick copies: index = X(x) +
     // Y(y) + Z(z) (a trilinear footprint touches about 1.8 cache lines
     // instead of 4 in the planar layout; 3.5% faster at -m 2 on 4 x 256^3 u8)
-    const uint8_t* base = bricks + size_t(c) * brick_stride;
     const uint32_t ax0 = ((x0 >> 2) << 6) | (x0 & 3u), ax1 = ((x1 >> 2) << 6) | (x1 & 3u);
     // 24-bit products (full-rate v_mul_u32_u24): brick coordinates and the
     // bricks per row / slab are below 2^24 (checked when the volume is set)
@@ -103,43 +113,142 @@ struct Ctx {
     const uint32_t az0 = (__umul24(z0 >> 2, nbxy) << 6) | ((z0 & 3u) << 4);
     const uint32_t az1 = (__umul24(z1 >> 2, nbxy) << 6) | ((z1 & 3u) << 4);
     const uint32_t r00 = ay0 + az0, r10 = ay1 + az0, r01 = ay0 + az1, r11 = ay1 + az1;
-    k.b000 = fetch_bits<DT>(base, r00 + ax0);
-    k.b100 = fetch_bits<DT>(base, r00 + ax1);
-    k.b010 = fetch_bits<DT>(base, r10 + ax0);
-    k.b110 = fetch_bits<DT>(base, r10 + ax1);
-    k.b001 = fetch_bits<DT>(base, r01 + ax0);
-    k.b101 = fetch_bits<DT>(base, r01 + ax1);
-    k.b011 = fetch_bits<DT>(base, r11 + ax0);
-    k.b111 = fetch_bits<DT>(base, r11 + ax1);
+    k.i[0] = r00 + ax0;
+    k.i[1] = r00 + ax1;
+    k.i[2] = r10 + ax0;
+    k.i[3] = r10 + ax1;
+    k.i[4] = r01 + ax0;
+    k.i[5] = r01 + ax1;
+    k.i[6] = r11 + ax0;
+    k.i[7] = r11 + ax1;
     return k;
   }
-  // TOGETHER false: for callers with several channels in flight.
-  template <bool TOGETHER = true>
+  __device__ __forceinline__ Corners corners(V3 p, int c) const {
+    const Foot f = foot(p);
+    const uint8_t* base = bricks + size_t(c) * brick_stride;
+    Corners k;
+    k.inside = f.inside;
+    k.fx = f.fx;
+    k.fy = f.fy;
+    k.fz = f.fz;
+    k.b000 = fetch_bits<DT>(base, f.i[0]);
+    k.b100 = fetch_bits<DT>(base, f.i[1]);
+    k.b010 = fetch_bits<DT>(base, f.i[2]);
+    k.b110 = fetch_bits<DT>(base, f.i[3]);
+    k.b001 = fetch_bits<DT>(base, f.i[4]);
+    k.b101 = fetch_bits<DT>(base, f.i[5]);
+    k.b011 = fetch_bits<DT>(base, f.i[6]);
+    k.b111 = fetch_bits<DT>(base, f.i[7]);
+    return k;
+  }
+  __device__ __forceinline__ float lerp8(const float v[8], float fx, float fy, float fz,
+                                         bool inside) const {
+    const float c00 = v[0] + fx * (v[1] - v[0]);
+    const float c10 = v[2] + fx * (v[3] - v[2]);
+    const float c01 = v[4] + fx * (v[5] - v[4]);
+    const float c11 = v[6] + fx * (v[7] - v[6]);
+    const float c0 = c00 + fy * (c10 - c00);
+    const float c1 = c01 + fy * (c11 - c01);
+    const float r = c0 + fz * (c1 - c0);
+    return inside ? r * scale + offset : qnan();
+  }
   __device__ __forceinline__ float trilinear(Corners k) const {
     // All eight loads in flight before the first value is used: left to itself
     // the scheduler saves address registers by issuing one load, waiting for it
     // and reusing its address pair, in some instances and not in others.
-    if (TOGETHER)
-      asm("" : "+v"(k.b000), "+v"(k.b100), "+v"(k.b010), "+v"(k.b110), "+v"(k.b001), "+v"(k.b101),
-               "+v"(k.b011), "+v"(k.b111));
-    const float v000 = voxel_value<DT>(k.b000), v100 = voxel_value<DT>(k.b100);
-    const float v010 = voxel_value<DT>(k.b010), v110 = voxel_value<DT>(k.b110);
-    const float v001 = voxel_value<DT>(k.b001), v101 = voxel_value<DT>(k.b101);
-    const float v011 = voxel_value<DT>(k.b011), v111 = voxel_value<DT>(k.b111);
-    const float c00 = v000 + k.fx * (v100 - v000);
-    const float c10 = v010 + k.fx * (v110 - v010);
-    const float c01 = v001 + k.fx * (v101 - v001);
-    const float c11 = v011 + k.fx * (v111 - v011);
-    const float c0 = c00 + k.fy * (c10 - c00);
-    const float c1 = c01 + k.fy * (c11 - c01);
-    const float r = c0 + k.fz * (c1 - c0);
-    return k.inside ? r * scale + offset : qnan();
+    asm("" : "+v"(k.b000), "+v"(k.b100), "+v"(k.b010), "+v"(k.b110), "+v"(k.b001), "+v"(k.b101),
+             "+v"(k.b011), "+v"(k.b111));
+    const float v[8] = {voxel_value<DT>(k.b000), voxel_value<DT>(k.b100), voxel_value<DT>(k.b010),
+                        voxel_value<DT>(k.b110), voxel_value<DT>(k.b001), voxel_value<DT>(k.b101),
+                        voxel_value<DT>(k.b011), voxel_value<DT>(k.b111)};
+    return lerp8(v, k.fx, k.fy, k.fz, k.inside);
   }
-  template <bool TOGETHER = true>
+
+  // Every channel at one position, in channel order. With the joint copy a
+  // corner's four channels are one load (4, 8 or 16 bytes), so a group of four
+  // takes eight loads and addresses instead of 32: the ray marchers, bound by
+  // VALU issue, went from 805 to 619 us a frame (-m 8, 640 x 480, 4 x 128^3 u8)
+  // with the next step's loads under this step's blend, and -m 3 / 4 / 5 from
+  // 73 / 79 / 79 to 38 / 39 / 38 us (half of it from several frames per launch).
+  // Without the copy (one channel, or no memory for it) each channel is loaded
+  // by itself. The first loads
+  // are issued by all_channels(), the rest as each() gets there.
+  static constexpr int kWords = DT == MDWT_DT_U8 ? 1 : (DT == MDWT_DT_F32 ? 4 : 2);
+  struct AllChannels {
+    Foot f;
+    uint32_t w[8][kWords];
+    __device__ __forceinline__ void arrived() {
+#pragma unroll
+      for (int j = 0; j < kWords; ++j)
+        asm volatile("" : "+v"(w[0][j]), "+v"(w[1][j]), "+v"(w[2][j]), "+v"(w[3][j]),
+                          "+v"(w[4][j]), "+v"(w[5][j]), "+v"(w[6][j]), "+v"(w[7][j]));
+    }
+  };
+  __device__ __forceinline__ void load_channels(AllChannels& a, int c0) const {
+    if (joint) {
+      const uint8_t* base = joint + size_t(c0 >> 2) * joint_stride;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if constexpr (kWords == 1) {
+          a.w[i][0] = reinterpret_cast<const uint32_t*>(base)[a.f.i[i]];
+        } else if constexpr (kWords == 2) {
+          const uint2 v = reinterpret_cast<const uint2*>(base)[a.f.i[i]];
+          a.w[i][0] = v.x;
+          a.w[i][1] = v.y;
+        } else {
+          const uint4 v = reinterpret_cast<const uint4*>(base)[a.f.i[i]];
+          a.w[i][0] = v.x;
+          a.w[i][1] = v.y;
+          a.w[i][2] = v.z;
+          a.w[i][3] = v.w;
+        }
+      }
+    } else {
+      const uint8_t* base = bricks + size_t(c0) * brick_stride;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        a.w[i][0] = fetch_bits<DT>(base, a.f.i[i]);
+#pragma unroll
+        for (int j = 1; j < kWords; ++j) a.w[i][j] = 0u;
+      }
+    }
+  }
+  __device__ __forceinline__ AllChannels all_channels(V3 p) const {
+    AllChannels a;
+    a.f = foot(p);
+    load_channels(a, 0);
+    return a;
+  }
+  // use(c, value) for channel 0, 1, ... until it returns false (value: NaN
+  // outside the unit cube)
+  template <class Use>
+  __device__ __forceinline__ void each(AllChannels& a, const Use& use) const {
+    const int step = joint ? 4 : 1;
+    for (int c0 = 0;;) {
+      a.arrived();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (k >= step || c0 + k >= C) break;
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t bits = DT == MDWT_DT_U8    ? (a.w[i][0] >> (8 * k)) & 0xffu
+                                : DT == MDWT_DT_F32 ? a.w[i][k]
+                                                    : (a.w[i][k >> 1] >> (16 * (k & 1))) & 0xffffu;
+          v[i] = voxel_value<DT>(bits);
+        }
+        if (!use(c0 + k, lerp8(v, a.f.fx, a.f.fy, a.f.fz, a.f.inside))) return;
+      }
+      c0 += step;
+      if (c0 >= C) return;
+      load_channels(a, c0);
+    }
+  }
+
   __device__ __forceinline__ float sample(V3 p, int c) const {
     if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
       return qnan();
-    return trilinear<TOGETHER>(corners(p, c));
+    return trilinear(corners(p, c));
   }
 
   // transferFunction (deviceCode.cu:27-42), opacity only; colour is looked

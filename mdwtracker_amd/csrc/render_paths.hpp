@@ -200,10 +200,11 @@ __device__ void trace_cumulative(const Ctx<DT>& X, const GridRay& g, float prd_t
         }
         float thr = rng.pair_thr() * majorant;
         u = rng.pair_dist();
-        for (int c = 0; c < X.C; ++c) {
-          const float value = X.sample(xT, c);
+        bool hit = false;
+        auto all = X.all_channels(xT);
+        X.each(all, [&](int c, float value) {
           cnt.samples++;
-          if (value != value) continue;
+          if (value != value) return true;
           float r2;
           const float a = X.tf_alpha(value, c, r2);
           if (a > 0.0f && thr < a) {
@@ -211,10 +212,13 @@ __device__ void trace_cumulative(const Ctx<DT>& X, const GridRay& g, float prd_t
             h.tHit = tWorld;
             h.channel = c;
             X.tf_rgb(r2, c, h);
-            return;
+            hit = true;
+            return false;
           }
           thr -= a;
-        }
+          return true;
+        });
+        if (hit) return;
         cnt.rejections++;
       }
     }
@@ -338,56 +342,50 @@ __device__ void trace_multi(const Ctx<DT>& X, const GridRay& g, float prd_t1, Rn
 // blendChannels (deviceCode.cu:222-241): maxOpacityBlend (165-179) for -m 4
 // and 7, mixBlend (182-201) for -m 5 and 8, densityBlend (204-220) for -m 6;
 // (0,0,0,0) outside the unit cube.
-// The ray marchers (-m 6-8) sample every channel at every step: with at most
-// four channels all channels are sampled first, so their voxel loads are in
-// flight together instead of one channel's after another's; the blend then
-// runs in channel order on the same values. Blend tracking (-m 4/5) blends
-// only at tentative collisions and keeps the plain loop (fewer registers).
+// A channel's colour is looked up only where its opacity is not 0 (its terms
+// are then +-0 and leave the sums, which start at +0, as they are).
 template <int MODE, int DT>
-__device__ float4 blend_channels(const Ctx<DT>& X, V3 p) {
-  if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
-    return make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool pre = MODE >= 6 && X.C <= 4;
-  float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (pre) {
-    v4.x = X.template sample<false>(p, 0);
-    if (X.C > 1) v4.y = X.template sample<false>(p, 1);
-    if (X.C > 2) v4.z = X.template sample<false>(p, 2);
-    if (X.C > 3) v4.w = X.template sample<false>(p, 3);
-  }
-  auto value = [&](int c) { return pre ? pick(v4, c) : X.sample(p, c); };
-  if (MODE == 6) {
-    float sum = 0.0f;
-    float4 col = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int c = 0; c < X.C; ++c) {
-      const float4 s = X.tf_rgba(value(c), c);
-      col.x = col.x + s.w * s.x;
-      col.y = col.y + s.w * s.y;
-      col.z = col.z + s.w * s.z;
-      col.w = col.w + s.w * s.w;
-      sum += s.w;
+__device__ __forceinline__ float4 blend_all(const Ctx<DT>& X, typename Ctx<DT>::AllChannels& all) {
+  if (!all.f.inside) return make_float4(0.f, 0.f, 0.f, 0.f);
+  float cr = 0.f, cg = 0.f, cb = 0.f, cw = 0.f, top = 0.0f;
+  X.each(all, [&](int c, float value) {
+    float r2;
+    const float w = X.tf_alpha(value, c, r2);
+    if (MODE == 4 || MODE == 7) {
+      if (w > top) {
+        top = w;
+        HitRec s;
+        X.tf_rgb(r2, c, s);
+        cr = s.r;
+        cg = s.g;
+        cb = s.b;
+      }
+    } else if (w != 0.0f) {
+      HitRec s;
+      X.tf_rgb(r2, c, s);
+      if (MODE == 6) {
+        cr = cr + w * s.r;
+        cg = cg + w * s.g;
+        cb = cb + w * s.b;
+        cw = cw + w * w;
+        top += w;
+      } else {
+        cr = cr + s.r * w;
+        cg = cg + s.g * w;
+        cb = cb + s.b * w;
+        if (w > top) top = w;
+      }
     }
-    if (sum <= 0.0f) return make_float4(0.f, 0.f, 0.f, 0.f);
-    return make_float4(col.x / sum, col.y / sum, col.z / sum, col.w / sum);
-  }
-  if (MODE == 4 || MODE == 7) {
-    float4 best = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int c = 0; c < X.C; ++c) {
-      const float4 s = X.tf_rgba(value(c), c);
-      if (s.w > best.w) best = s;
-    }
-    return best;
-  }
-  float cr = 0.f, cg = 0.f, cb = 0.f, mo = 0.0f;  // -m 5 and 8
-  for (int c = 0; c < X.C; ++c) {
-    const float4 s = X.tf_rgba(value(c), c);
-    cr = cr + s.x * s.w;
-    cg = cg + s.y * s.w;
-    cb = cb + s.z * s.w;
-    if (s.w > mo) mo = s.w;
-  }
-  if (mo <= 0.0f) return make_float4(0.f, 0.f, 0.f, 0.f);
-  return make_float4(cr / mo, cg / mo, cb / mo, mo);
+    return true;
+  });
+  if (MODE == 4 || MODE == 7) return make_float4(cr, cg, cb, top);
+  if (top <= 0.0f) return make_float4(0.f, 0.f, 0.f, 0.f);
+  return make_float4(cr / top, cg / top, cb / top, MODE == 6 ? cw / top : top);
+}
+template <int MODE, int DT>
+__device__ __forceinline__ float4 blend_channels(const Ctx<DT>& X, V3 p) {
+  auto all = X.all_channels(p);
+  return blend_all<MODE, DT>(X, all);
 }
 
 // -m 4 / 5, blendDTCH (deviceCode.cu:972-1065): Woodcock tracking on the
@@ -460,9 +458,14 @@ __device__ void march_blend(const RenderParams& P, const Ctx<DT>& X, V3 org, V3 
   float cr = 0.f, cg = 0.f, cb = 0.f;
   const bool shadows = LIT && P.fr.sh.shadows != 0;
   float hiC = 0.0f, hiT = 0.0f;
+  // the next step's voxels are requested before this step's are blended (the
+  // position does not depend on the blend; indices are clamped, so the request
+  // past the last step is in bounds)
+  auto cur = X.all_channels(pos * w2u);
   for (float t = prd_t0; (t < prd_t1) && (alpha < 0.99f); t += dt) {
-    const V3 posTex = pos * w2u;
-    const float4 b = blend_channels<MODE, DT>(X, posTex);
+    pos = org + dir * t;
+    auto next = X.all_channels(pos * w2u);
+    const float4 b = blend_all<MODE, DT>(X, cur);
     cnt.samples += uint32_t(X.C);
     const float k = 1.f - alpha;
     cr = cr + b.x * b.w * k;
@@ -473,7 +476,7 @@ __device__ void march_blend(const RenderParams& P, const Ctx<DT>& X, V3 org, V3 
       hiC = b.w;
       hiT = t;
     }
-    pos = org + dir * t;
+    cur = next;
   }
   // deviceCode.cu:1117-1154: one marched shadow ray from the most opaque
   // sample towards the light; its first sample sits one world unit from that

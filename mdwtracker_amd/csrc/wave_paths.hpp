@@ -230,55 +230,65 @@ __device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& 
   const float4 ow = Y.org_w2g, dg = Y.dir_g2w;
   const float tWorld = t * dg.w;
   const V3 xT = (v3(ow.x, ow.y, ow.z) + tWorld * v3(dg.x, dg.y, dg.z)) * w2u;
-  // the (first) channel's voxels are requested before the pair is drawn: its
-  // Philox block runs while they are on their way (1 to 2 % of a frame; the
-  // compiler otherwise moves the block behind the wait)
-  [[maybe_unused]] typename Ctx<DT>::Corners k0;
-  if constexpr (MODE <= 3) {
-    k0 = X.corners(xT, MODE == 3 ? 0 : c);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  // the voxels (-m 3-5: of the first channels) are requested before the pair is
+  // drawn: its Philox block runs while they are on their way (1 to 2 % of a
+  // frame; the compiler otherwise moves the block behind the wait)
+  [[maybe_unused]] typename Ctx<DT>::Corners one;
+  [[maybe_unused]] typename Ctx<DT>::AllChannels all;
+  if constexpr (MODE >= 3)
+    all = X.all_channels(xT);
+  else
+    one = X.corners(xT, c);
+  __builtin_amdgcn_sched_barrier(0);
   uint32_t w[4];
   philox(D.frame, D.sample, 1u + (((R.vl & kVisitMask) << 4) | uint32_t(c)), D.stream | ((j >> 1) << 1),
          D.seed, Y.pixel, w);
-  if constexpr (MODE <= 3) {  // in this order: loads, block, values
-    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
-    k0.arrived();
-  }
+  // in this order: loads, block, values
+  asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+  if constexpr (MODE >= 3)
+    all.arrived();
+  else
+    one.arrived();
   const float thr = to_unit((j & 1u) ? w[2] : w[0]) * m;
   const float un = to_unit((j & 1u) ? w[3] : w[1]);
+  bool hit = false;
+  int hit_c = MODE >= 3 ? 0 : c;
   if (MODE == 4 || MODE == 5) {
-    // blendDTCH (deviceCode.cu:972-1065): one blended sample of all channels
-    const float4 sb = blend_channels<MODE, DT>(X, xT);
-    if (sb.w > 0.0f && thr < sb.w) {
-      on_hit<MODE>(L, R, 0, t);
-      return false;
-    }
+    // blendDTCH (deviceCode.cu:972-1065): the opacity of the blended sample of
+    // all channels, the largest in both blends (its colour is only needed at
+    // the hit; outside the unit cube the values are NaN and it stays 0)
+    float top = 0.0f;
+    X.each(all, [&](int k, float value) {
+      const float a = alpha_lookup(s_a, X.chtf[k], value);
+      if (a > top) top = a;
+      return true;
+    });
+    hit = top > 0.0f && thr < top;
   } else if (MODE == 3) {
     // cummilativeDTCH (deviceCode.cu:585-609): the channels in order take
     // their opacity off the threshold until one exceeds what is left
     float th = thr;
-    for (int k = 0; k < X.C; ++k) {
-      const float value = k == 0 ? X.trilinear(k0) : X.sample(xT, k);
-      if (value != value) continue;
+    X.each(all, [&](int k, float value) {
+      if (value != value) return true;
       const float a = alpha_lookup(s_a, X.chtf[k], value);
       if (a > 0.0f && th < a) {
-        on_hit<MODE>(L, R, k, t);
+        hit = true;
+        hit_c = k;
         return false;
       }
       th -= a;
-    }
+      return true;
+    });
   } else {
-    const float value = X.trilinear(k0);
-    bool hit = false;
+    const float value = X.trilinear(one);
     if (!(value != value)) {
       const float a = alpha_lookup(s_a, X.chtf[c], value);
       hit = a > 0.0f && thr < a;
     }
-    if (hit) {
-      on_hit<MODE>(L, R, c, t);
-      return false;
-    }
+  }
+  if (hit) {
+    on_hit<MODE>(L, R, hit_c, t);
+    return false;
   }
   tn = t - (plogf_poly(1.0f - un) / m) * X.dt * ow.w;
   if (tn >= R.t1) return false;  // leaves the cell

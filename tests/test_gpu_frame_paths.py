@@ -100,3 +100,27 @@ def test_several_frames_in_one_launch(capi, mode, channels, dtype, shaded):
             r.close()
         for a, b in zip(*out):
             np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("channels,dtype", [(2, np.uint8), (3, np.uint16), (5, np.float16), (9, np.float32)])
+@pytest.mark.parametrize("mode", [3, 4, 5, 6, 7, 8])
+def test_channels_side_by_side_match_the_oracle(capi, mode, channels, dtype):
+    """The modes that read every channel at a position, with channel counts
+    that fill their groups of four in part, against the CPU oracle."""
+    from oracle import pyoracle
+    vols, tfs = volume(channels, dtype, dims=(19, 22, 17))
+    print(f"[paths] mode {mode} channels {channels} {np.dtype(dtype)}", flush=True)
+    g = renderer(capi, vols, tfs, mode, (43, 30), 1, 1, mc=(4, 5, 3), opacity=0.2)
+    o = pyoracle.OracleRenderer()
+    for v in vols:
+        o.push_channel(v)
+    o.init(mode, (4, 5, 3), False)
+    for c, t in enumerate(tfs):
+        o.set_tf(c, t, 0.2, (0.0, 1.0))
+    o.set_frame(43, 30, 1, True, (0.1, 0.2, 0.3))
+    o.set_camera(*scenes.orbit_camera(1.6))
+    o.set_seed(11)
+    g.render(2)
+    o.render(2, threads=4)
+    np.testing.assert_array_equal(g.read_accum().view(np.uint32), o.read_accum().view(np.uint32))
+    g.close()
