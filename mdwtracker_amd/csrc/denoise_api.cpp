@@ -12,11 +12,13 @@
 
 #include <hip/hip_runtime.h>
 
-#include <chrono>
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "denoise_internal.hpp"
@@ -29,9 +31,20 @@ struct Conv {
   int cin_pad32 = 0;              // dgrad N (multiple of 32)
   bool relu = true;
   size_t nw = 0;                  // 9 * cout * cin
-  float *w = nullptr, *b = nullptr, *gw = nullptr, *gb = nullptr;
-  float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
+  size_t off = 0;                 // of its weights in the parameter arrays, the biases behind them
+  float *w = nullptr, *b = nullptr;  // in mdwt_denoiser::params
   uint16_t *wf = nullptr, *wd = nullptr;
+};
+
+// What a training step on a batch of `images` images keeps on the device.
+// Activations are bf16; gm0 / gm1 hold the masked gradients of two consecutive
+// layers, skip1 / skip3 the fp32 gradients of the two skip connections.
+struct TrainBufs {
+  int images = 0;
+  std::vector<void*> bufs;
+  float *in32 = nullptr, *tgt = nullptr, *inv = nullptr;
+  uint16_t *x0, *a0, *a1, *p1, *a2, *a3, *p2, *a4, *a5, *a6, *a7, *a8, *a9, *gm0, *gm1;
+  float *skip1, *skip3;
 };
 
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
@@ -47,12 +60,15 @@ struct mdwt_denoiser {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   Conv c[11];
   std::vector<void*> bufs;
-  // activations (bf16)
-  uint16_t *x0, *a0, *a1, *p1, *a2, *a3, *p2, *a4, *a5, *u2, *a6, *a7, *u1, *a8, *a9, *gm;
-  // fp32: network io and gradients
-  float *in32, *tgt, *out32, *pred, *err_sum;
-  float* wpart;  // partial weight gradients of the row bands
-  float *gout, *g9, *g8, *gu1, *g7, *g6, *gu2, *g5, *g4, *gp2, *g3, *g2, *gp1, *g1, *g0;
+  // fp32 parameters, gradients and Adam moments of every layer: its weights,
+  // then its biases (the layout of mdwt_dn_get_params)
+  size_t n_params = 0;
+  float *params = nullptr, *grads = nullptr, *mom = nullptr, *var = nullptr;
+  // inference: activations (bf16) and network io (fp32)
+  uint16_t *x0, *a0, *a1, *p1, *a2, *a3, *p2, *a4, *a5, *u2, *a6, *a7, *u1, *a8, *a9;
+  float *in32, *out32, *pred, *err_sum;
+  float* wpart = nullptr;  // partial weight gradients of the workgroups
+  TrainBufs train;  // made by the first step, grown by a larger batch
   int step = 0;
   bool fused = true;  // inference: fused upsample/concat, pooling and filter
 };
@@ -83,8 +99,7 @@ int alloc(mdwt_denoiser* d, T** p, size_t n) {
 
 // layer table: (cin, cout, relu); c0 reads the input (cin set per handle),
 // c10 writes the kTaps filter logits
-// largest image (pixels) a denoiser handle accepts
-constexpr size_t kMaxPixels = size_t(1) << 24;
+using mdwt::dn::kMaxPixels;  // largest image (pixels) a denoiser handle accepts
 
 const int kLayers[11][3] = {{0, 32, 1}, {32, 32, 1}, {32, 64, 1},
                             {64, 64, 1},  {64, 96, 1}, {96, 96, 1}, {160, 64, 1},
@@ -92,9 +107,11 @@ const int kLayers[11][3] = {{0, 32, 1}, {32, 32, 1}, {32, 64, 1},
 
 // width in pixels of the Gaussian filter the untrained network applies
 constexpr float kInitSigma = 1.5f;
-// floats of partial weight gradients (16 MiB): at least 9 * cout * cin of
-// every layer, and room for enough row bands to fill the GPU
-constexpr size_t kWgradPart = size_t(4) << 20;
+// floats of partial weight gradients (48 MiB): at least 9 * cout * cin + cout of
+// every layer, and room for enough workgroups to fill the GPU
+constexpr size_t kWgradPart = size_t(12) << 20;
+// pixels of one training batch on the device (3 GB); larger batches go in parts
+constexpr size_t kTrainPixels = size_t(1) << 20;
 
 int setup(mdwt_denoiser* d, uint32_t seed) {
   std::mt19937 gen(seed);
@@ -107,12 +124,18 @@ int setup(mdwt_denoiser* d, uint32_t seed) {
     L.cout_pad = round_up(L.cout, 32);
     L.cin_pad32 = round_up(L.cin, 32);
     L.nw = size_t(9) * L.cout * L.cin;
-    int rc;
-    if ((rc = alloc(d, &L.w, L.nw)) || (rc = alloc(d, &L.gw, L.nw)) || (rc = alloc(d, &L.mw, L.nw)) ||
-        (rc = alloc(d, &L.vw, L.nw)) || (rc = alloc(d, &L.b, size_t(L.cout))) ||
-        (rc = alloc(d, &L.gb, size_t(L.cout))) || (rc = alloc(d, &L.mb, size_t(L.cout))) ||
-        (rc = alloc(d, &L.vb, size_t(L.cout))) ||
-        (rc = alloc(d, &L.wf, size_t(9) * L.cout_pad * L.cin_pad)) ||
+    L.off = d->n_params;
+    d->n_params += L.nw + size_t(L.cout);
+  }
+  int rc;
+  if ((rc = alloc(d, &d->params, d->n_params)) || (rc = alloc(d, &d->grads, d->n_params)) ||
+      (rc = alloc(d, &d->mom, d->n_params)) || (rc = alloc(d, &d->var, d->n_params)))
+    return rc;
+  for (int i = 0; i < 11; ++i) {
+    Conv& L = d->c[i];
+    L.w = d->params + L.off;
+    L.b = L.w + L.nw;
+    if ((rc = alloc(d, &L.wf, size_t(9) * L.cout_pad * L.cin_pad)) ||
         (rc = alloc(d, &L.wd, size_t(9) * L.cin_pad32 * L.cout_pad)))
       return rc;
     // He initialisation for ReLU layers; the output layer starts small
@@ -134,7 +157,6 @@ int setup(mdwt_denoiser* d, uint32_t seed) {
     }
   }
   const size_t n = size_t(d->H) * d->W, n4 = n / 4, n16 = n / 16;
-  int rc;
   if ((rc = alloc(d, &d->x0, n * d->in_pad)) || (rc = alloc(d, &d->a0, n * 32)) ||
       (rc = alloc(d, &d->a1, n * 32)) || (rc = alloc(d, &d->p1, n4 * 32)) ||
       (rc = alloc(d, &d->a2, n4 * 64)) || (rc = alloc(d, &d->a3, n4 * 64)) ||
@@ -142,38 +164,122 @@ int setup(mdwt_denoiser* d, uint32_t seed) {
       (rc = alloc(d, &d->a5, n16 * 96)) || (rc = alloc(d, &d->u2, n4 * 160)) ||
       (rc = alloc(d, &d->a6, n4 * 64)) || (rc = alloc(d, &d->a7, n4 * 64)) ||
       (rc = alloc(d, &d->u1, n * 96)) || (rc = alloc(d, &d->a8, n * 32)) ||
-      (rc = alloc(d, &d->a9, n * 32)) || (rc = alloc(d, &d->gm, n * mdwt::dn::kLogitStride)))
+      (rc = alloc(d, &d->a9, n * 32)))
     return rc;
-  if ((rc = alloc(d, &d->in32, n * d->inputs)) || (rc = alloc(d, &d->tgt, n * 3)) ||
+  if ((rc = alloc(d, &d->in32, n * d->inputs)) ||
       (rc = alloc(d, &d->out32, n * mdwt::dn::kLogitStride)) || (rc = alloc(d, &d->pred, n * 3)) ||
-      (rc = alloc(d, &d->err_sum, 1)) || (rc = alloc(d, &d->wpart, kWgradPart)) ||
-      (rc = alloc(d, &d->gout, n * mdwt::dn::kLogitStride)) ||
-      (rc = alloc(d, &d->g9, n * 32)) || (rc = alloc(d, &d->g8, n * 32)) ||
-      (rc = alloc(d, &d->gu1, n * 96)) || (rc = alloc(d, &d->g7, n4 * 64)) ||
-      (rc = alloc(d, &d->g6, n4 * 64)) || (rc = alloc(d, &d->gu2, n4 * 160)) ||
-      (rc = alloc(d, &d->g5, n16 * 96)) || (rc = alloc(d, &d->g4, n16 * 96)) ||
-      (rc = alloc(d, &d->gp2, n16 * 64)) || (rc = alloc(d, &d->g3, n4 * 64)) ||
-      (rc = alloc(d, &d->g2, n4 * 64)) || (rc = alloc(d, &d->gp1, n4 * 32)) ||
-      (rc = alloc(d, &d->g1, n * 32)) || (rc = alloc(d, &d->g0, n * 32)))
+      (rc = alloc(d, &d->err_sum, 1)))
     return rc;
   return MDWT_OK;
 }
 
-int refresh_weights(mdwt_denoiser* d) {
-  for (Conv& L : d->c)
-    DNCHK(d, mdwt::dn::weight_layouts(L.w, L.cin, L.cout, L.cin_pad, L.cout_pad, L.wf,
-                                      L.cin_pad32, L.cout_pad, L.wd, d->stream));
+void free_train(TrainBufs* t) {
+  for (void* p : t->bufs) (void)hipFree(p);
+  *t = TrainBufs{};
+}
+
+// Device memory for training on up to `images` images at a time. If it is not
+// there for more than the present buffers hold, those stay (and the batch goes
+// in smaller parts).
+int train_bufs(mdwt_denoiser* d, int images) {
+  images = int(std::max<size_t>(1, std::min(size_t(images), kTrainPixels / (size_t(d->H) * d->W))));
+  if (images <= d->train.images) return MDWT_OK;
+  if (!d->wpart) {
+    int rc = alloc(d, &d->wpart, kWgradPart);
+    if (rc) return rc;
+  }
+  while (images > d->train.images) {
+    TrainBufs t;
+    t.images = images;
+    bool ok = true;
+    auto get = [&](auto** p, size_t n) {
+      void* q = nullptr;
+      if (ok && hipMalloc(&q, n * sizeof(**p)) == hipSuccess)
+        t.bufs.push_back(q);
+      else
+        ok = false;
+      *p = static_cast<std::remove_reference_t<decltype(*p)>>(q);
+    };
+    const size_t n = size_t(images) * d->H * d->W, n4 = n / 4, n16 = n / 16;
+    get(&t.in32, n * d->inputs);
+    get(&t.tgt, n * 3);
+    get(&t.inv, size_t(images));
+    get(&t.x0, n * d->in_pad);
+    get(&t.a0, n * 32);
+    get(&t.a1, n * 32);
+    get(&t.p1, n4 * 32);
+    get(&t.a2, n4 * 64);
+    get(&t.a3, n4 * 64);
+    get(&t.p2, n16 * 64);
+    get(&t.a4, n16 * 96);
+    get(&t.a5, n16 * 96);
+    get(&t.a6, n4 * 64);
+    get(&t.a7, n4 * 64);
+    get(&t.a8, n * 32);
+    get(&t.a9, n * 32);
+    get(&t.gm0, n * mdwt::dn::kLogitStride);
+    get(&t.gm1, n * mdwt::dn::kLogitStride);
+    get(&t.skip1, n * 32);
+    get(&t.skip3, n4 * 64);
+    if (ok) {
+      free_train(&d->train);
+      d->train = std::move(t);
+      return MDWT_OK;
+    }
+    (void)hipGetLastError();
+    free_train(&t);
+    if (d->train.images > 0) return MDWT_OK;
+    if (images == 1) return fail(d, MDWT_ERR_OOM, "denoiser training buffers");
+    images = (images + 1) / 2;
+  }
   return MDWT_OK;
+}
+
+int refresh_weights(mdwt_denoiser* d) {
+  mdwt::dn::LayoutArgs a;
+  for (int i = 0; i < mdwt::dn::kLayers; ++i) {
+    const Conv& L = d->c[i];
+    a.layer[i] = {L.w, L.wf, L.wd, L.cin, L.cout, L.cin_pad, L.cout_pad, L.cin_pad32};
+  }
+  DNCHK(d, mdwt::dn::weight_layouts(a, d->stream));
+  return MDWT_OK;
+}
+
+// conv layer i forward with an input source / epilogue (ConvArgs)
+int fwd_fused(mdwt_denoiser* d, int i, mdwt::dn::ConvArgs a, int src, int epi) {
+  const Conv& L = d->c[i];
+  a.cin = L.cin_pad;
+  a.w = L.wf;
+  a.bias = L.b;
+  a.cout = L.cout;
+  a.cout_pad = L.cout_pad;
+  a.relu = L.relu ? 1 : 0;
+  DNCHK(d, mdwt::dn::conv(a, src, epi, d->stream));
+  return MDWT_OK;
+}
+
+mdwt::dn::ConvArgs conv_args(const uint16_t* x, int xs, int nimg, int H, int W, uint16_t* y16, int ys) {
+  mdwt::dn::ConvArgs a{};
+  a.x = x;
+  a.xs = xs;
+  a.nimg = nimg;
+  a.H = H;
+  a.W = W;
+  a.y16 = y16;
+  a.ys = ys;
+  return a;
 }
 
 // conv layer i forward: x (stride xs, offset xo) -> y16 / y32 (stride ys)
 int fwd(mdwt_denoiser* d, int i, const uint16_t* x, int H, int W, int xs, int xo, uint16_t* y16,
         float* y32, int ys) {
-  const Conv& L = d->c[i];
-  DNCHK(d, mdwt::dn::conv3x3(x, H, W, xs, xo, L.cin_pad, L.wf, L.b, L.cout, L.cout_pad, y16, y32,
-                             ys, 0, L.relu, false, d->stream));
-  return MDWT_OK;
+  mdwt::dn::ConvArgs a = conv_args(x, xs, 1, H, W, y16, ys);
+  a.xo = xo;
+  a.y32 = y32;
+  return fwd_fused(d, i, a, mdwt::dn::kSrcPlain, mdwt::dn::kEpiPlain);
 }
+
+// Inference with a kernel for every step of the network (mdwt_dn_set_fused 0)
 
 int forward(mdwt_denoiser* d) {
   const int H = d->H, W = d->W, n = H * W;
@@ -202,19 +308,6 @@ int forward(mdwt_denoiser* d) {
   return MDWT_OK;
 }
 
-// conv layer i forward with a fused input source / epilogue (ConvArgs)
-int fwd_fused(mdwt_denoiser* d, int i, mdwt::dn::ConvArgs a, int src, int epi) {
-  const Conv& L = d->c[i];
-  a.cin = L.cin_pad;
-  a.w = L.wf;
-  a.bias = L.b;
-  a.cout = L.cout;
-  a.cout_pad = L.cout_pad;
-  a.relu = L.relu ? 1 : 0;
-  DNCHK(d, mdwt::dn::conv(a, src, epi, d->stream));
-  return MDWT_OK;
-}
-
 // Inference forward: the same values as forward() (every fused step
 // computes what the kernel it replaces would have stored), without
 // materialising the packed input, the pooled, upsampled and concatenated
@@ -223,18 +316,11 @@ int fwd_fused(mdwt_denoiser* d, int i, mdwt::dn::ConvArgs a, int src, int epi) {
 // c10 applies the filter in its epilogue.
 int forward_fused(mdwt_denoiser* d) {
   using namespace mdwt::dn;
-  const int H = d->H, W = d->W, n = H * W;
+  const int H = d->H, W = d->W;
   const int H2 = H / 2, W2 = W / 2, H4 = H / 4, W4 = W / 4;
   int rc;
   auto args = [](const uint16_t* x, int xs, int Hh, int Ww, uint16_t* y16, int ys) {
-    ConvArgs a{};
-    a.x = x;
-    a.xs = xs;
-    a.H = Hh;
-    a.W = Ww;
-    a.y16 = y16;
-    a.ys = ys;
-    return a;
+    return conv_args(x, xs, 1, Hh, Ww, y16, ys);
   };
   ConvArgs a = args(nullptr, 0, H, W, d->a0, 32);  // c0 reads the fp32 input
   a.kin = d->in32;
@@ -268,72 +354,147 @@ int forward_fused(mdwt_denoiser* d) {
   return fwd_fused(d, 10, a, kSrcPlain, kEpiKpn);
 }
 
-// backward of conv layer i: gy (fp32, stride gs) of its output y (bf16,
-// stride ys); input x (stride xs, offset xo); gx (fp32, stride gxs) gets
-// the input gradient (skipped when null)
-int bwd(mdwt_denoiser* d, int i, const float* gy, int gs, const uint16_t* y, int ys,
-        const uint16_t* x, int xs, int xo, int H, int W, float* gx, int gxs) {
+// Backward of conv layer i at B images of H x W: its weight and bias gradients
+// from gm (the masked bf16 gradient of its output, stride cout_pad) and its
+// input (x, or for a concatenated input xl upsampled and x), then, where epi
+// >= 0, the input gradient through epilogue epi of `a` (the target fields).
+int bwd(mdwt_denoiser* d, int i, int B, int H, int W, const uint16_t* gm, const uint16_t* x, int xs,
+        const uint16_t* xl, int cu, mdwt::dn::ConvArgs a, int epi) {
   const Conv& L = d->c[i];
-  hipStream_t s = d->stream;
-  // the bias partial sums use the weight-gradient scratch, reduced before wgrad runs
-  DNCHK(d, mdwt::dn::relu_grad(gy, gs, y, ys, 0, H * W, L.cout, L.cout_pad, L.relu, d->gm, L.gb,
-                               d->wpart, kWgradPart, s));
-  DNCHK(d, mdwt::dn::wgrad(d->gm, L.cout_pad, x, xs, xo, H, W, L.cin, L.cout, L.gw, d->wpart,
-                           kWgradPart, s));
-  if (gx)
-    DNCHK(d, mdwt::dn::conv3x3(d->gm, H, W, L.cout_pad, 0, L.cout_pad, L.wd, nullptr, L.cin,
-                               L.cin_pad32, nullptr, gx, gxs, 0, false, false, s));
+  mdwt::dn::WgradArgs g{};
+  g.g = gm;
+  g.gs = L.cout_pad;
+  g.x = x;
+  g.xs = xs;
+  g.xl = xl;
+  g.cu = cu;
+  g.nimg = B;
+  g.H = H;
+  g.W = W;
+  g.cin = L.cin;
+  g.cout = L.cout;
+  g.part = d->wpart;
+  DNCHK(d, mdwt::dn::wgrad(g, d->grads + L.off, kWgradPart, d->stream));
+  if (epi < 0) return MDWT_OK;
+  a.x = gm;
+  a.xs = L.cout_pad;
+  a.nimg = B;
+  a.H = H;
+  a.W = W;
+  a.cin = L.cout_pad;
+  a.w = L.wd;
+  a.cout = L.cin;
+  a.cout_pad = L.cin_pad32;
+  DNCHK(d, mdwt::dn::conv(a, mdwt::dn::kSrcPlain, epi, d->stream));
   return MDWT_OK;
 }
 
-int backward(mdwt_denoiser* d) {
-  const int H = d->H, W = d->W, n = H * W;
+// Loss gradient of the B images in the training buffers, added to grads (and
+// the squared error to err_sum): the forward of forward_fused over the batch,
+// keeping the activations, then the layers in reverse. Every kernel takes the
+// whole batch: image by image, a step of 8 x 256^2 was about 1000 launches of 5
+// to 30 us, most of them too small for the chip: 8.0 ms of kernels, 1.4 ms so.
+int train_batch(mdwt_denoiser* d, int B) {
+  using namespace mdwt::dn;
+  TrainBufs& t = d->train;
+  const int H = d->H, W = d->W;
   const int H2 = H / 2, W2 = W / 2, H4 = H / 4, W4 = W / 4;
-  hipStream_t s = d->stream;
   int rc;
-  DNCHK(d, hipMemsetAsync(d->g1, 0, size_t(n) * 32 * sizeof(float), s));
-  DNCHK(d, hipMemsetAsync(d->g3, 0, size_t(H2) * W2 * 64 * sizeof(float), s));
-  if ((rc = bwd(d, 10, d->gout, mdwt::dn::kLogitStride, nullptr, 0, d->a9, 32, 0, H, W, d->g9,
-                32)))
-    return rc;
-  if ((rc = bwd(d, 9, d->g9, 32, d->a9, 32, d->a8, 32, 0, H, W, d->g8, 32))) return rc;
-  if ((rc = bwd(d, 8, d->g8, 32, d->a8, 32, d->u1, 96, 0, H, W, d->gu1, 96))) return rc;
-  DNCHK(d, mdwt::dn::up_grad(d->gu1, H, W, 96, 0, 64, d->g7, s));
-  DNCHK(d, mdwt::dn::add_slice(d->gu1, 96, 64, n, 32, d->g1, s));
-  if ((rc = bwd(d, 7, d->g7, 64, d->a7, 64, d->a6, 64, 0, H2, W2, d->g6, 64))) return rc;
-  if ((rc = bwd(d, 6, d->g6, 64, d->a6, 64, d->u2, 160, 0, H2, W2, d->gu2, 160))) return rc;
-  DNCHK(d, mdwt::dn::up_grad(d->gu2, H2, W2, 160, 0, 96, d->g5, s));
-  DNCHK(d, mdwt::dn::add_slice(d->gu2, 160, 96, H2 * W2, 64, d->g3, s));
-  if ((rc = bwd(d, 5, d->g5, 96, d->a5, 96, d->a4, 96, 0, H4, W4, d->g4, 96))) return rc;
-  if ((rc = bwd(d, 4, d->g4, 96, d->a4, 96, d->p2, 64, 0, H4, W4, d->gp2, 64))) return rc;
-  DNCHK(d, mdwt::dn::pool_grad(d->gp2, H2, W2, 64, d->g3, s));
-  if ((rc = bwd(d, 3, d->g3, 64, d->a3, 64, d->a2, 64, 0, H2, W2, d->g2, 64))) return rc;
-  if ((rc = bwd(d, 2, d->g2, 64, d->a2, 64, d->p1, 32, 0, H2, W2, d->gp1, 32))) return rc;
-  DNCHK(d, mdwt::dn::pool_grad(d->gp1, H, W, 32, d->g1, s));
-  if ((rc = bwd(d, 1, d->g1, 32, d->a1, 32, d->a0, 32, 0, H, W, d->g0, 32))) return rc;
-  if ((rc = bwd(d, 0, d->g0, 32, d->a0, 32, d->x0, d->in_pad, 0, H, W, nullptr, 0))) return rc;
-  return MDWT_OK;
+  DNCHK(d, pack_input(t.in32, B * H * W, d->inputs, d->in_pad, t.x0, d->stream));
+  if ((rc = fwd_fused(d, 0, conv_args(t.x0, d->in_pad, B, H, W, t.a0, 32), kSrcPlain, kEpiPlain))) return rc;
+  ConvArgs a = conv_args(t.a0, 32, B, H, W, t.a1, 32);
+  a.pool16 = t.p1;
+  a.ps = 32;
+  if ((rc = fwd_fused(d, 1, a, kSrcPlain, kEpiPool))) return rc;
+  if ((rc = fwd_fused(d, 2, conv_args(t.p1, 32, B, H2, W2, t.a2, 64), kSrcPlain, kEpiPlain))) return rc;
+  a = conv_args(t.a2, 64, B, H2, W2, t.a3, 64);
+  a.pool16 = t.p2;
+  a.ps = 64;
+  if ((rc = fwd_fused(d, 3, a, kSrcPlain, kEpiPool))) return rc;
+  if ((rc = fwd_fused(d, 4, conv_args(t.p2, 64, B, H4, W4, t.a4, 96), kSrcPlain, kEpiPlain))) return rc;
+  if ((rc = fwd_fused(d, 5, conv_args(t.a4, 96, B, H4, W4, t.a5, 96), kSrcPlain, kEpiPlain))) return rc;
+  a = conv_args(t.a3, 64, B, H2, W2, t.a6, 64);
+  a.xl = t.a5;
+  a.cu = 96;
+  if ((rc = fwd_fused(d, 6, a, kSrcUpCat, kEpiPlain))) return rc;
+  if ((rc = fwd_fused(d, 7, conv_args(t.a6, 64, B, H2, W2, t.a7, 64), kSrcPlain, kEpiPlain))) return rc;
+  a = conv_args(t.a1, 32, B, H, W, t.a8, 32);
+  a.xl = t.a7;
+  a.cu = 64;
+  if ((rc = fwd_fused(d, 8, a, kSrcUpCat, kEpiPlain))) return rc;
+  if ((rc = fwd_fused(d, 9, conv_args(t.a8, 32, B, H, W, t.a9, 32), kSrcPlain, kEpiPlain))) return rc;
+  a = conv_args(t.a9, 32, B, H, W, t.gm0, kLogitStride);
+  a.kin = t.in32;
+  a.inputs = d->inputs;
+  a.target = t.tgt;
+  a.inv_count = t.inv;
+  a.err = d->err_sum;
+  if ((rc = fwd_fused(d, 10, a, kSrcPlain, kEpiKpnLoss))) return rc;
+
+  // the gradient through the ReLU of the layer whose output is act
+  auto mask = [](const uint16_t* act, int ys, uint16_t* gm) {
+    ConvArgs m{};
+    m.act = act;
+    m.ys = ys;
+    m.y16 = gm;
+    return m;
+  };
+  // through an upsample-and-concatenate: channels < cu to the low-resolution
+  // layer (output act), the others to the skip's fp32 gradient
+  auto upgrad = [](const uint16_t* act, int cu, uint16_t* gm, float* skip, int ss) {
+    ConvArgs m{};
+    m.act = act;
+    m.cu = cu;
+    m.y16 = gm;
+    m.y32 = skip;
+    m.ys = ss;
+    return m;
+  };
+  auto poolgrad = [](const uint16_t* act, int ys, uint16_t* gm, const float* skip) {
+    ConvArgs m{};
+    m.act = act;
+    m.ys = ys;
+    m.y16 = gm;
+    m.skip = skip;
+    return m;
+  };
+  uint16_t *g0 = t.gm0, *g1 = t.gm1;
+  if ((rc = bwd(d, 10, B, H, W, g0, t.a9, 32, nullptr, 0, mask(t.a9, 32, g1), kEpiMask))) return rc;
+  if ((rc = bwd(d, 9, B, H, W, g1, t.a8, 32, nullptr, 0, mask(t.a8, 32, g0), kEpiMask))) return rc;
+  if ((rc = bwd(d, 8, B, H, W, g0, t.a1, 32, t.a7, 64, upgrad(t.a7, 64, g1, t.skip1, 32), kEpiUpGrad))) return rc;
+  if ((rc = bwd(d, 7, B, H2, W2, g1, t.a6, 64, nullptr, 0, mask(t.a6, 64, g0), kEpiMask))) return rc;
+  if ((rc = bwd(d, 6, B, H2, W2, g0, t.a3, 64, t.a5, 96, upgrad(t.a5, 96, g1, t.skip3, 64), kEpiUpGrad))) return rc;
+  if ((rc = bwd(d, 5, B, H4, W4, g1, t.a4, 96, nullptr, 0, mask(t.a4, 96, g0), kEpiMask))) return rc;
+  if ((rc = bwd(d, 4, B, H4, W4, g0, t.p2, 64, nullptr, 0, poolgrad(t.a3, 64, g1, t.skip3), kEpiPoolGrad))) return rc;
+  if ((rc = bwd(d, 3, B, H2, W2, g1, t.a2, 64, nullptr, 0, mask(t.a2, 64, g0), kEpiMask))) return rc;
+  if ((rc = bwd(d, 2, B, H2, W2, g0, t.p1, 32, nullptr, 0, poolgrad(t.a1, 32, g1, t.skip1), kEpiPoolGrad))) return rc;
+  if ((rc = bwd(d, 1, B, H, W, g1, t.a0, 32, nullptr, 0, mask(t.a0, 32, g0), kEpiMask))) return rc;
+  return bwd(d, 0, B, H, W, g0, t.x0, d->in_pad, nullptr, 0, ConvArgs{}, -1);
 }
 
-int zero_grads(mdwt_denoiser* d) {
-  for (Conv& L : d->c) {
-    DNCHK(d, hipMemsetAsync(L.gw, 0, L.nw * sizeof(float), d->stream));
-    DNCHK(d, hipMemsetAsync(L.gb, 0, size_t(L.cout) * sizeof(float), d->stream));
+// Loss gradient of `count` host pairs into grads and err_sum, in parts of as
+// many images as the training buffers hold; pair i's squared error is weighted
+// by inv * weights[i] (1 without weights).
+int loss_gradient(mdwt_denoiser* d, const float* in, const float* tgt, const float* weights, int count,
+                  float inv) {
+  const size_t n = size_t(d->H) * d->W;
+  int rc = train_bufs(d, count);
+  if (rc) return rc;
+  DNCHK(d, hipMemsetAsync(d->grads, 0, d->n_params * sizeof(float), d->stream));
+  DNCHK(d, hipMemsetAsync(d->err_sum, 0, sizeof(float), d->stream));
+  std::vector<float> w(size_t(std::min(count, d->train.images)));
+  for (int i = 0; i < count; i += d->train.images) {
+    const int B = std::min(count - i, d->train.images);
+    for (int k = 0; k < B; ++k) w[size_t(k)] = weights ? inv * weights[i + k] : inv;
+    DNCHK(d, hipMemcpyAsync(d->train.inv, w.data(), size_t(B) * sizeof(float), hipMemcpyHostToDevice, d->stream));
+    DNCHK(d, hipMemcpyAsync(d->train.in32, in + size_t(i) * n * d->inputs, size_t(B) * n * d->inputs * sizeof(float),
+                            hipMemcpyHostToDevice, d->stream));
+    DNCHK(d, hipMemcpyAsync(d->train.tgt, tgt + size_t(i) * n * 3, size_t(B) * n * 3 * sizeof(float),
+                            hipMemcpyHostToDevice, d->stream));
+    if ((rc = train_batch(d, B))) return rc;
+    DNCHK(d, hipStreamSynchronize(d->stream));  // the host's arrays are its own again
   }
   return MDWT_OK;
-}
-
-// upload one (input, target) pair and accumulate its loss gradient
-int one_pair(mdwt_denoiser* d, const float* in, const float* tgt, float inv_count) {
-  const size_t n = size_t(d->H) * d->W;
-  DNCHK(d, hipMemcpyAsync(d->in32, in, n * d->inputs * sizeof(float),
-                          hipMemcpyHostToDevice, d->stream));
-  DNCHK(d, hipMemcpyAsync(d->tgt, tgt, n * 3 * sizeof(float), hipMemcpyHostToDevice, d->stream));
-  int rc = forward(d);
-  if (rc) return rc;
-  DNCHK(d, mdwt::dn::kpn_loss_grad(d->in32, d->inputs, d->out32, d->pred, d->tgt, d->H, d->W,
-                                   inv_count, d->gout, d->err_sum, d->stream));
-  return backward(d);
 }
 
 }  // namespace
@@ -379,6 +540,7 @@ int mdwt_dn_destroy(mdwt_denoiser* d) {
   if (!d) return MDWT_ERR_ARG;
   (void)hipSetDevice(d->device);
   if (d->stream) (void)hipStreamSynchronize(d->stream);
+  free_train(&d->train);
   for (void* p : d->bufs) (void)hipFree(p);
   if (d->ev0) (void)hipEventDestroy(d->ev0);
   if (d->ev1) (void)hipEventDestroy(d->ev1);
@@ -391,9 +553,7 @@ const char* mdwt_dn_last_error(const mdwt_denoiser* d) { return d ? d->err.c_str
 
 int mdwt_dn_num_params(const mdwt_denoiser* d, int* n) {
   if (!d || !n) return MDWT_ERR_ARG;
-  size_t t = 0;
-  for (const Conv& L : d->c) t += L.nw + size_t(L.cout);
-  *n = int(t);
+  *n = int(d->n_params);
   return MDWT_OK;
 }
 
@@ -401,12 +561,7 @@ int mdwt_dn_get_params(mdwt_denoiser* d, float* out) {
   if (!d || !out) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   DNCHK(d, hipStreamSynchronize(d->stream));
-  for (const Conv& L : d->c) {
-    DNCHK(d, hipMemcpy(out, L.w, L.nw * sizeof(float), hipMemcpyDeviceToHost));
-    out += L.nw;
-    DNCHK(d, hipMemcpy(out, L.b, size_t(L.cout) * sizeof(float), hipMemcpyDeviceToHost));
-    out += L.cout;
-  }
+  DNCHK(d, hipMemcpy(out, d->params, d->n_params * sizeof(float), hipMemcpyDeviceToHost));
   return MDWT_OK;
 }
 
@@ -414,12 +569,7 @@ int mdwt_dn_set_params(mdwt_denoiser* d, const float* in) {
   if (!d || !in) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   DNCHK(d, hipStreamSynchronize(d->stream));
-  for (Conv& L : d->c) {
-    DNCHK(d, hipMemcpy(L.w, in, L.nw * sizeof(float), hipMemcpyHostToDevice));
-    in += L.nw;
-    DNCHK(d, hipMemcpy(L.b, in, size_t(L.cout) * sizeof(float), hipMemcpyHostToDevice));
-    in += L.cout;
-  }
+  DNCHK(d, hipMemcpy(d->params, in, d->n_params * sizeof(float), hipMemcpyHostToDevice));
   int rc = refresh_weights(d);
   if (rc) return rc;
   DNCHK(d, hipStreamSynchronize(d->stream));
@@ -455,17 +605,9 @@ int mdwt_dn_gradient(mdwt_denoiser* d, const float* input, const float* target, 
   if (!d || !input || !target || !grad) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   const size_t n = size_t(d->H) * d->W;
-  int rc = zero_grads(d);
+  int rc = loss_gradient(d, input, target, nullptr, 1, 1.f / float(n * 3));
   if (rc) return rc;
-  DNCHK(d, hipMemsetAsync(d->err_sum, 0, sizeof(float), d->stream));
-  if ((rc = one_pair(d, input, target, 1.f / float(n * 3)))) return rc;
-  DNCHK(d, hipStreamSynchronize(d->stream));
-  for (const Conv& L : d->c) {
-    DNCHK(d, hipMemcpy(grad, L.gw, L.nw * sizeof(float), hipMemcpyDeviceToHost));
-    grad += L.nw;
-    DNCHK(d, hipMemcpy(grad, L.gb, size_t(L.cout) * sizeof(float), hipMemcpyDeviceToHost));
-    grad += L.cout;
-  }
+  DNCHK(d, hipMemcpy(grad, d->grads, d->n_params * sizeof(float), hipMemcpyDeviceToHost));
   if (loss) {
     float e = 0.f;
     DNCHK(d, hipMemcpy(&e, d->err_sum, sizeof(float), hipMemcpyDeviceToHost));
@@ -481,25 +623,14 @@ int mdwt_dn_train_step(mdwt_denoiser* d, const float* inputs, const float* targe
     if (!(weights[i] >= 0.f) || std::isinf(weights[i])) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   const size_t n = size_t(d->H) * d->W;
-  int rc = zero_grads(d);
-  if (rc) return rc;
-  DNCHK(d, hipMemsetAsync(d->err_sum, 0, sizeof(float), d->stream));
   const float inv = 1.f / float(n * 3 * size_t(count));
-  for (int i = 0; i < count; ++i) {
-    const float* xi = inputs + size_t(i) * n * d->inputs;
-    const float wi = weights ? inv * weights[i] : inv;
-    if ((rc = one_pair(d, xi, targets + size_t(i) * n * 3, wi))) return rc;
-    DNCHK(d, hipStreamSynchronize(d->stream));  // host inputs are reused by the caller
-  }
+  int rc = loss_gradient(d, inputs, targets, weights, count, inv);
+  if (rc) return rc;
   ++d->step;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   const float c1 = 1.f - std::pow(b1, float(d->step)), c2 = 1.f - std::pow(b2, float(d->step));
-  for (Conv& L : d->c) {
-    DNCHK(d, mdwt::dn::adam(L.w, L.gw, L.mw, L.vw, int(L.nw), lr, b1, b2, c1, c2, eps, nullptr,
-                            d->stream));
-    DNCHK(d, mdwt::dn::adam(L.b, L.gb, L.mb, L.vb, L.cout, lr, b1, b2, c1, c2, eps, nullptr,
-                            d->stream));
-  }
+  DNCHK(d, mdwt::dn::adam(d->params, d->grads, d->mom, d->var, int(d->n_params), lr, b1, b2, c1, c2, eps,
+                          d->stream));
   rc = refresh_weights(d);
   if (rc) return rc;
   float e = 0.f;

@@ -1,7 +1,6 @@
 // Kernels of the learned denoiser (a 3-level U-Net of 3x3 convolutions): BF16
 // activations and weights, FP32 accumulation on the matrix cores
-// (v_mfma_f32_32x32x16_bf16 for the convolutions, v_mfma_f32_32x32x8bf16_1k
-// for the weight gradients), FP32 gradients and Adam state. No reference
+// (v_mfma_f32_32x32x16_bf16), FP32 gradients and Adam state. No reference
 // counterpart (the reference renders plain accumulation only).
 //
 // Tensors are NHWC with a channel stride (so that a convolution can read or
@@ -26,7 +25,6 @@ namespace mdwt {
 namespace dn {
 namespace {
 
-typedef short s4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
@@ -39,10 +37,8 @@ __device__ __forceinline__ uint32_t f2bf2(float lo, float hi) {
 __device__ __forceinline__ uint16_t f2bf(float f) { return uint16_t(f2bf2(f, 0.f)); }
 
 // 4 consecutive bf16 (8 bytes, 8-byte aligned) or zeros
-__device__ __forceinline__ s4 load4(const uint16_t* p, bool ok) {
-  if (!ok) return s4{0, 0, 0, 0};
-  const uint2 v = *reinterpret_cast<const uint2*>(p);
-  return s4{short(v.x & 0xffffu), short(v.x >> 16), short(v.y & 0xffffu), short(v.y >> 16)};
+__device__ __forceinline__ uint2 load4(const uint16_t* p, bool ok) {
+  return ok ? *reinterpret_cast<const uint2*>(p) : make_uint2(0u, 0u);
 }
 
 // Kernel-predicting output (Bako et al. 2017): per pixel, the softmax of
@@ -66,9 +62,6 @@ __device__ __forceinline__ float kpn_weights_z(const float* z, float* w) {
   }
   return sum;
 }
-__device__ __forceinline__ float kpn_weights(const float* logits, int p, float* w) {
-  return kpn_weights_z(logits + size_t(p) * kLogitStride, w);
-}
 // out[0..2] = sum_j softmax(z)_j * rgb(neighbour j) for pixel (py, px)
 __device__ __forceinline__ void kpn_filter(const float* __restrict__ in, int inputs, const float* z,
                                            int py, int px, int H, int W, float* out) {
@@ -89,8 +82,8 @@ __device__ __forceinline__ void kpn_filter(const float* __restrict__ in, int inp
 
 // y = conv3x3(x) (+ bias, ReLU) on v_mfma_f32_32x32x16_bf16: weights w
 // [9][cout_pad][cin] (tap-major, K contiguous); output channel n of pixel p
-// to y16[p * ys + yo + n] (bf16) and/or y32[p * ys + yo + n] (fp32, added to
-// the existing value when accum); channels n >= cout are not written.
+// to y16[p * ys + yo + n] (bf16) and/or y32[p * ys + yo + n] (fp32, fp32);
+// channels n >= cout are not written.
 //
 // A workgroup (4 waves, WX along x by WR along rows) computes R = 2 WR image
 // rows x TP = 32 WX pixels x TN = 32 NT output channels; each wave 2 rows x
@@ -112,6 +105,16 @@ __device__ __forceinline__ void kpn_filter(const float* __restrict__ in, int inp
 // the stored bf16 output to pool16 (stride ps), as pool_kernel computes it.
 // kEpiKpn stages the fp32 logits of the tile in LDS and applies the
 // kernel-predicting filter (as kpn_apply_kernel) to write pred directly.
+// Training (a batch of nimg images, each with its own zero border):
+// kEpiKpnLoss goes on from the filtered colour to the squared error against
+// target (summed into err) and its gradient with respect to the logits, stored
+// as the bf16 the backward convolutions read; the three gradient epilogues turn
+// an input gradient straight into the next layer's masked bf16 gradient
+// (act > 0 is the ReLU's derivative there): kEpiMask at the same resolution;
+// kEpiUpGrad through the upsampling (channels < cu: the 2 x 2 sum) and the skip
+// (channels >= cu: fp32 to y32); kEpiPoolGrad through the 2 x 2 mean, onto the
+// skip's fp32 gradient. No fp32 gradient of an activation but the two skips'
+// goes through memory, and no element-wise kernel is left in the step.
 constexpr int kChunk = 32;   // input channels per staged chunk
 constexpr int kPitch = 40;   // LDS row (bf16): 32 channels + 8 padding
 constexpr int kZPitch = kLogitStride + 1;  // LDS row (fp32) of one pixel's logits
@@ -148,6 +151,63 @@ __device__ __forceinline__ void kpn_filter_tile(const float* z, const float* rgb
   out[0] = r * inv;
   out[1] = g * inv;
   out[2] = b * inv;
+}
+
+// The filtered colour of one pixel as kpn_filter_tile gives it, its squared
+// error against target (returned) and the gradient of inv_count times the
+// error with respect to the logits, dz_j = w_j (c_j - pred) . gpred with gpred
+// = 2 inv_count (pred - target), as bf16 into gz (zero past kTaps). The logits z
+// (in LDS) are overwritten by their weights: kept in registers, the 49 weights
+// spilled 95 VGPRs.
+__device__ __forceinline__ float kpn_loss_tile(float* z, const float* rgb, int pitch,
+                                               const float* target, float inv_count, uint16_t* gz) {
+  float m = z[0];
+  for (int j = 1; j < kTaps; ++j) m = fmaxf(m, z[j]);
+  float sum = 0.f, r = 0.f, g = 0.f, b = 0.f;
+#pragma unroll 7
+  for (int j = 0; j < kTaps; ++j) {
+    const float w = __expf(z[j] - m);
+    z[j] = w;
+    sum += w;
+    const float* c = rgb + ((j / kKernel) * pitch + j % kKernel) * 3;
+    r += w * c[0];
+    g += w * c[1];
+    b += w * c[2];
+  }
+  const float inv = 1.f / sum;
+  const float pr = r * inv, pg = g * inv, pb = b * inv;
+  const float dr = pr - target[0], dg = pg - target[1], db = pb - target[2];
+  const float s = 2.f * inv_count;
+  const float gr = s * dr, gg = s * dg, gb = s * db;
+  const float base = pr * gr + pg * gg + pb * gb;
+#pragma unroll
+  for (int j0 = 0; j0 < kLogitStride; j0 += 8) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int j = j0 + e;
+      v[e] = 0.f;
+      if (j < kTaps) {
+        const float* c = rgb + ((j / kKernel) * pitch + j % kKernel) * 3;
+        v[e] = z[j] * inv * (c[0] * gr + c[1] * gg + c[2] * gb - base);
+      }
+    }
+    *reinterpret_cast<uint4*>(gz + j0) =
+        make_uint4(f2bf2(v[0], v[1]), f2bf2(v[2], v[3]), f2bf2(v[4], v[5]), f2bf2(v[6], v[7]));
+  }
+  return dr * dr + dg * dg + db * db;
+}
+
+// lane l ^ 1's value (DPP quad_perm [1, 0, 3, 2])
+__device__ __forceinline__ float lane_xor1(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, false));
+}
+// 4 gradient values through a ReLU whose output is act, as bf16
+__device__ __forceinline__ void store_masked(uint16_t* y, const uint16_t* act, const float v[4]) {
+  const uint2 k = *reinterpret_cast<const uint2*>(act);
+  const float m0 = bf2f(uint16_t(k.x)) > 0.f ? v[0] : 0.f, m1 = bf2f(uint16_t(k.x >> 16)) > 0.f ? v[1] : 0.f;
+  const float m2 = bf2f(uint16_t(k.y)) > 0.f ? v[2] : 0.f, m3 = bf2f(uint16_t(k.y >> 16)) > 0.f ? v[3] : 0.f;
+  *reinterpret_cast<uint2*>(y) = make_uint2(f2bf2(m0, m1), f2bf2(m2, m3));
 }
 
 // The MFMAs of one staged chunk for waves of one 32-channel tile: 9 taps x
@@ -194,14 +254,17 @@ template <int WX, int WR, int NT, int SRC, int EPI>
 __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
   using S = ConvShape<WX, WR, NT>;
   constexpr int RW = S::RW, R = S::R, TP = S::TP, XP = S::XP, TN = S::TN;
-  static_assert(EPI != kEpiKpn || (R * TP * kZPitch + (R + 2 * kKernelRadius) *
+  constexpr bool kKpn = EPI == kEpiKpn || EPI == kEpiKpnLoss;
+  static_assert(!kKpn || (R * TP * kZPitch + (R + 2 * kKernelRadius) *
                                                       (TP + 2 * kKernelRadius) * 3) * 4 <= S::kLds * 2,
                 "filter tile");
   __shared__ __align__(16) uint16_t lds[S::kLds];
   uint16_t* sA = lds;
   uint16_t* sB = lds + S::kARows * kPitch;
   const int t = threadIdx.x, l = t & 63, wv = t >> 6;
-  const int tiles_x = (a.W + TP - 1) / TP, ntiles = tiles_x * ((a.H + R - 1) / R);
+  const int tiles_x = (a.W + TP - 1) / TP, tiles_img = tiles_x * ((a.H + R - 1) / R);
+  const int ntiles = tiles_img * a.nimg;
+  const uint32_t img_px = uint32_t(a.H) * uint32_t(a.W);
   const int n0 = blockIdx.y * TN;
   const int wx = wv % WX, wr = wv / WX;
   const int r32 = l & 31, kh = (l >> 5) * 8, kq = (l >> 5) * 4;
@@ -224,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
   if (first >= last) return;
   // one chunk of input channels: the weights stay in LDS for every tile
   // (not with the filter epilogue, whose logits overwrite them)
-  const bool b_once = EPI != kEpiKpn && a.cin <= kChunk;
+  const bool b_once = !kKpn && a.cin <= kChunk;
 
   uint4 pa[S::kAPer], pb[S::kBPer];
   // kSrcF32: the fp32 network input, 8 values per granule, converted to
@@ -232,7 +295,9 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
   constexpr int kF32 = SRC == kSrcF32 ? S::kAPer : 1;
   float pf[kF32][8];
   auto fetch = [&](int tile, int kc, bool with_b) {
-    const int y0 = (tile / tiles_x) * R, x0 = (tile % tiles_x) * TP;
+    const int img = tile / tiles_img, it = tile - img * tiles_img;
+    const int y0 = (it / tiles_x) * R, x0 = (it % tiles_x) * TP;
+    const uint32_t p0 = uint32_t(img) * img_px;  // first pixel of the image
 #pragma unroll
     for (int i = 0; i < S::kAPer; ++i) {
       const int f = t + 256 * i;
@@ -245,7 +310,8 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
         const int sy = y0 + row - 1, sx = x0 + px - 1, c = kc + 8 * g;
         if (sy >= 0 && sy < a.H && sx >= 0 && sx < a.W && c < a.cin) {
           if constexpr (SRC == kSrcF32) {
-            const float* q = a.kin + (uint32_t(sy) * uint32_t(a.W) + uint32_t(sx)) * uint32_t(a.inputs);
+            const float* q =
+                a.kin + (p0 + uint32_t(sy) * uint32_t(a.W) + uint32_t(sx)) * uint32_t(a.inputs);
 #pragma unroll
             for (int e = 0; e < 8; ++e)
               if (c + e < a.inputs) pf[i][e] = q[c + e];
@@ -253,10 +319,10 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
           }
           const uint16_t* p;
           if (SRC == kSrcUpCat && c < a.cu)
-            p = a.xl + (uint32_t(sy >> 1) * uint32_t(a.W >> 1) + uint32_t(sx >> 1)) * uint32_t(a.cu) +
+            p = a.xl + (p0 / 4u + uint32_t(sy >> 1) * uint32_t(a.W >> 1) + uint32_t(sx >> 1)) * uint32_t(a.cu) +
                 uint32_t(c);
           else
-            p = a.x + (uint32_t(sy) * uint32_t(a.W) + uint32_t(sx)) * uint32_t(a.xs) +
+            p = a.x + (p0 + uint32_t(sy) * uint32_t(a.W) + uint32_t(sx)) * uint32_t(a.xs) +
                 uint32_t(a.xo + (SRC == kSrcUpCat ? c - a.cu : c));
           pa[i] = *reinterpret_cast<const uint4*>(p);
         }
@@ -301,6 +367,7 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
   for (int r = 0; r < RW; ++r)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[r][j] = f16v{};
+  [[maybe_unused]] float err = 0.f;  // kEpiKpnLoss: this thread's squared error
   // stages (tile, chunk) in order; the next stage's granules are loaded while
   // the current one is multiplied and while the finished tile is stored
   int tile = first, kc = 0;
@@ -346,13 +413,15 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
     }
     __syncthreads();
     if (nkc == 0) {  // the tile is complete
-      const int y0 = (tile / tiles_x) * R, x0 = (tile % tiles_x) * TP;
+      const int img = tile / tiles_img, it = tile - img * tiles_img;
+      const int y0 = (it / tiles_x) * R, x0 = (it % tiles_x) * TP;
+      const uint32_t p0 = uint32_t(img) * img_px;
       // acc[r][j]: D = weights x pixels, so lane l holds pixel r32 of row
       // y0 + wr * RW + r and, in register v, output channel
       // j * 32 + (v / 4) * 8 + kq + v % 4: four consecutive channels per
       // register group
       const int px = x0 + wx * 32 + r32;
-      if constexpr (EPI == kEpiKpn) {
+      if constexpr (kKpn) {
         // logits (fp32, kLogitStride per pixel; n0 == 0, TN == kLogitStride)
         // of the tile into LDS, and after them the input colours of the tile
         // with a kKernelRadius halo (coordinates clamped to the image); then
@@ -369,7 +438,7 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
             const int iy = q / kRgbCols, ix = q - iy * kRgbCols;
             const int sy = min(max(y0 - kKernelRadius + iy, 0), a.H - 1);
             const int sx = min(max(x0 - kKernelRadius + ix, 0), a.W - 1);
-            const float* c = a.kin + (size_t(sy) * a.W + sx) * a.inputs;
+            const float* c = a.kin + (size_t(p0) + size_t(sy) * a.W + sx) * a.inputs;
             cr[i][0] = c[0];
             cr[i][1] = c[1];
             cr[i][2] = c[2];
@@ -401,11 +470,77 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
         __syncthreads();
         for (int pl = t; pl < R * TP; pl += 256) {
           const int ly = pl / TP, lx = pl % TP, py = y0 + ly, qx = x0 + lx;
-          if (py >= a.H || qx >= a.W) continue;
-          kpn_filter_tile(sz + pl * kZPitch, srgb + (ly * kRgbCols + lx) * 3, kRgbCols,
-                          a.pred + (size_t(py) * a.W + qx) * 3);
+          const bool in = py < a.H && qx < a.W;
+          const size_t p = size_t(p0) + size_t(py) * a.W + qx;
+          const float* rgb = srgb + (ly * kRgbCols + lx) * 3;
+          if constexpr (EPI == kEpiKpn) {
+            if (in) kpn_filter_tile(sz + pl * kZPitch, rgb, kRgbCols, a.pred + p * 3);
+          } else {
+            if (in)
+              err += kpn_loss_tile(sz + pl * kZPitch, rgb, kRgbCols, a.target + p * 3,
+                                   a.inv_count[img], a.y16 + p * kLogitStride);
+          }
         }
         __syncthreads();  // before the next stage overwrites the logits
+      } else if constexpr (EPI == kEpiMask || EPI == kEpiUpGrad || EPI == kEpiPoolGrad) {
+        const int y = y0 + wr * RW;
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+          for (int gq = 0; gq < 4; ++gq) {
+            const int n = n0 + j * 32 + gq * 8 + kq;  // channels n .. n + 3 (cout % 4 == 0)
+            if constexpr (EPI == kEpiMask) {
+#pragma unroll
+              for (int r = 0; r < RW; ++r) {
+                if (y + r >= a.H || px >= a.W || n >= a.cout) continue;
+                const uint32_t o = (p0 + uint32_t(y + r) * uint32_t(a.W) + uint32_t(px)) *
+                                       uint32_t(a.ys) + uint32_t(n);
+                const float v[4] = {acc[r][j][gq * 4], acc[r][j][gq * 4 + 1], acc[r][j][gq * 4 + 2],
+                                    acc[r][j][gq * 4 + 3]};
+                store_masked(a.y16 + o, a.act + o, v);
+              }
+            } else if constexpr (EPI == kEpiUpGrad) {
+              if (n0 + j * 32 < a.cu) {  // whole 32-channel tiles on either side
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                  const float u0 = acc[0][j][gq * 4 + e], u1 = acc[1][j][gq * 4 + e];
+                  v[e] = u0 + lane_xor1(u0) + u1 + lane_xor1(u1);
+                }
+                if ((r32 & 1) == 0 && y < a.H && px < a.W) {
+                  const uint32_t o = (p0 / 4u + uint32_t(y >> 1) * uint32_t(a.W >> 1) + uint32_t(px >> 1)) *
+                                         uint32_t(a.cu) + uint32_t(n);
+                  store_masked(a.y16 + o, a.act + o, v);
+                }
+              } else {
+#pragma unroll
+                for (int r = 0; r < RW; ++r) {
+                  if (y + r >= a.H || px >= a.W || n >= a.cout) continue;
+                  const uint32_t o = (p0 + uint32_t(y + r) * uint32_t(a.W) + uint32_t(px)) *
+                                         uint32_t(a.ys) + uint32_t(n - a.cu);
+                  *reinterpret_cast<float4*>(a.y32 + o) =
+                      make_float4(acc[r][j][gq * 4], acc[r][j][gq * 4 + 1], acc[r][j][gq * 4 + 2],
+                                  acc[r][j][gq * 4 + 3]);
+                }
+              }
+            } else {
+#pragma unroll
+              for (int r = 0; r < RW; ++r) {
+                if (y + r >= a.H || px >= a.W || n >= a.cout) continue;
+                const float v[4] = {acc[r][j][gq * 4], acc[r][j][gq * 4 + 1], acc[r][j][gq * 4 + 2],
+                                    acc[r][j][gq * 4 + 3]};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  const uint32_t o = (4u * p0 + uint32_t(2 * (y + r) + (q >> 1)) * uint32_t(2 * a.W) +
+                                      uint32_t(2 * px + (q & 1))) * uint32_t(a.ys) + uint32_t(n);
+                  const float4 sk = *reinterpret_cast<const float4*>(a.skip + o);
+                  const float u[4] = {sk.x + 0.25f * v[0], sk.y + 0.25f * v[1], sk.z + 0.25f * v[2],
+                                      sk.w + 0.25f * v[3]};
+                  store_masked(a.y16 + o, a.act + o, u);
+                }
+              }
+            }
+          }
       } else {
         const int y = y0 + wr * RW;  // even: R and RW are
 #pragma unroll
@@ -429,23 +564,16 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
               if (y + r >= a.H || px >= a.W || n >= a.cout) continue;
               // element offsets stay below 2^31 (at most 2^24 pixels x 96
               // channels at full resolution, 160 at half)
-              const uint32_t o = (uint32_t(y + r) * uint32_t(a.W) + uint32_t(px)) * uint32_t(a.ys) +
+              const uint32_t o = (p0 + uint32_t(y + r) * uint32_t(a.W) + uint32_t(px)) * uint32_t(a.ys) +
                                  uint32_t(a.yo + n);
               if (n + 3 < a.cout) {  // 8-byte bf16 / 16-byte fp32 stores
                 if (a.y16) *reinterpret_cast<uint2*>(a.y16 + o) = make_uint2(o16[r][0], o16[r][1]);
-                if (a.y32) {
-                  float4* q = reinterpret_cast<float4*>(a.y32 + o);
-                  float4 v4 = make_float4(o32[0], o32[1], o32[2], o32[3]);
-                  if (a.accum) {
-                    const float4 old = *q;
-                    v4 = make_float4(old.x + v4.x, old.y + v4.y, old.z + v4.z, old.w + v4.w);
-                  }
-                  *q = v4;
-                }
+                if (a.y32)
+                  *reinterpret_cast<float4*>(a.y32 + o) = make_float4(o32[0], o32[1], o32[2], o32[3]);
               } else {
                 for (int e = 0; n + e < a.cout; ++e) {
                   if (a.y16) a.y16[o + e] = uint16_t(o16[r][e >> 1] >> ((e & 1) * 16));
-                  if (a.y32) a.y32[o + e] = a.accum ? a.y32[o + e] + o32[e] : o32[e];
+                  if (a.y32) a.y32[o + e] = o32[e];
                 }
               }
             }
@@ -468,7 +596,7 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
                   mf[e] = 0.25f * s;
                 }
                 const uint32_t m01 = f2bf2(mf[0], mf[1]), m23 = f2bf2(mf[2], mf[3]);
-                const uint32_t o = (uint32_t(y >> 1) * uint32_t(a.W >> 1) + uint32_t(px >> 1)) *
+                const uint32_t o = (p0 / 4u + uint32_t(y >> 1) * uint32_t(a.W >> 1) + uint32_t(px >> 1)) *
                                        uint32_t(a.ps) + uint32_t(n);
                 if (n + 3 < a.cout)
                   *reinterpret_cast<uint2*>(a.pool16 + o) = make_uint2(m01, m23);
@@ -488,107 +616,195 @@ __global__ __launch_bounds__(256, 2) void conv_kernel(ConvArgs a) {
     tile = ntile;
     kc = nkc;
   }
+  if constexpr (EPI == kEpiKpnLoss) {
+    for (int o = 32; o > 0; o >>= 1) err += __shfl_down(err, o, 64);
+    if (l == 0) atomicAdd(a.err, err);
+  }
 }
 
-// Weight gradient, GEMM M = output channels, N = input channels, K =
-// pixels:
-//   part[band][tap][co][ci] = sum over the band's pixels p of g[p][co] * x[p + tap][ci]
-// g: bf16 [H*W][gs] (the masked output gradient), x: bf16 [H*W][xs] channels
-// xo .. xo+cin. One wave per (ci tile, co tile, band of image rows, tap row
-// dy): the 3 taps of one row share the staged input. Each 32-pixel row
-// segment is staged through LDS once: the gradient tile transposed ([co][px],
-// so a lane's 4 consecutive pixels are one 8-byte read) and the input row
-// y + dy with a one-pixel halo ([ci][px + 1]); the 3 taps read shifted
-// windows of it. Bands write partial sums, which wgrad_reduce_kernel adds
-// into dw in a fixed order (no atomics).
-constexpr int kSeg = 32;         // pixels per row segment: 4 MFMA K steps
-constexpr int kRow = kSeg + 4;   // LDS row (u16): kSeg + 2 pixels, 8-byte multiple
+// Weight gradient, GEMM M = output channels, N = input channels, K = pixels:
+//   part[wg][tap][co][ci] = sum over the workgroup's pixels p of g[p][co] * x[p + tap][ci]
+//   part[wg][9 * cout * cin + co] = sum of g[p][co] (the bias gradient)
+// g: bf16 [image][H*W][gs] (the masked output gradient), x: the layer's input
+// (for a concatenated input the channels < cu are the half-resolution tensor
+// xl's, nearest upsampled, so nothing is materialised).
+//
+// A wave owns one (32 output x 32 input channels) tile with all nine taps
+// (9 accumulators of 32 x 32) and walks down units of 32 columns x kUnitRows
+// rows of an image: per row it stages one gradient row and one new input row
+// (the last two stay in a ring of three), transposed to [channel][pixel], and
+// multiplies 2 K steps x 9 taps. The MFMA needs 8 consecutive pixels of a
+// channel per lane: a lane loads 4 pixels x 4 channels, transposes them in
+// registers (v_perm) and writes 4 pixels of a channel with one 8-byte store;
+// the taps' one- and two-pixel shifts are funnel shifts of one 16 + 4-byte read.
+// Per row 18 MFMAs stand against about 130 VALU and 30 LDS instructions. The
+// next row is loaded into registers while the current one is multiplied; waves
+// share nothing until their four sums are added (in order) at the end, so the
+// result does not depend on scheduling. The eleven layers of a step on 8 x
+// 256^2: 2591 us with one tap row per wave, element-by-element transposed
+// staging and an image at a time, 451 us so (124 GFLOP: 275 TFLOP/s), the bias
+// sums (753 + 440 us as kernels of their own) included.
+// orders a wave's own LDS writes and reads (its lanes exchange rows through it)
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+constexpr int kSeg = 32;       // columns of a unit: 2 MFMA K steps
+constexpr int kUnitRows = 8;   // rows of a unit (2 more input rows are staged)
+constexpr int kWPitch = 40;    // LDS row: 34 pixels, 16-byte reads, conflict-free as kPitch
 
-__global__ __launch_bounds__(64) void wgrad_band_kernel(const uint16_t* __restrict__ g, int gs,
-                                                        const uint16_t* __restrict__ x, int xs,
-                                                        int xo, int H, int W, int cin, int cout,
-                                                        int rows, float* __restrict__ part) {
-  __shared__ __align__(16) uint16_t gT[32 * kRow];
-  __shared__ __align__(16) uint16_t xT[32 * kRow];
-  const int l = threadIdx.x;
+// rows (pixels) of 4 channels -> rows (channels) of 4 pixels
+__device__ __forceinline__ void transpose4(const uint2 p[4], uint2 c[4]) {
+  c[0] = make_uint2(__builtin_amdgcn_perm(p[1].x, p[0].x, 0x05040100u),
+                    __builtin_amdgcn_perm(p[3].x, p[2].x, 0x05040100u));
+  c[1] = make_uint2(__builtin_amdgcn_perm(p[1].x, p[0].x, 0x07060302u),
+                    __builtin_amdgcn_perm(p[3].x, p[2].x, 0x07060302u));
+  c[2] = make_uint2(__builtin_amdgcn_perm(p[1].y, p[0].y, 0x05040100u),
+                    __builtin_amdgcn_perm(p[3].y, p[2].y, 0x05040100u));
+  c[3] = make_uint2(__builtin_amdgcn_perm(p[1].y, p[0].y, 0x07060302u),
+                    __builtin_amdgcn_perm(p[3].y, p[2].y, 0x07060302u));
+}
+
+__global__ __launch_bounds__(256, 2) void wgrad_kernel(WgradArgs a) {
+  constexpr int kRowsG = 32 * kWPitch;  // one staged row of 32 channels
+  constexpr int kWave = 4 * kRowsG;     // gradient row + ring of three input rows
+  __shared__ __align__(16) uint16_t lds[4 * kWave];
+  static_assert(9 * 32 * 32 * 4 + 32 * 4 <= int(sizeof(lds)), "the waves' sums are added in the same LDS");
+  const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ci0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
-  const int band = blockIdx.z / 3, dyi = blockIdx.z % 3;
-  const int y0 = band * rows, y1 = min(H, y0 + rows);
-  const int r32 = l & 31, kq = (l >> 5) * 4;
-  f16v acc[3] = {f16v{}, f16v{}, f16v{}};
-  // stages: (row y, 32-pixel segment) in row order; the next stage's
-  // gradient (32 px x 8 groups of 4 channels) and input row y + dy - 1
-  // (34 px x 8 groups) are loaded into registers while this one is multiplied
-  constexpr int kGPer = kSeg * 8 / 64, kXPer = ((kSeg + 2) * 8 + 63) / 64;
-  const int segs = (W + kSeg - 1) / kSeg;
-  const int nst = (y1 - y0) * segs;
-  s4 pg[kGPer], pxv[kXPer];
-  auto fetch = [&](int st) {
-    const int y = y0 + st / segs, x0 = (st % segs) * kSeg, sy = y + dyi - 1;
+  const int r32 = l & 31, kh = (l >> 5) * 8, kq = (l >> 5) * 4;
+  const int pg = l & 7, cg = l >> 3;  // this lane's 4 pixels and 4 channels of a staged row
+  uint16_t* sg = lds + wave * kWave;
+  uint16_t* sx = sg + kRowsG;
+  const bool up = ci0 < a.cu;
+  const uint16_t* xb = up ? a.xl + ci0 : a.x + a.xo + ci0 - a.cu;
+  const int xs = up ? a.cu : a.xs, sh = up ? 1 : 0, xw = a.W >> sh;
+  const bool g_ok = co0 + 4 * cg < a.gs, x_ok = ci0 + 4 * cg < a.xc;
+  const int segs = (a.W + kSeg - 1) / kSeg, nb = (a.H + kUnitRows - 1) / kUnitRows;
+  const int units = a.nimg * nb * segs;
+
+  f16v acc[9], accb = f16v{};
 #pragma unroll
-    for (int i = 0; i < kGPer; ++i) {
-      const int idx = l + 64 * i, px = idx >> 3, grp = idx & 7, c = co0 + grp * 4, xx = x0 + px;
-      pg[i] = load4(g + (size_t(y) * W + xx) * gs + c, xx < W && c < cout);
-    }
+  for (int t = 0; t < 9; ++t) acc[t] = f16v{};
+  const bf8 ones = {__bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f),
+                    __bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f)};
+
+  for (int unit = int(blockIdx.z) * 4 + wave; unit < units; unit += int(gridDim.z) * 4) {
+    const int seg = unit % segs, rest = unit / segs, band = rest % nb, img = rest / nb;
+    const int x0 = seg * kSeg, y0 = band * kUnitRows, y1 = min(a.H, y0 + kUnitRows);
+    const uint16_t* gi = a.g + size_t(img) * a.H * a.W * a.gs + co0 + 4 * cg;
+    const uint16_t* xi = xb + size_t(img) * ((a.H >> sh) * size_t(xw)) * xs + 4 * cg;
+    uint2 rg[4], rx[4], rh[2];
+    auto load_g = [&](int y) {
 #pragma unroll
-    for (int i = 0; i < kXPer; ++i) {
-      const int idx = l + 64 * i, grp = idx & 7, px = idx >> 3;
-      const int sx = x0 + px - 1, c = ci0 + grp * 4;
-      const bool in = idx < (kSeg + 2) * 8 && sy >= 0 && sy < H && sx >= 0 && sx < W && c < cin;
-      pxv[i] = load4(x + (size_t(in ? sy * W + sx : 0) * xs + xo + (in ? c : 0)), in);
-    }
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int i = 0; i < kGPer; ++i) {
-      const int idx = l + 64 * i, px = idx >> 3, grp = idx & 7, c = co0 + grp * 4;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        gT[(grp * 4 + j) * kRow + px] = c + j < cout ? uint16_t(pg[i][j]) : uint16_t(0);
-    }
-#pragma unroll
-    for (int i = 0; i < kXPer; ++i) {
-      const int idx = l + 64 * i, grp = idx & 7, px = idx >> 3, c = ci0 + grp * 4;
-      if (idx >= (kSeg + 2) * 8) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        xT[(grp * 4 + j) * kRow + px] = c + j < cin ? uint16_t(pxv[i][j]) : uint16_t(0);
-    }
-  };
-  if (nst > 0) fetch(0);
-  for (int st = 0; st < nst; ++st) {
-    store();
-    __syncthreads();
-    if (st + 1 < nst) fetch(st + 1);
-#pragma unroll
-    for (int ks = 0; ks < kSeg / 8; ++ks) {
-      const int kb = ks * 8 + kq;  // this lane's 4 pixels of the K step
-      const s4 a = *reinterpret_cast<const s4*>(&gT[r32 * kRow + kb]);
-#pragma unroll
-      for (int dx = 0; dx < 3; ++dx) {
-        const uint16_t* xr = &xT[r32 * kRow + kb + dx];
-        const s4 b = s4{short(xr[0]), short(xr[1]), short(xr[2]), short(xr[3])};
-        acc[dx] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc[dx], 0, 0, 0);
+      for (int i = 0; i < 4; ++i) {
+        const int px = x0 + 4 * pg + i;
+        rg[i] = load4(gi + (size_t(y) * a.W + px) * a.gs, g_ok && y < y1 && px < a.W);
       }
+    };
+    // staged position s of an input row is column x0 - 1 + s, s = 0 .. 33
+    auto load_x = [&](int y) {
+      const bool row = x_ok && y >= 0 && y < a.H;
+      const uint16_t* q = xi + size_t(row ? y >> sh : 0) * xw * xs;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int px = x0 - 1 + 4 * pg + i;
+        rx[i] = load4(q + size_t(px >> sh) * xs, row && px >= 0 && px < a.W);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int px = x0 + kSeg - 1 + i;
+        rh[i] = load4(q + size_t(px >> sh) * xs, row && pg == 0 && px < a.W);
+      }
+    };
+    auto store_g = [&]() {
+      uint2 c[4];
+      transpose4(rg, c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2*>(sg + (4 * cg + j) * kWPitch + 4 * pg) = c[j];
+    };
+    auto store_x = [&](int slot) {
+      uint16_t* q = sx + slot * kRowsG + 4 * cg * kWPitch;
+      uint2 c[4];
+      transpose4(rx, c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) *reinterpret_cast<uint2*>(q + j * kWPitch + 4 * pg) = c[j];
+      if (pg == 0) {
+        const uint2 h[4] = {rh[0], rh[1], make_uint2(0u, 0u), make_uint2(0u, 0u)};
+        transpose4(h, c);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<uint32_t*>(q + j * kWPitch + kSeg) = c[j].x;
+      }
+    };
+    int slot = 0;  // ring slot of row y - 1 (y: the row being multiplied)
+    load_x(y0 - 1);
+    store_x(0);
+    load_x(y0);
+    store_x(1);
+    load_x(y0 + 1);
+    load_g(y0);
+    for (int y = y0; y < y1; ++y) {
+      store_x(slot == 0 ? 2 : slot - 1);  // row y + 1
+      store_g();
+      wave_lds_sync();
+      load_x(y + 2);
+      load_g(y + 1);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        const bf8 fg = lds_frag(sg + r32 * kWPitch + 16 * ks + kh);
+        if (ci0 == 0) accb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg, ones, accb, 0, 0, 0);
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy) {
+          const int sl = slot + dy >= 3 ? slot + dy - 3 : slot + dy;
+          const uint16_t* q = sx + sl * kRowsG + r32 * kWPitch + 16 * ks + kh;
+          const uint4 w = *reinterpret_cast<const uint4*>(q);
+          const uint32_t w4 = *reinterpret_cast<const uint32_t*>(q + 8);
+          const uint4 s1 = make_uint4(__builtin_amdgcn_alignbit(w.y, w.x, 16), __builtin_amdgcn_alignbit(w.z, w.y, 16),
+                                      __builtin_amdgcn_alignbit(w.w, w.z, 16), __builtin_amdgcn_alignbit(w4, w.w, 16));
+          const uint4 s2 = make_uint4(w.y, w.z, w.w, w4);
+          acc[dy * 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg, __builtin_bit_cast(bf8, w), acc[dy * 3], 0, 0, 0);
+          acc[dy * 3 + 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg, __builtin_bit_cast(bf8, s1), acc[dy * 3 + 1], 0, 0, 0);
+          acc[dy * 3 + 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg, __builtin_bit_cast(bf8, s2), acc[dy * 3 + 2], 0, 0, 0);
+        }
+      }
+      wave_lds_sync();
+      slot = slot == 2 ? 0 : slot + 1;
     }
+  }
+  // the four waves' sums, in order
+  float* red = reinterpret_cast<float*>(lds);
+  float* redb = red + 9 * 32 * 32;
+  for (int w = 0; w < 4; ++w) {
     __syncthreads();
-  }
-  const int ci = ci0 + r32;
-  if (ci >= cin) return;
+    if (wave == w) {
 #pragma unroll
-  for (int dx = 0; dx < 3; ++dx) {
-    const int tap = dyi * 3 + dx;
+      for (int t = 0; t < 9; ++t)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int co = co0 + (v >> 2) * 8 + kq + (v & 3);
-      if (co < cout) part[((size_t(band) * 9 + tap) * cout + co) * cin + ci] = acc[dx][v];
+        for (int v = 0; v < 16; ++v) {
+          float* o = red + (t * 32 + (v >> 2) * 8 + kq + (v & 3)) * 32 + r32;
+          *o = w == 0 ? acc[t][v] : *o + acc[t][v];
+        }
+      if (r32 == 0)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          float* o = redb + (v >> 2) * 8 + kq + (v & 3);
+          *o = w == 0 ? accb[v] : *o + accb[v];
+        }
     }
   }
+  __syncthreads();
+  float* part = a.part + size_t(blockIdx.z) * (size_t(9) * a.cout * a.cin + a.cout);
+  for (int i = threadIdx.x; i < 9 * 32 * 32; i += 256) {
+    const int ci = ci0 + (i & 31), co = co0 + ((i >> 5) & 31), t = i >> 10;
+    if (ci < a.cin && co < a.cout) part[(size_t(t) * a.cout + co) * a.cin + ci] = red[i];
+  }
+  if (ci0 == 0 && threadIdx.x < 32 && co0 + int(threadIdx.x) < a.cout)
+    part[size_t(9) * a.cout * a.cin + co0 + threadIdx.x] = redb[threadIdx.x];
 }
 
-// dw[i] += sum over bands of part[band][i]. Block: 16 consecutive outputs x
-// 16 band groups (group g sums bands g, g + 16, ...); the groups are then
-// added in order, so the result does not depend on scheduling.
+// dw[i] += sum over the workgroups of part[wg][i]. Block: 16 consecutive
+// outputs x 16 groups (group g sums workgroups g, g + 16, ...); the groups are
+// then added in order, so the result does not depend on scheduling.
 __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restrict__ part,
                                                            int bands, int n,
                                                            float* __restrict__ dw) {
@@ -607,48 +823,6 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const float* __restri
   }
 }
 
-// gm = bf16(gy * (y > 0)) for ReLU layers (gy * 1 otherwise).
-// gy: fp32 [n][gs]; y: bf16 [n][ys] at offset yo; gm: bf16 [n][cout_pad]
-// (channels >= cout zeroed). One thread per (pixel, channel).
-__global__ void relu_grad_kernel(const float* __restrict__ gy, int gs,
-                                 const uint16_t* __restrict__ y, int ys, int yo, int npix,
-                                 int cout, int cout_pad, int relu, uint16_t* gm) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= npix * cout_pad) return;
-  const int p = i / cout_pad, c = i - p * cout_pad;
-  float v = 0.f;
-  if (c < cout) {
-    v = gy[size_t(p) * gs + c];
-    if (relu && !(bf2f(y[size_t(p) * ys + yo + c]) > 0.f)) v = 0.f;
-  }
-  gm[size_t(p) * cout_pad + c] = f2bf(v);
-}
-
-// part[chunk][c] = sum over a chunk of pixels of gm[p][c]: block (c, chunk),
-// 256 threads, a fixed-order reduction inside the block
-__global__ __launch_bounds__(256) void bias_grad_kernel(const uint16_t* __restrict__ gm,
-                                                        int cout_pad, int npix, int chunk,
-                                                        float* __restrict__ part) {
-  __shared__ float sums[4];
-  const int c = blockIdx.x;
-  const int p0 = blockIdx.y * chunk, p1 = min(npix, p0 + chunk);
-  float sum = 0.f;
-  for (int p = p0 + int(threadIdx.x); p < p1; p += blockDim.x) sum += bf2f(gm[size_t(p) * cout_pad + c]);
-  for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o, 64);
-  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = sum;
-  __syncthreads();
-  if (threadIdx.x == 0) part[size_t(blockIdx.y) * gridDim.x + c] = sums[0] + sums[1] + sums[2] + sums[3];
-}
-// db[c] += sum over chunks of part[chunk][c], chunks in order (no atomics)
-__global__ void bias_reduce_kernel(const float* __restrict__ part, int chunks, int cout,
-                                   float* __restrict__ db) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cout) return;
-  float sum = 0.f;
-  for (int k = 0; k < chunks; ++k) sum += part[size_t(k) * cout + c];
-  db[c] += sum;
-}
-
 // 2x2 average pool: y[(py, px)] = mean of x over the 2x2 block (bf16, C channels)
 __global__ void pool_kernel(const uint16_t* x, int H, int W, int C, uint16_t* y) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -659,28 +833,12 @@ __global__ void pool_kernel(const uint16_t* x, int H, int W, int C, uint16_t* y)
   const float s = bf2f(x[b]) + bf2f(x[b + C]) + bf2f(x[b + size_t(W) * C]) + bf2f(x[b + size_t(W) * C + C]);
   y[i] = f2bf(0.25f * s);
 }
-// gx[p] += gy[p / 2] / 4 (fp32; gx channel stride C)
-__global__ void pool_grad_kernel(const float* gy, int H, int W, int C, float* gx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= H * W * C) return;
-  const int c = i % C, p = i / C, py = p / W, px = p - py * W;
-  gx[i] += 0.25f * gy[(size_t(py / 2) * (W / 2) + px / 2) * C + c];
-}
 // nearest upsample into a channel slice: y[(p)][yo + c] = x[p / 2][c]
 __global__ void up_kernel(const uint16_t* x, int H, int W, int C, uint16_t* y, int ys, int yo) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= H * W * C) return;
   const int c = i % C, p = i / C, py = p / W, px = p - py * W;
   y[size_t(p) * ys + yo + c] = x[(size_t(py / 2) * (W / 2) + px / 2) * C + c];
-}
-// gx[q][c] = sum of gy over the 2x2 block of q (gy: slice yo of stride ys)
-__global__ void up_grad_kernel(const float* gy, int H, int W, int ys, int yo, int C, float* gx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int h = H / 2, w = W / 2;
-  if (i >= h * w * C) return;
-  const int c = i % C, q = i / C, qy = q / w, qx = q - qy * w;
-  const size_t b = (size_t(2 * qy) * W + 2 * qx) * ys + yo + c;
-  gx[i] = gy[b] + gy[b + ys] + gy[b + size_t(W) * ys] + gy[b + size_t(W) * ys + ys];
 }
 // copy a channel slice (bf16): y[p][yo + c] = x[p][xo + c]
 __global__ void copy_slice_kernel(const uint16_t* x, int xs, int xo, int n, int C, uint16_t* y,
@@ -690,14 +848,6 @@ __global__ void copy_slice_kernel(const uint16_t* x, int xs, int xo, int n, int 
   const int c = i % C, p = i / C;
   y[size_t(p) * ys + yo + c] = x[size_t(p) * xs + xo + c];
 }
-// gx[p][c] += gy[p][yo + c] (fp32 slices)
-__global__ void add_slice_kernel(const float* gy, int ys, int yo, int n, int C, float* gx) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * C) return;
-  const int c = i % C, p = i / C;
-  gx[i] += gy[size_t(p) * ys + yo + c];
-}
-
 // network input: in (fp32 [n][inputs]) -> bf16 [n][in_pad] (channels from
 // inputs up zero)
 __global__ void pack_input_kernel(const float* in, int n, int inputs, int in_pad, uint16_t* x) {
@@ -725,41 +875,9 @@ __global__ void kpn_apply_kernel(const float* __restrict__ in, int inputs,
   const int py = p / W, px = p - py * W;
   kpn_filter(in, inputs, logits + size_t(p) * kLogitStride, py, px, H, W, pred + size_t(p) * 3);
 }
-// Squared error of pred against target: err += sum (pred - target)^2, and
-// the gradient of inv_count * that sum with respect to the logits,
-// dz_j = w_j * (c_j - pred) . gpred with gpred = 2 inv_count (pred - target),
-// into gz [n][kLogitStride] (channels < kTaps).
-__global__ void kpn_loss_grad_kernel(const float* __restrict__ in, int inputs,
-                                     const float* __restrict__ logits,
-                                     const float* __restrict__ pred, const float* __restrict__ target,
-                                     int H, int W, float inv_count, float* __restrict__ gz,
-                                     float* err) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  float e = 0.f;
-  if (p < H * W) {
-    const int py = p / W, px = p - py * W;
-    float w[kTaps];
-    const float inv = 1.f / kpn_weights(logits, p, w);
-    const float pr = pred[size_t(p) * 3], pg = pred[size_t(p) * 3 + 1], pb = pred[size_t(p) * 3 + 2];
-    const float dr = pr - target[size_t(p) * 3], dg = pg - target[size_t(p) * 3 + 1],
-                db = pb - target[size_t(p) * 3 + 2];
-    e = dr * dr + dg * dg + db * db;
-    const float s = 2.f * inv_count;
-    const float gr = s * dr, gg = s * dg, gb = s * db;
-    const float base = pr * gr + pg * gg + pb * gb;
-#pragma unroll
-    for (int j = 0; j < kTaps; ++j) {
-      const float* c = in + size_t(kpn_neighbour(py, px, j, H, W)) * inputs;
-      gz[size_t(p) * kLogitStride + j] = w[j] * inv * (c[0] * gr + c[1] * gg + c[2] * gb - base);
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) e += __shfl_down(e, o, 64);
-  if ((threadIdx.x & 63) == 0) atomicAdd(err, e);
-}
-
-// Adam step on fp32 masters (Kingma & Ba 2015), then the bf16 forward copy.
+// Adam step on fp32 masters (Kingma & Ba 2015), every parameter of the network.
 __global__ void adam_kernel(float* w, const float* g, float* m, float* v, int n, float lr,
-                            float b1, float b2, float c1, float c2, float eps, uint16_t* w16) {
+                            float b1, float b2, float c1, float c2, float eps) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const float gi = g[i];
@@ -769,24 +887,23 @@ __global__ void adam_kernel(float* w, const float* g, float* m, float* v, int n,
   v[i] = vi;
   const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
   w[i] = wi;
-  if (w16) w16[i] = f2bf(wi);
 }
 
 // forward weights [9][cout_pad][cin_pad] (bf16) and dgrad weights
-// [9][cin_pad32][cout_pad8] = w[8 - tap][co][ci] from the fp32 master
-// [9][cout][cin]; padding zero.
-__global__ void weight_layouts_kernel(const float* w, int cin, int cout, int cin_pad, int cout_pad,
-                                      uint16_t* wf, int cin_pad32, int cout_pad8, uint16_t* wd) {
+// [9][cin_pad32][cout_pad] = w[8 - tap][co][ci] from the fp32 master
+// [9][cout][cin]; padding zero. Layer blockIdx.y.
+__global__ void weight_layouts_kernel(LayoutArgs a) {
+  const LayoutArgs::Layer& y = a.layer[blockIdx.y];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int nf = 9 * cout_pad * cin_pad, nd = 9 * cin_pad32 * cout_pad8;
+  const int nf = 9 * y.cout_pad * y.cin_pad, nd = 9 * y.cin_pad32 * y.cout_pad;
   if (i < nf) {
-    const int ci = i % cin_pad, r = i / cin_pad, co = r % cout_pad, tap = r / cout_pad;
-    wf[i] = (ci < cin && co < cout) ? f2bf(w[(size_t(tap) * cout + co) * cin + ci]) : uint16_t(0);
+    const int ci = i % y.cin_pad, r = i / y.cin_pad, co = r % y.cout_pad, tap = r / y.cout_pad;
+    y.wf[i] = (ci < y.cin && co < y.cout) ? f2bf(y.w[(size_t(tap) * y.cout + co) * y.cin + ci]) : uint16_t(0);
   }
   if (i < nd) {
-    const int co = i % cout_pad8, r = i / cout_pad8, ci = r % cin_pad32, tap = r / cin_pad32;
-    wd[i] = (ci < cin && co < cout) ? f2bf(w[(size_t(8 - tap) * cout + co) * cin + ci])
-                                    : uint16_t(0);
+    const int co = i % y.cout_pad, r = i / y.cout_pad, ci = r % y.cin_pad32, tap = r / y.cin_pad32;
+    y.wd[i] = (ci < y.cin && co < y.cout) ? f2bf(y.w[(size_t(8 - tap) * y.cout + co) * y.cin + ci])
+                                          : uint16_t(0);
   }
 }
 
@@ -818,15 +935,28 @@ hipError_t conv(const ConvArgs& a, int src, int epi, hipStream_t s) {
     return hipErrorInvalidValue;
   if (src == kSrcF32 && (!a.kin || a.inputs > a.cin)) return hipErrorInvalidValue;
   if (epi == kEpiPool && (a.H % 2 || a.W % 2 || !a.pool16 || !a.y16)) return hipErrorInvalidValue;
-  if (epi == kEpiKpn && (a.cout_pad != kLogitStride || !a.kin || !a.pred)) return hipErrorInvalidValue;
+  const bool kpn = epi == kEpiKpn || epi == kEpiKpnLoss;
+  if (kpn && (a.cout_pad != kLogitStride || !a.kin)) return hipErrorInvalidValue;
+  if (epi == kEpiKpn && !a.pred) return hipErrorInvalidValue;
+  if (epi == kEpiKpnLoss && (!a.target || !a.inv_count || !a.y16 || !a.err)) return hipErrorInvalidValue;
+  if (epi >= kEpiMask && epi <= kEpiPoolGrad && (a.cout % 4 || !a.act || !a.y16 || a.bias))
+    return hipErrorInvalidValue;
+  if (epi == kEpiMask && a.cout > a.ys) return hipErrorInvalidValue;
+  if (epi == kEpiUpGrad && (a.cu % 32 || a.cu >= a.cout || a.cout - a.cu > a.ys || a.H % 2 || a.W % 2 ||
+                            !a.y32))
+    return hipErrorInvalidValue;
+  if (epi == kEpiPoolGrad && (a.cout > a.ys || !a.skip)) return hipErrorInvalidValue;
+  // 32-bit element offsets, of the pooled gradient's full resolution too
+  if (a.nimg < 1 || uint64_t(a.nimg) * a.H * a.W * (epi == kEpiPoolGrad ? 4 : 1) > kMaxPixels)
+    return hipErrorInvalidValue;
   // workgroup shape: 2 x 2 waves of 32 pixels x 2 rows (64 pixels x 4 rows),
   // each with 64 output channels, 96 (the 96-channel level) or 32
   const int shape = a.cout_pad % 64 == 0 ? 2 : a.cout_pad % 96 == 0 ? 3 : 1;
   const int TP = 64, R = 4, TN = 32 * shape;
-  if (epi == kEpiKpn && shape != 2) return hipErrorInvalidValue;
+  if (kpn && shape != 2) return hipErrorInvalidValue;
   // a resident grid (two workgroups per CU, one for the 96-channel shape)
   // whose workgroups loop over the tiles
-  const int tiles = ((a.W + TP - 1) / TP) * ((a.H + R - 1) / R), ny = a.cout_pad / TN;
+  const int tiles = a.nimg * ((a.W + TP - 1) / TP) * ((a.H + R - 1) / R), ny = a.cout_pad / TN;
   const int resident = std::max(1, cu_count() * (shape == 3 ? 1 : 2) / ny);
   const dim3 grid(unsigned(std::min(tiles, resident)), unsigned(ny));
   const int key = shape * 100 + src * 10 + epi;
@@ -840,74 +970,39 @@ hipError_t conv(const ConvArgs& a, int src, int epi, hipStream_t s) {
     case 202: hipLaunchKernelGGL((conv_kernel<2, 2, 2, kSrcPlain, kEpiKpn>), grid, dim3(256), 0, s, a); break;
     case 210: hipLaunchKernelGGL((conv_kernel<2, 2, 2, kSrcUpCat, kEpiPlain>), grid, dim3(256), 0, s, a); break;
     case 300: hipLaunchKernelGGL((conv_kernel<2, 2, 3, kSrcPlain, kEpiPlain>), grid, dim3(256), 0, s, a); break;
+    case 103: hipLaunchKernelGGL((conv_kernel<2, 2, 1, kSrcPlain, kEpiMask>), grid, dim3(256), 0, s, a); break;
+    case 104: hipLaunchKernelGGL((conv_kernel<2, 2, 1, kSrcPlain, kEpiUpGrad>), grid, dim3(256), 0, s, a); break;
+    case 105: hipLaunchKernelGGL((conv_kernel<2, 2, 1, kSrcPlain, kEpiPoolGrad>), grid, dim3(256), 0, s, a); break;
+    case 203: hipLaunchKernelGGL((conv_kernel<2, 2, 2, kSrcPlain, kEpiMask>), grid, dim3(256), 0, s, a); break;
+    case 205: hipLaunchKernelGGL((conv_kernel<2, 2, 2, kSrcPlain, kEpiPoolGrad>), grid, dim3(256), 0, s, a); break;
+    case 206: hipLaunchKernelGGL((conv_kernel<2, 2, 2, kSrcPlain, kEpiKpnLoss>), grid, dim3(256), 0, s, a); break;
+    case 303: hipLaunchKernelGGL((conv_kernel<2, 2, 3, kSrcPlain, kEpiMask>), grid, dim3(256), 0, s, a); break;
+    case 304: hipLaunchKernelGGL((conv_kernel<2, 2, 3, kSrcPlain, kEpiUpGrad>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-hipError_t conv3x3(const uint16_t* x, int H, int W, int xs, int xo, int cin, const uint16_t* w,
-                   const float* bias, int cout, int cout_pad, uint16_t* y16, float* y32, int ys,
-                   int yo, bool relu, bool accum, hipStream_t s) {
-  ConvArgs a{};
-  a.x = x;
-  a.xs = xs;
-  a.xo = xo;
-  a.H = H;
-  a.W = W;
-  a.cin = cin;
-  a.w = w;
-  a.bias = bias;
-  a.cout = cout;
-  a.cout_pad = cout_pad;
-  a.y16 = y16;
-  a.y32 = y32;
-  a.ys = ys;
-  a.yo = yo;
-  a.relu = relu ? 1 : 0;
-  a.accum = accum ? 1 : 0;
-  return conv(a, kSrcPlain, kEpiPlain, s);
-}
+// workgroups of one weight-gradient launch over all its channel tiles: two per
+// CU, one resident round (each adds 36 KiB of partial sums to the reduction)
+constexpr int kWgradGroups = 512;
 
-// waves of one weight-gradient launch (8192 measured no faster: the band
-// reduction grows with them)
-constexpr int kWgradWaves = 2048;
-
-hipError_t wgrad(const uint16_t* g, int gs, const uint16_t* x, int xs, int xo, int H, int W,
-                 int cin, int cout, float* dw, float* part, size_t part_cap, hipStream_t s) {
+hipError_t wgrad(WgradArgs a, float* dw, size_t part_cap, hipStream_t s) {
   // 8-byte channel groups: strides and offsets in whole groups, and the
   // groups that hold the last channels inside the row
-  if (gs % 4 || xs % 4 || xo % 4 || (cout + 3) / 4 * 4 > gs || xo + (cin + 3) / 4 * 4 > xs)
+  if (a.gs % 4 || a.xs % 4 || a.xo % 4 || (a.cout + 3) / 4 * 4 > a.gs || a.cu % 32 || a.nimg < 1)
     return hipErrorInvalidValue;
-  const int tiles = ((cin + 31) / 32) * ((cout + 31) / 32);
-  const size_t per_band = size_t(9) * cout * cin;
-  if (per_band > part_cap) return hipErrorInvalidValue;
-  // about kWgradWaves waves (3 tap rows per band), within the partial-sum buffer
-  int bands = std::max(1, std::min(H, std::min((kWgradWaves / 3 + tiles - 1) / tiles, int(part_cap / per_band))));
-  const int rows = (H + bands - 1) / bands;
-  bands = (H + rows - 1) / rows;
-  const dim3 grid(unsigned((cin + 31) / 32), unsigned((cout + 31) / 32), unsigned(bands * 3));
-  hipLaunchKernelGGL(wgrad_band_kernel, grid, dim3(64), 0, s, g, gs, x, xs, xo, H, W, cin, cout,
-                     rows, part);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nb(per_band, 16)), dim3(256), 0, s, part, bands,
-                     int(per_band), dw);
-  return hipGetLastError();
-}
-
-hipError_t relu_grad(const float* gy, int gs, const uint16_t* y, int ys, int yo, int npix, int cout,
-                     int cout_pad, bool relu, uint16_t* gm, float* db, float* part,
-                     size_t part_cap, hipStream_t s) {
-  const int chunk = 4096;
-  const int chunks = (npix + chunk - 1) / chunk;
-  if (size_t(chunks) * cout > part_cap) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(relu_grad_kernel, dim3(nb(size_t(npix) * cout_pad)), dim3(256), 0, s, gy, gs,
-                     y, ys, yo, npix, cout, cout_pad, relu ? 1 : 0, gm);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(bias_grad_kernel, dim3(unsigned(cout), unsigned(chunks)), dim3(256), 0, s, gm,
-                     cout_pad, npix, chunk, part);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(bias_reduce_kernel, dim3(nb(size_t(cout))), dim3(256), 0, s, part, chunks,
-                     cout, db);
+  if (a.cu ? (a.cin % 4 || a.xo + a.cin - a.cu > a.xs || !a.xl || a.H % 2 || a.W % 2)
+           : a.xo + (a.cin + 3) / 4 * 4 > a.xs)
+    return hipErrorInvalidValue;
+  a.xc = (a.cin + 3) / 4 * 4;
+  const int tx = (a.cin + 31) / 32, ty = (a.cout + 31) / 32;
+  const size_t per = size_t(9) * a.cout * a.cin + a.cout;
+  if (per > part_cap) return hipErrorInvalidValue;
+  const int units = a.nimg * ((a.H + kUnitRows - 1) / kUnitRows) * ((a.W + kSeg - 1) / kSeg);
+  const int groups = std::max(1, std::min({(units + 3) / 4, kWgradGroups / (tx * ty), int(part_cap / per)}));
+  hipLaunchKernelGGL(wgrad_kernel, dim3(unsigned(tx), unsigned(ty), unsigned(groups)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nb(per, 16)), dim3(256), 0, s, a.part, groups, int(per), dw);
   return hipGetLastError();
 }
 
@@ -916,30 +1011,15 @@ hipError_t pool(const uint16_t* x, int H, int W, int C, uint16_t* y, hipStream_t
                      C, y);
   return hipGetLastError();
 }
-hipError_t pool_grad(const float* gy, int H, int W, int C, float* gx, hipStream_t s) {
-  hipLaunchKernelGGL(pool_grad_kernel, dim3(nb(size_t(H) * W * C)), dim3(256), 0, s, gy, H, W, C,
-                     gx);
-  return hipGetLastError();
-}
 hipError_t up(const uint16_t* x, int H, int W, int C, uint16_t* y, int ys, int yo, hipStream_t s) {
   hipLaunchKernelGGL(up_kernel, dim3(nb(size_t(H) * W * C)), dim3(256), 0, s, x, H, W, C, y, ys,
                      yo);
-  return hipGetLastError();
-}
-hipError_t up_grad(const float* gy, int H, int W, int ys, int yo, int C, float* gx, hipStream_t s) {
-  hipLaunchKernelGGL(up_grad_kernel, dim3(nb(size_t(H / 2) * (W / 2) * C)), dim3(256), 0, s, gy, H,
-                     W, ys, yo, C, gx);
   return hipGetLastError();
 }
 hipError_t copy_slice(const uint16_t* x, int xs, int xo, int n, int C, uint16_t* y, int ys, int yo,
                       hipStream_t s) {
   hipLaunchKernelGGL(copy_slice_kernel, dim3(nb(size_t(n) * C)), dim3(256), 0, s, x, xs, xo, n, C,
                      y, ys, yo);
-  return hipGetLastError();
-}
-hipError_t add_slice(const float* gy, int ys, int yo, int n, int C, float* gx, hipStream_t s) {
-  hipLaunchKernelGGL(add_slice_kernel, dim3(nb(size_t(n) * C)), dim3(256), 0, s, gy, ys, yo, n, C,
-                     gx);
   return hipGetLastError();
 }
 hipError_t pack_input(const float* in, int n, int inputs, int in_pad, uint16_t* x, hipStream_t s) {
@@ -954,24 +1034,17 @@ hipError_t kpn_apply(const float* in, int inputs, const float* logits, int H, in
                      logits, H, W, pred);
   return hipGetLastError();
 }
-hipError_t kpn_loss_grad(const float* in, int inputs, const float* logits, const float* pred,
-                         const float* target, int H, int W, float inv_count, float* gz, float* err,
-                         hipStream_t s) {
-  hipLaunchKernelGGL(kpn_loss_grad_kernel, dim3(nb(size_t(H) * W)), dim3(256), 0, s, in, inputs,
-                     logits, pred, target, H, W, inv_count, gz, err);
-  return hipGetLastError();
-}
 hipError_t adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2,
-                float c1, float c2, float eps, uint16_t* w16, hipStream_t s) {
+                float c1, float c2, float eps, hipStream_t s) {
   hipLaunchKernelGGL(adam_kernel, dim3(nb(size_t(n))), dim3(256), 0, s, w, g, m, v, n, lr, b1, b2,
-                     c1, c2, eps, w16);
+                     c1, c2, eps);
   return hipGetLastError();
 }
-hipError_t weight_layouts(const float* w, int cin, int cout, int cin_pad, int cout_pad,
-                          uint16_t* wf, int cin_pad32, int cout_pad8, uint16_t* wd, hipStream_t s) {
-  const size_t n = std::max(size_t(9) * cout_pad * cin_pad, size_t(9) * cin_pad32 * cout_pad8);
-  hipLaunchKernelGGL(weight_layouts_kernel, dim3(nb(n)), dim3(256), 0, s, w, cin, cout, cin_pad,
-                     cout_pad, wf, cin_pad32, cout_pad8, wd);
+hipError_t weight_layouts(const LayoutArgs& a, hipStream_t s) {
+  int n = 0;
+  for (const auto& y : a.layer)
+    n = std::max({n, 9 * y.cout_pad * y.cin_pad, 9 * y.cin_pad32 * y.cout_pad});
+  hipLaunchKernelGGL(weight_layouts_kernel, dim3(nb(size_t(n)), kLayers), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
