@@ -162,6 +162,15 @@ __global__ void rgba8_kernel(const float4* acc, uint32_t* out, int n) {
   out[i] = to8(c.x) | (to8(c.y) << 8) | (to8(c.z) << 16) | (to8(c.w) << 24);
 }
 
+// the auxiliary buffers without their padding, as mdwt_read_aov returns them
+__global__ __launch_bounds__(256) void pack_aov_kernel(const float* __restrict__ aov, int row, int nv,
+                                                       size_t n, float* __restrict__ out) {
+  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= n * size_t(nv)) return;
+  const size_t p = i / uint32_t(nv);
+  out[i] = aov[p * size_t(row) + (i - p * size_t(nv))];
+}
+
 __global__ __launch_bounds__(256) void copy_kernel(const float4* __restrict__ src,
                                                    float4* __restrict__ dst, size_t n) {
   size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -347,6 +356,12 @@ uint32_t* fb_scratch(int device) {
 hipError_t launch_rgba8(const void* accum, uint32_t* out, int n, hipStream_t s) {
   hipLaunchKernelGGL(rgba8_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s,
                      reinterpret_cast<const float4*>(accum), out, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_pack_aov(const float* aov, int row, int nv, size_t n, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(pack_aov_kernel, dim3(unsigned((n * size_t(nv) + 255) / 256)), dim3(256), 0, s, aov,
+                     row, nv, n, out);
   return hipGetLastError();
 }
 

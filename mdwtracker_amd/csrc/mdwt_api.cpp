@@ -124,7 +124,9 @@ struct mdwt_renderer {
   size_t fb_pixels = 0;
   unsigned long long* d_counters = nullptr;
   uint32_t* d_order = nullptr;
-  std::vector<uint32_t> order;  // host copy of d_order
+  uint32_t* d_order_tmp = nullptr;  // the cost sort's
+  void* d_read = nullptr;           // read-back conversions
+  size_t read_bytes = 0;
   int n_blocks = 0;
   int* d_win = nullptr;
   uint32_t* d_wave_cost = nullptr;  // per-wave ticks of the last recorded frame
@@ -369,7 +371,12 @@ void free_frame(mdwt_renderer* h) {
   if (h->d_accum) (void)hipFree(h->d_accum);
   if (h->d_m2) (void)hipFree(h->d_m2);
   if (h->d_order) (void)hipFree(h->d_order);
+  if (h->d_order_tmp) (void)hipFree(h->d_order_tmp);
   if (h->d_wave_cost) (void)hipFree(h->d_wave_cost);
+  if (h->d_read) (void)hipFree(h->d_read);
+  h->d_order_tmp = nullptr;
+  h->d_read = nullptr;
+  h->read_bytes = 0;
   h->d_accum = h->d_m2 = nullptr;
   h->d_order = nullptr;
   h->d_wave_cost = nullptr;
@@ -377,32 +384,17 @@ void free_frame(mdwt_renderer* h) {
   h->fb_pixels = 0;
 }
 
-// Cost-sorted block order (longest processing time first): blocks sorted by
-// the summed wall-clock ticks of their waves in the last recorded frame,
-// heaviest first. Workgroup i runs on XCD i % 8, so the sorted list is dealt
-// round-robin over the XCDs and the slowest blocks start first instead of
-// trailing at the end of the frame.
-int resort_blocks(mdwt_renderer* h) {
-  const size_t nb = size_t(h->n_blocks);
-  const size_t wpb = size_t(h->bw * h->bh / 64);  // waves per block
-  std::vector<uint32_t> ticks(wpb * nb);
-  HIPCHK(h, hipMemcpyAsync(ticks.data(), h->d_wave_cost, ticks.size() * sizeof(uint32_t),
-                           hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  std::vector<std::pair<uint64_t, uint32_t>> cost(nb);
-  for (size_t s = 0; s < nb; ++s) {
-    uint64_t c = 0;
-    for (size_t w = 0; w < wpb; ++w) c += ticks[wpb * s + w];
-    cost[s] = {c, h->order[s]};
+// Device scratch of at least `bytes` for a read-back's conversion, kept until
+// the frame size changes.
+int read_scratch(mdwt_renderer* h, size_t bytes, void** out) {
+  if (bytes > h->read_bytes) {
+    if (h->d_read) (void)hipFree(h->d_read);
+    h->d_read = nullptr;
+    h->read_bytes = 0;
+    HIPCHK(h, hipMalloc(&h->d_read, bytes));
+    h->read_bytes = bytes;
   }
-  std::stable_sort(cost.begin(), cost.end(),
-                   [](const std::pair<uint64_t, uint32_t>& a, const std::pair<uint64_t, uint32_t>& b) {
-                     return a.first > b.first;
-                   });
-  for (size_t s = 0; s < nb; ++s) h->order[s] = cost[s].second;
-  HIPCHK(h, hipMemcpyAsync(h->d_order, h->order.data(), nb * sizeof(uint32_t), hipMemcpyHostToDevice,
-                           h->stream));
-  h->cost_ready = false;
+  *out = h->d_read;
   return MDWT_OK;
 }
 
@@ -446,6 +438,9 @@ int alloc_frame(mdwt_renderer* h) {
     HIPCHK(h, hipMemsetAsync(h->d_m2, 0, n * sizeof(Float4), h->stream));
   }
   h->fb_pixels = n;
+  // the RGBA8 frame buffer
+  void* fb = nullptr;
+  if (const int rc = read_scratch(h, n * sizeof(uint32_t), &fb)) return rc;
   if (h->aov_on) {
     const size_t na = size_t(mdwt::aov_groups(h->C)) * n;
     HIPCHK(h, hipMalloc(&h->d_aov, na * sizeof(Float4)));
@@ -458,9 +453,9 @@ int alloc_frame(mdwt_renderer* h) {
   HIPCHK(h, hipMalloc(&h->d_order, order.size() * sizeof(uint32_t)));
   HIPCHK(h, hipMemcpyAsync(h->d_order, order.data(), order.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice, h->stream));
+  HIPCHK(h, hipMalloc(&h->d_order_tmp, order.size() * sizeof(uint32_t)));
   HIPCHK(h, hipMalloc(&h->d_wave_cost, 4 * order.size() * sizeof(uint32_t)));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  h->order = std::move(order);
   h->cost_ready = false;
   h->need_resort = true;
   return MDWT_OK;
@@ -1108,8 +1103,9 @@ int mdwt_render(mdwt_renderer* h, int n_frames, float* ms_out) {
   if (n_frames < 0) return fail(h, MDWT_ERR_ARG, "negative frame count");
   HIPCHK(h, hipSetDevice(h->device));
   if (h->order_mode == 2 && h->need_resort && h->cost_ready) {
-    rc = resort_blocks(h);
-    if (rc != MDWT_OK) return rc;
+    HIPCHK(h, mdwt::launch_cost_order(h->d_order, h->d_wave_cost, h->d_order_tmp, h->n_blocks,
+                                      h->bw * h->bh / 64, h->stream));
+    h->cost_ready = false;
     h->need_resort = false;
   }
   HIPCHK(h, hipEventRecord(h->ev0, h->stream));
@@ -1153,14 +1149,12 @@ int mdwt_read_fb(mdwt_renderer* h, uint32_t* rgba8) {
   if (!h->inited) return fail(h, MDWT_ERR_STATE, "renderer not initialized");
   if (!rgba8) return fail(h, MDWT_ERR_ARG, "null output");
   HIPCHK(h, hipSetDevice(h->device));
-  uint32_t* d = nullptr;
-  HIPCHK(h, hipMalloc(&d, h->fb_pixels * sizeof(uint32_t)));
-  hipError_t e = mdwt::launch_rgba8(h->d_accum, d, int(h->fb_pixels), h->stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(rgba8, d, h->fb_pixels * sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-  (void)hipFree(d);
-  if (e != hipSuccess) return fail(h, MDWT_ERR_HIP, std::string("read_fb: ") + hipGetErrorString(e));
+  void* d = nullptr;
+  const int rc = read_scratch(h, h->fb_pixels * sizeof(uint32_t), &d);
+  if (rc != MDWT_OK) return rc;
+  HIPCHK(h, mdwt::launch_rgba8(h->d_accum, static_cast<uint32_t*>(d), int(h->fb_pixels), h->stream));
+  HIPCHK(h, hipMemcpyAsync(rgba8, d, h->fb_pixels * sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream));
+  HIPCHK(h, hipStreamSynchronize(h->stream));
   return MDWT_OK;
 }
 
@@ -2133,12 +2127,19 @@ int mdwt_read_aov(mdwt_renderer* h, float* out) {
   if (!h || !out) return MDWT_ERR_ARG;
   if (!h->aov_on || !h->d_aov) return fail(h, MDWT_ERR_STATE, "auxiliary buffers are off");
   HIPCHK(h, hipSetDevice(h->device));
+  const int row = 4 * mdwt::aov_groups(h->C), nv = 2 + h->C;
+  const size_t bytes = h->fb_pixels * size_t(nv) * sizeof(float);
+  const void* src = h->d_aov;
+  if (row != nv) {  // the padding is dropped on the device
+    void* d = nullptr;
+    const int rc = read_scratch(h, bytes, &d);
+    if (rc != MDWT_OK) return rc;
+    HIPCHK(h, mdwt::launch_pack_aov(reinterpret_cast<const float*>(h->d_aov), row, nv, h->fb_pixels,
+                                    static_cast<float*>(d), h->stream));
+    src = d;
+  }
+  HIPCHK(h, hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  const int ng = mdwt::aov_groups(h->C), nv = 2 + h->C;
-  std::vector<float> tmp(size_t(4 * ng) * h->fb_pixels);
-  HIPCHK(h, hipMemcpy(tmp.data(), h->d_aov, tmp.size() * sizeof(float), hipMemcpyDeviceToHost));
-  for (size_t p = 0; p < h->fb_pixels; ++p)
-    std::memcpy(out + size_t(nv) * p, tmp.data() + size_t(4 * ng) * p, size_t(nv) * sizeof(float));
   return MDWT_OK;
 }
 

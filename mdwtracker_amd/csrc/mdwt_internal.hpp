@@ -24,6 +24,12 @@ size_t wave_lds_bytes(const RenderParams& p);
 
 hipError_t launch_ranges(const RangeParams& p, int dtype, hipStream_t s);
 hipError_t launch_majorants(const MajorantParams& p, hipStream_t s);
+// order (nb blocks) by decreasing cost, block b's being the sum of ticks[wpb * b ..]
+// (the block at position b); tmp: nb entries
+hipError_t launch_cost_order(uint32_t* order, const uint32_t* ticks, uint32_t* tmp, int nb, int wpb,
+                             hipStream_t s);
+// out[p][0 .. nv) = aov[p][0 .. nv) of rows of `row` floats, n pixels
+hipError_t launch_pack_aov(const float* aov, int row, int nv, size_t n, float* out, hipStream_t s);
 // v.bricks (brick_stride bytes per channel) = v.vol in 4 x 4 x 4 bricks
 hipError_t launch_bricks(const VolumeParams& v, int dtype, hipStream_t s);
 // v.joint (joint_stride bytes per group of four channels) from v.vol

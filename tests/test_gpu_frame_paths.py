@@ -124,3 +124,26 @@ def test_channels_side_by_side_match_the_oracle(capi, mode, channels, dtype):
     o.render(2, threads=4)
     np.testing.assert_array_equal(g.read_accum().view(np.uint32), o.read_accum().view(np.uint32))
     g.close()
+
+
+@pytest.mark.parametrize("conservative", [False, True])
+@pytest.mark.parametrize("mode", [1, 3])
+@pytest.mark.parametrize("texels", [1, 2, 16, 17, 300])
+def test_majorants_match_the_oracle(capi, texels, mode, conservative):
+    """Tables shorter and longer than the lanes that share a cell, reversed and
+    offset ranges, against the CPU oracle."""
+    from oracle import pyoracle
+    vols, _ = volume(3, np.uint16, dims=(19, 22, 17))
+    rng = np.random.default_rng(texels)
+    tfs = [rng.uniform(0, 1, (texels, 4)).astype(np.float32) for _ in vols]
+    out = []
+    for r in (capi.MdwtRenderer(0), pyoracle.OracleRenderer()):
+        for v in vols:
+            r.push_channel(v)
+        r.init(mode, (9, 7, 8), False)
+        r.set_conservative_majorants(conservative)
+        for c, (t, xr) in enumerate(zip(tfs, ((0.0, 1.0), (0.8, 0.2), (-0.3, 0.6)))):
+            r.set_tf(c, t, 0.7, xr)
+        out.append(r.read_majorants().view(np.uint32))
+        r.close()
+    np.testing.assert_array_equal(out[0], out[1])
