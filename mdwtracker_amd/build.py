@@ -37,7 +37,8 @@ COMMON = [
 
 SOURCES = ["kernels_build.hip", "kernels_render.hip", "kernels_batch.hip", "kernels_wave.hip",
            "kernels_wave_lit.hip",
-           "kernels_denoise.hip", "mdwt_api.cpp", "denoise_api.cpp"]
+           "kernels_denoise.hip", "mdwt_api.cpp", "denoise_api.cpp",
+           "host_copy.hip"]
 
 
 def _run(cmd: list[str], verbose: bool) -> None:

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "denoise_internal.hpp"
+#include "host_copy.hpp"
 
 namespace {
 
@@ -487,10 +488,10 @@ int loss_gradient(mdwt_denoiser* d, const float* in, const float* tgt, const flo
     const int B = std::min(count - i, d->train.images);
     for (int k = 0; k < B; ++k) w[size_t(k)] = weights ? inv * weights[i + k] : inv;
     DNCHK(d, hipMemcpyAsync(d->train.inv, w.data(), size_t(B) * sizeof(float), hipMemcpyHostToDevice, d->stream));
-    DNCHK(d, hipMemcpyAsync(d->train.in32, in + size_t(i) * n * d->inputs, size_t(B) * n * d->inputs * sizeof(float),
-                            hipMemcpyHostToDevice, d->stream));
-    DNCHK(d, hipMemcpyAsync(d->train.tgt, tgt + size_t(i) * n * 3, size_t(B) * n * 3 * sizeof(float),
-                            hipMemcpyHostToDevice, d->stream));
+    DNCHK(d, mdwt::copy_to_device(d->train.in32, in + size_t(i) * n * d->inputs,
+                                  size_t(B) * n * d->inputs * sizeof(float), d->device, d->stream));
+    DNCHK(d, mdwt::copy_to_device(d->train.tgt, tgt + size_t(i) * n * 3, size_t(B) * n * 3 * sizeof(float),
+                                  d->device, d->stream));
     if ((rc = train_batch(d, B))) return rc;
     DNCHK(d, hipStreamSynchronize(d->stream));  // the host's arrays are its own again
   }
@@ -514,6 +515,7 @@ int mdwt_dn_create(mdwt_denoiser** out, int hip_device, int width, int height, i
   if (size_t(width) * size_t(height) > kMaxPixels) return MDWT_ERR_LIMIT;
   auto* d = new (std::nothrow) mdwt_denoiser();
   if (!d) return MDWT_ERR_OOM;
+  mdwt::host_copy_acquire();
   d->device = hip_device;
   d->W = width;
   d->H = height;
@@ -545,6 +547,7 @@ int mdwt_dn_destroy(mdwt_denoiser* d) {
   if (d->ev0) (void)hipEventDestroy(d->ev0);
   if (d->ev1) (void)hipEventDestroy(d->ev1);
   if (d->stream) (void)hipStreamDestroy(d->stream);
+  mdwt::host_copy_release();
   delete d;
   return MDWT_OK;
 }
@@ -561,7 +564,7 @@ int mdwt_dn_get_params(mdwt_denoiser* d, float* out) {
   if (!d || !out) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   DNCHK(d, hipStreamSynchronize(d->stream));
-  DNCHK(d, hipMemcpy(out, d->params, d->n_params * sizeof(float), hipMemcpyDeviceToHost));
+  DNCHK(d, mdwt::copy_to_host(out, d->params, d->n_params * sizeof(float), d->device, d->stream));
   return MDWT_OK;
 }
 
@@ -580,13 +583,12 @@ int mdwt_dn_infer(mdwt_denoiser* d, const float* input, float* output, float* ms
   if (!d || !input || !output) return MDWT_ERR_ARG;
   DNCHK(d, hipSetDevice(d->device));
   const size_t n = size_t(d->H) * d->W;
-  DNCHK(d, hipMemcpyAsync(d->in32, input, n * d->inputs * sizeof(float),
-                          hipMemcpyHostToDevice, d->stream));
+  DNCHK(d, mdwt::copy_to_device(d->in32, input, n * d->inputs * sizeof(float), d->device, d->stream));
   DNCHK(d, hipEventRecord(d->ev0, d->stream));
   int rc = d->fused ? forward_fused(d) : forward(d);
   if (rc) return rc;
   DNCHK(d, hipEventRecord(d->ev1, d->stream));
-  DNCHK(d, hipMemcpyAsync(output, d->pred, n * 3 * sizeof(float), hipMemcpyDeviceToHost, d->stream));
+  DNCHK(d, mdwt::copy_to_host(output, d->pred, n * 3 * sizeof(float), d->device, d->stream));
   DNCHK(d, hipStreamSynchronize(d->stream));
   float t = 0.f;
   DNCHK(d, hipEventElapsedTime(&t, d->ev0, d->ev1));
@@ -607,7 +609,7 @@ int mdwt_dn_gradient(mdwt_denoiser* d, const float* input, const float* target, 
   const size_t n = size_t(d->H) * d->W;
   int rc = loss_gradient(d, input, target, nullptr, 1, 1.f / float(n * 3));
   if (rc) return rc;
-  DNCHK(d, hipMemcpy(grad, d->grads, d->n_params * sizeof(float), hipMemcpyDeviceToHost));
+  DNCHK(d, mdwt::copy_to_host(grad, d->grads, d->n_params * sizeof(float), d->device, d->stream));
   if (loss) {
     float e = 0.f;
     DNCHK(d, hipMemcpy(&e, d->err_sum, sizeof(float), hipMemcpyDeviceToHost));

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "batch_deal.hpp"
+#include "host_copy.hpp"
 #include "mdwt.h"
 #include "mdwt_internal.hpp"
 #include "mdwt_types.hpp"
@@ -719,6 +720,7 @@ int mdwt_create(mdwt_renderer** out, int hip_device) {
     return MDWT_ERR_OOM;
   }
   h->device = hip_device;
+  mdwt::host_copy_acquire();
   for (int c = 0; c < MDWT_MAX_CHANNELS; ++c) {
     h->os[c] = 1.0f;  // TFData defaults (renderer.h:45-49)
     h->xlo[c] = 0.f;
@@ -742,6 +744,7 @@ int mdwt_destroy(mdwt_renderer* h) {
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
   }
+  mdwt::host_copy_release();
   delete h;
   return MDWT_OK;
 }
@@ -869,8 +872,8 @@ int mdwt_init(mdwt_renderer* h, int mode, const int mc[3], int auto_camera) {
   if (hipMalloc(&h->d_vol, h->chan_stride * h->C) != hipSuccess)
     return fail(h, MDWT_ERR_OOM, "device allocation of the volume failed");
   for (int c = 0; c < h->C; ++c)
-    HIPCHK(h, hipMemcpyAsync(h->d_vol + size_t(c) * h->chan_stride, h->staging[c].data(), chan_bytes,
-                             hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, mdwt::copy_to_device(h->d_vol + size_t(c) * h->chan_stride, h->staging[c].data(), chan_bytes,
+                                   h->device, h->stream));
   int rc0 = build_range_grid(h, wx, wy, wz);
   if (rc0 != MDWT_OK) return rc0;
   if ((rc0 = make_bricks(h)) != MDWT_OK || (rc0 = make_joint(h)) != MDWT_OK) return rc0;
@@ -1138,9 +1141,8 @@ int mdwt_read_accum(mdwt_renderer* h, float* rgba, float* m2) {
   HIPCHK(h, hipSetDevice(h->device));
   const size_t bytes = h->fb_pixels * sizeof(Float4);
   if (m2 && !h->d_m2) return fail(h, MDWT_ERR_STATE, "second moments are off (mdwt_set_moments)");
-  if (rgba) HIPCHK(h, hipMemcpyAsync(rgba, h->d_accum, bytes, hipMemcpyDeviceToHost, h->stream));
-  if (m2) HIPCHK(h, hipMemcpyAsync(m2, h->d_m2, bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  if (rgba) HIPCHK(h, mdwt::copy_to_host(rgba, h->d_accum, bytes, h->device, h->stream));
+  if (m2) HIPCHK(h, mdwt::copy_to_host(m2, h->d_m2, bytes, h->device, h->stream));
   return MDWT_OK;
 }
 
@@ -1153,8 +1155,7 @@ int mdwt_read_fb(mdwt_renderer* h, uint32_t* rgba8) {
   const int rc = read_scratch(h, h->fb_pixels * sizeof(uint32_t), &d);
   if (rc != MDWT_OK) return rc;
   HIPCHK(h, mdwt::launch_rgba8(h->d_accum, static_cast<uint32_t*>(d), int(h->fb_pixels), h->stream));
-  HIPCHK(h, hipMemcpyAsync(rgba8, d, h->fb_pixels * sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, mdwt::copy_to_host(rgba8, d, h->fb_pixels * sizeof(uint32_t), h->device, h->stream));
   return MDWT_OK;
 }
 
@@ -2008,12 +2009,11 @@ int mdwt_batch_read_view(mdwt_renderer* h, int view, float* rgba, float* m2) {
   if (!h) return MDWT_ERR_ARG;
   if (view < 0 || size_t(view) >= h->views.size()) return fail(h, MDWT_ERR_ARG, "no such view");
   HIPCHK(h, hipSetDevice(h->device));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
   const auto& v = h->views[size_t(view)];
   const size_t bytes = size_t(v.width) * v.height * sizeof(Float4);
   if (m2 && !v.m2) return fail(h, MDWT_ERR_STATE, "second moments are off (mdwt_set_moments)");
-  if (rgba) HIPCHK(h, hipMemcpy(rgba, v.accum, bytes, hipMemcpyDeviceToHost));
-  if (m2) HIPCHK(h, hipMemcpy(m2, v.m2, bytes, hipMemcpyDeviceToHost));
+  if (rgba) HIPCHK(h, mdwt::copy_to_host(rgba, v.accum, bytes, h->device, h->stream));
+  if (m2) HIPCHK(h, mdwt::copy_to_host(m2, v.m2, bytes, h->device, h->stream));
   return MDWT_OK;
 }
 
@@ -2138,8 +2138,7 @@ int mdwt_read_aov(mdwt_renderer* h, float* out) {
                                     static_cast<float*>(d), h->stream));
     src = d;
   }
-  HIPCHK(h, hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, mdwt::copy_to_host(out, src, bytes, h->device, h->stream));
   return MDWT_OK;
 }
 
