@@ -34,6 +34,7 @@ struct Ctx {
   uint64_t brick_stride;
   const uint8_t* joint;
   uint64_t joint_stride;
+  bool bricks32;       // every channel's bricks within 4 GiB
   uint32_t nbx, nbxy;  // bricks per row and per slab (both below 2^24)
   int nx, ny, nz;
   float scale, offset;
@@ -48,6 +49,7 @@ struct Ctx {
                                        const ChanTf* ch_lds) {
     bricks = P.vol.bricks;
     brick_stride = P.vol.brick_stride;
+    bricks32 = brick_stride * uint64_t(P.vol.channels) <= 0xffffffffull;
     joint = P.vol.joint;
     joint_stride = P.vol.joint_stride;
     nbx = uint32_t(P.vol.nbx);
@@ -72,6 +74,7 @@ struct Ctx {
   // that a caller can do other work while the voxels are on their way:
   // corners() issues the eight loads (indices are clamped, so they are in
   // bounds for every p, NaN included), trilinear() waits for them.
+  static constexpr uint32_t kBytes = DT == MDWT_DT_U8 ? 1u : (DT == MDWT_DT_F32 ? 4u : 2u);
   struct Corners {
     uint32_t b000, b100, b010, b110, b001, b101, b011, b111;  // stored bits
     float fx, fy, fz;
@@ -99,19 +102,20 @@ struct Ctx {
     k.fx = x - flx;
     k.fy = y - fly;
     k.fz = z - flz;
-    const uint32_t x0 = uint32_t(clamp_index(flx, nx)), x1 = uint32_t(clamp_index_plus1(flx, nx));
-    const uint32_t y0 = uint32_t(clamp_index(fly, ny)), y1 = uint32_t(clamp_index_plus1(fly, ny));
-    const uint32_t z0 = uint32_t(clamp_index(flz, nz)), z1 = uint32_t(clamp_index_plus1(flz, nz));
+    int x0, x1, y0, y1, z0, z1;
+    clamp_pair(flx, nx, x0, x1);
+    clamp_pair(fly, ny, y0, y1);
+    clamp_pair(flz, nz, z0, z1);
     // the voxels are read from the 4 x 4 x 4 brick copies: index = X(x) +
     // Y(y) + Z(z) (a trilinear footprint touches about 1.8 cache lines
     // instead of 4 in the planar layout; 3.5% faster at -m 2 on 4 x 256^3 u8)
-    const uint32_t ax0 = ((x0 >> 2) << 6) | (x0 & 3u), ax1 = ((x1 >> 2) << 6) | (x1 & 3u);
-    // 24-bit products (full-rate v_mul_u32_u24): brick coordinates and the
-    // bricks per row / slab are below 2^24 (checked when the volume is set)
-    const uint32_t ay0 = (__umul24(y0 >> 2, nbx) << 6) | ((y0 & 3u) << 2);
-    const uint32_t ay1 = (__umul24(y1 >> 2, nbx) << 6) | ((y1 & 3u) << 2);
-    const uint32_t az0 = (__umul24(z0 >> 2, nbxy) << 6) | ((z0 & 3u) << 4);
-    const uint32_t az1 = (__umul24(z1 >> 2, nbxy) << 6) | ((z1 & 3u) << 4);
+    const uint32_t ax0 = (uint32_t(x0 >> 2) << 6) | (x0 & 3), ax1 = (uint32_t(x1 >> 2) << 6) | (x1 & 3);
+    // brick coordinates and the bricks per row / slab are below 2^24 (checked
+    // when the volume is set)
+    const uint32_t ay0 = (mul_u24(y0 >> 2, nbx) << 6) | ((y0 & 3) << 2);
+    const uint32_t ay1 = (mul_u24(y1 >> 2, nbx) << 6) | ((y1 & 3) << 2);
+    const uint32_t az0 = (mul_u24(z0 >> 2, nbxy) << 6) | ((z0 & 3) << 4);
+    const uint32_t az1 = (mul_u24(z1 >> 2, nbxy) << 6) | ((z1 & 3) << 4);
     const uint32_t r00 = ay0 + az0, r10 = ay1 + az0, r01 = ay0 + az1, r11 = ay1 + az1;
     k.i[0] = r00 + ax0;
     k.i[1] = r00 + ax1;
@@ -125,20 +129,35 @@ struct Ctx {
   }
   __device__ __forceinline__ Corners corners(V3 p, int c) const {
     const Foot f = foot(p);
-    const uint8_t* base = bricks + size_t(c) * brick_stride;
     Corners k;
     k.inside = f.inside;
     k.fx = f.fx;
     k.fy = f.fy;
     k.fz = f.fz;
-    k.b000 = fetch_bits<DT>(base, f.i[0]);
-    k.b100 = fetch_bits<DT>(base, f.i[1]);
-    k.b010 = fetch_bits<DT>(base, f.i[2]);
-    k.b110 = fetch_bits<DT>(base, f.i[3]);
-    k.b001 = fetch_bits<DT>(base, f.i[4]);
-    k.b101 = fetch_bits<DT>(base, f.i[5]);
-    k.b011 = fetch_bits<DT>(base, f.i[6]);
-    k.b111 = fetch_bits<DT>(base, f.i[7]);
+    if (bricks32) {
+      // byte offsets from the array's uniform base in 32 bits (channel bases
+      // differ between lanes): no 64-bit address per voxel
+      const uint32_t at = uint32_t(c) * uint32_t(brick_stride);
+      k.b000 = fetch_bits_at<DT>(bricks, at + f.i[0] * kBytes);
+      k.b100 = fetch_bits_at<DT>(bricks, at + f.i[1] * kBytes);
+      k.b010 = fetch_bits_at<DT>(bricks, at + f.i[2] * kBytes);
+      k.b110 = fetch_bits_at<DT>(bricks, at + f.i[3] * kBytes);
+      k.b001 = fetch_bits_at<DT>(bricks, at + f.i[4] * kBytes);
+      k.b101 = fetch_bits_at<DT>(bricks, at + f.i[5] * kBytes);
+      k.b011 = fetch_bits_at<DT>(bricks, at + f.i[6] * kBytes);
+      k.b111 = fetch_bits_at<DT>(bricks, at + f.i[7] * kBytes);
+    } else {
+      const uint8_t* base = bricks + size_t(c) * brick_stride;
+      k.b000 = fetch_bits<DT>(base, f.i[0]);
+      k.b100 = fetch_bits<DT>(base, f.i[1]);
+      k.b010 = fetch_bits<DT>(base, f.i[2]);
+      k.b110 = fetch_bits<DT>(base, f.i[3]);
+      k.b001 = fetch_bits<DT>(base, f.i[4]);
+      k.b101 = fetch_bits<DT>(base, f.i[5]);
+      k.b011 = fetch_bits<DT>(base, f.i[6]);
+      k.b111 = fetch_bits<DT>(base, f.i[7]);
+      k.arrived();  // (keeps the compiler from merging the two branches' loads again)
+    }
     return k;
   }
   __device__ __forceinline__ float lerp8(const float v[8], float fx, float fy, float fz,
@@ -184,24 +203,33 @@ struct Ctx {
                           "+v"(w[4][j]), "+v"(w[5][j]), "+v"(w[6][j]), "+v"(w[7][j]));
     }
   };
+  // a voxel of a group of the joint copy
+  template <class Offset>
+  static __device__ __forceinline__ void load_group(uint32_t (&w)[kWords], const uint8_t* base, Offset at) {
+    if constexpr (kWords == 1) {
+      w[0] = *reinterpret_cast<const uint32_t*>(base + at);
+    } else if constexpr (kWords == 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(base + at);
+      w[0] = v.x;
+      w[1] = v.y;
+    } else {
+      const uint4 v = *reinterpret_cast<const uint4*>(base + at);
+      w[0] = v.x;
+      w[1] = v.y;
+      w[2] = v.z;
+      w[3] = v.w;
+    }
+  }
   __device__ __forceinline__ void load_channels(AllChannels& a, int c0) const {
     if (joint) {
       const uint8_t* base = joint + size_t(c0 >> 2) * joint_stride;
+      if (joint_stride <= 0xffffffffull) {  // 32-bit byte offsets, as corners()
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if constexpr (kWords == 1) {
-          a.w[i][0] = reinterpret_cast<const uint32_t*>(base)[a.f.i[i]];
-        } else if constexpr (kWords == 2) {
-          const uint2 v = reinterpret_cast<const uint2*>(base)[a.f.i[i]];
-          a.w[i][0] = v.x;
-          a.w[i][1] = v.y;
-        } else {
-          const uint4 v = reinterpret_cast<const uint4*>(base)[a.f.i[i]];
-          a.w[i][0] = v.x;
-          a.w[i][1] = v.y;
-          a.w[i][2] = v.z;
-          a.w[i][3] = v.w;
-        }
+        for (int i = 0; i < 8; ++i) load_group(a.w[i], base, a.f.i[i] * (4u * kBytes));
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) load_group(a.w[i], base, uint64_t(a.f.i[i]) * (4u * kBytes));
+        a.arrived();
       }
     } else {
       const uint8_t* base = bricks + size_t(c0) * brick_stride;
