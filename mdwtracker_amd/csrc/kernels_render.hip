@@ -51,16 +51,7 @@ __device__ __forceinline__ void render_body(const RenderParams& P) {
 
   const uint32_t slot = block_slot(blockIdx.x, uint32_t(P.fr.n_blocks));
   const uint32_t bxy = P.fr.block_order[slot];
-  ViewCtx V;
-  V.cam = &P.cam;
-  V.W = P.fr.width;
-  V.H = P.fr.height;
-  V.spp = P.fr.spp;
-  V.seed = P.fr.seed;
-  V.frame_id = P.fr.frame_id;
-  V.accum_id = P.fr.accum_id;
-  V.accum = P.fr.accum;
-  V.m2 = P.fr.m2;
+  const ViewCtx V = frame_view(P);
   render_block<MODE, DT, COUNT, LIT>(P, X, V, int(bxy & 0xffffu), int(bxy >> 16), cnt);
   if (COUNT) flush_counts(P, cnt);
   // per-wave duration for the cost-sorted block order of later frames
@@ -83,6 +74,70 @@ template <int MODE, int DT, bool COUNT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void render_kernel_w6(
     RenderParams P) {
   render_body<MODE, DT, COUNT, false>(P);
+}
+
+// The ray marchers, several frames per launch (team_quad): workgroup i renders
+// quad i % q of the pixel block at position i / q of the block order. Frame by
+// frame, a launch's few long waves left a SIMD 1.5 of them on average (70 % of
+// the cycles issuing vector instructions): 620 us a frame (-m 8, 640 x 480,
+// 4 x 128^3 u8), 340 us at four frames per launch. Four waves per SIMD are stated
+// (the natural budget of 170 VGPRs gives two: 510 us; three: 400 us), three for
+// f32, whose voxels in flight take more (535 and 419 us at two and three on four
+// channels, 573 with the spills of four).
+template <int MODE, int DT, bool LIT>
+__device__ __forceinline__ void march_team(const RenderParams& P) {
+  extern __shared__ float4 s_tf[];
+  __shared__ ChanTf s_ch[kMaxChannels];
+  __shared__ FoldLds s_fold[kThreads / 64];
+  const uint64_t t_begin = P.fr.wave_cost ? wall_clock64() : 0ull;
+  load_tf_lds(P, s_tf, s_ch);
+  __syncthreads();
+  Ctx<DT> X;
+  X.init(P, s_tf, s_ch);
+  const uint32_t q = uint32_t(P.fr.bw * P.fr.bh) / 64u;
+  const uint32_t slot_b = blockIdx.x / q, quad = blockIdx.x - slot_b * q;
+  const uint32_t bxy = P.fr.block_order[slot_b];
+  const ViewCtx V = frame_view(P);
+  team_quad(
+      P, V, int(bxy & 0xffffu), int(bxy >> 16), int(quad), P.fr.team_frames,
+      [&](int w) -> FoldLds& { return s_fold[w]; },
+      [&](int f, int s, int px, int py, bool valid, uint32_t pixel, HitRec& h) {
+        Counts cnt = {0, 0, 0, 0};
+        h.missed = true;
+        return valid ? pixel_sample<MODE, DT, LIT>(P, X, V, V.frame_id + uint32_t(f), s, px, py, pixel, h, cnt)
+                     : make_float4(0.f, 0.f, 0.f, 0.f);
+      });
+  if (P.fr.wave_cost && threadIdx.x == 0)
+    P.fr.wave_cost[blockIdx.x] = uint32_t(wall_clock64() - t_begin);
+}
+
+template <int MODE, int DT, bool LIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void march_team_kernel(
+    RenderParams P) {
+  march_team<MODE, DT, LIT>(P);
+}
+template <int MODE, bool LIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void march_team_kernel_f32(
+    RenderParams P) {
+  march_team<MODE, MDWT_DT_F32, LIT>(P);
+}
+
+template <int MODE, bool LIT>
+RenderFn march_team_dt(int dtype) {
+  switch (dtype) {
+    case MDWT_DT_U8: return march_team_kernel<MODE, MDWT_DT_U8, LIT>;
+    case MDWT_DT_U16: return march_team_kernel<MODE, MDWT_DT_U16, LIT>;
+    case MDWT_DT_F16: return march_team_kernel<MODE, MDWT_DT_F16, LIT>;
+    default: return march_team_kernel_f32<MODE, LIT>;
+  }
+}
+RenderFn select_march_team(int mode, int dtype, bool lit) {
+  switch (mode) {
+    case 6: return lit ? march_team_dt<6, true>(dtype) : march_team_dt<6, false>(dtype);
+    case 7: return lit ? march_team_dt<7, true>(dtype) : march_team_dt<7, false>(dtype);
+    case 8: return lit ? march_team_dt<8, true>(dtype) : march_team_dt<8, false>(dtype);
+    default: return march_team_dt<9, false>(dtype);  // no lighting
+  }
 }
 
 // ---------------------------------------------------------- test hooks -----
@@ -294,16 +349,22 @@ hipError_t prepare(RenderFn f, size_t lds) {
 }
 }  // namespace
 
+bool several_frames_apply(const RenderParams& p, int mode, bool count) {
+  return !count && (mode >= 6 || (p.fr.schedule == 1 && wave_schedule_applies(p, mode, count)));
+}
+
 hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s) {
   const bool lit = is_lit(p);
   const bool wave = p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
-  if (p.fr.team_frames > 0 && !wave) return hipErrorInvalidValue;
-  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, p.fr.team_frames > 0 ? 3 : 0)
-                          : select_render(mode, dtype, count, lit, six_waves(p, dtype));
+  const bool team = p.fr.team_frames > 0;
+  if (team && !several_frames_apply(p, mode, count)) return hipErrorInvalidValue;
+  const RenderFn f = wave   ? select_wave_kernel(p, mode, dtype, team ? 3 : 0)
+                     : team ? select_march_team(mode, dtype, is_shaded(p))
+                            : select_render(mode, dtype, count, lit, six_waves(p, dtype));
   const hipError_t e = prepare(f, lds);
   if (e != hipSuccess) return e;
-  if (p.fr.team_frames > 0) {  // one workgroup per 8x8 quad
+  if (team) {  // one workgroup per 8x8 quad
     hipLaunchKernelGGL(f, dim3(unsigned(p.fr.n_blocks) * unsigned(p.fr.bw * p.fr.bh / 64)),
                        dim3(kThreads), lds, s, p);
     return hipGetLastError();

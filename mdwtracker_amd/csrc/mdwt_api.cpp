@@ -625,13 +625,13 @@ mdwt::RenderParams render_params(const mdwt_renderer* h) {
 }
 
 // Frames of the next launch when `left` are to be rendered: several by the
-// team kernel (see team_quad in wave_paths.hpp), whose four waves take four
+// team kernel (see team_quad in render_paths.hpp), whose four waves take four
 // draws (samples) at a time, or 0 for one frame by the one-frame kernels. Only
 // whole rounds of four draws: in a partial one, waves hold their workgroup's
 // LDS and do nothing. About 32 draws: longer launches gained under 1 %.
 constexpr int kTeamDraws = 32;
 int team_frames(const mdwt_renderer* h, const mdwt::RenderParams& p, int left) {
-  if (p.fr.schedule != 1 || !mdwt::wave_schedule_applies(p, h->mode, false)) return 0;
+  if (!mdwt::several_frames_apply(p, h->mode, false)) return 0;
   // the auxiliary buffers stop at their own frame count
   if (p.fr.aov && h->aov_frames) left = std::min(left, int(uint32_t(h->aov_frames) - h->accum_id));
   const int step = h->spp % 4 == 0 ? 1 : (h->spp % 2 == 0 ? 2 : 4);

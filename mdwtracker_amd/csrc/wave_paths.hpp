@@ -822,109 +822,24 @@ __device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>&
   if (valid) finish_pixel(P, V.accum, V.m2, V.accum_id, V.spp, pixel, fr, fg, fb, fa);
 }
 
-// One 8x8 pixel quad, `frames` frames: the workgroup's four waves trace four
-// consecutive draws (frame, sample) of the quad at a time and the workgroup
-// folds their contributions into the running means in draw order, so the image
-// is the one that frame after frame gives, bit for bit. The frame kernel issues
-// VALU instructions over 80% of its cycles, so what can go is the rest: the
-// accumulator moves once per launch instead of once per frame, the waves of a
-// workgroup read the same cells and voxels (one L1), and the launch's tail,
-// its set-up and its tables are shared by the frames. 64 frames of 1024^2
-// (-m 2, 4 x 256^3 u8): 137 us a frame one by one, 130 / 121 / 118 us at 4 / 8 /
-// 32 draws per launch. Each wave looping over the frames of its own quad
-// without the fold gave 124 us (and nothing on 640 x 480, where the quads alone
-// do not fill the chip: 8 frames of 4 samples 2180 -> 2090 us against 1630).
-// Folding: lane l of wave w owns component l % 4 of the quad's pixel
-// 16 w + l / 4. The contributions pass through the waves' record lists, which
-// are free after a draw.
-struct FoldLds {
-  float4 add[64];
-  float2 hit[64];  // first-hit distance, hit channel (bits; ~0: a miss)
-};
+// One 8x8 pixel quad, `frames` frames (team_quad): the contributions pass through
+// the waves' record lists, which are free after a draw.
 static_assert(sizeof(FoldLds) <= sizeof(Record) * kRecords, "folded through the record list");
-
 template <int MODE, int DT, bool WIDE, bool LIT>
-__device__ __forceinline__ void team_quad(const RenderParams& P, const Ctx<DT>& X, WaveLds* s_wave,
-                                          const float* s_alpha, const ViewCtx& V, int bx, int by,
-                                          int quad, int frames) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int qs = P.fr.bw == 16 ? 1 : 0;
-  const int qx = bx * P.fr.bw + (quad & qs) * 8, qy = by * P.fr.bh + (quad >> qs) * 8;
-  if (qx >= V.W || qy >= V.H) return;  // the whole workgroup
-  const int px = qx + (lane & 7), py = qy + (lane >> 3);
-  const bool valid = px < V.W && py < V.H;
-  const uint32_t pixel = valid ? uint32_t(px) + uint32_t(V.W) * uint32_t(py) : 0u;
+__device__ __forceinline__ void wave_team_quad(const RenderParams& P, const Ctx<DT>& X, WaveLds* s_wave,
+                                               const float* s_alpha, const ViewCtx& V, int bx, int by,
+                                               int quad, int frames) {
+  WaveLds& L = s_wave[threadIdx.x >> 6];
   const V3 w2u = world_to_unit(P);
-  const int draws = frames * V.spp;
-  // this lane's component of the fold
-  const int fp = 16 * wave + (lane >> 2), comp_i = lane & 3;
-  const int fx = qx + (fp & 7), fy = qy + (fp >> 3);
-  const bool fold = fx < V.W && fy < V.H;
-  const size_t fi = fold ? 4 * (size_t(fx) + size_t(V.W) * fy) + comp_i : 0;
-  const size_t fpix = fi >> 2;
-  float* accum = reinterpret_cast<float*>(V.accum) + fi;
-  float* m2 = V.m2 ? reinterpret_cast<float*>(V.m2) + fi : nullptr;
-  const int ng = aov_groups(P.vol.channels);
-  float* aov = P.fr.aov ? reinterpret_cast<float*>(P.fr.aov) + 4 * size_t(ng) * fpix + comp_i : nullptr;
-  const float sum0 = comp_i == 3 ? 1.f : 0.f, spp = float(V.spp);
-  float mean = 0.f, sq = 0.f, sum = sum0;
-  int sample = 0;
-  uint32_t accum_id = V.accum_id;
-  for (int d0 = 0; d0 < draws; d0 += 4) {
-    const int dr = d0 + wave;
-    if (dr < draws) {
-      WaveLds& L = s_wave[wave];
-      const int f = dr / V.spp, s = dr - f * V.spp;
-      HitRec h;
-      const float4 o = trace_sample<MODE, DT, WIDE, LIT>(P, X, L, s_alpha, V, V.frame_id + uint32_t(f),
-                                                         s, px, py, valid, pixel, w2u, h);
-      wave_sync();
-      FoldLds& F = *reinterpret_cast<FoldLds*>(L.rec);
-      F.add[lane] = o;
-      if (P.fr.aov)
-        F.hit[lane] = make_float2(h.tHit, __uint_as_float(h.missed ? ~0u : uint32_t(h.channel)));
-    }
-    if (d0 == 0 && fold && P.fr.accumulate) {
-      mean = *accum;
-      if (m2) sq = *m2;
-    }
-    __syncthreads();
-    if (fold) {
-      for (int k = 0; k < 4 && d0 + k < draws; ++k) {
-        const FoldLds& F = *reinterpret_cast<const FoldLds*>(s_wave[k].rec);
-        sum = sum + reinterpret_cast<const float*>(&F.add[fp])[comp_i];
-        if (aov) {  // aov_sample
-          const float2 hh = F.hit[fp];
-          const uint32_t code = __float_as_uint(hh.y);
-          const bool hit = code != ~0u;
-          const uint32_t n = (P.fr.accumulate ? accum_id * uint32_t(V.spp) : 0u) + uint32_t(sample);
-          const float kf = float(n), k1 = float(n + 1u);
-          for (int g = 0; g < ng; ++g) {
-            const int slot = 4 * g + comp_i;
-            const float v = slot == 0 ? (hit ? hh.x : 0.f)
-                            : slot == 1 ? (hit ? 0.f : 1.f)
-                                        : (hit && int(code) == slot - 2 ? 1.f : 0.f);
-            const float old = n ? aov[4 * g] : 0.f;
-            aov[4 * g] = (v + kf * old) / k1;
-          }
-        }
-        if (++sample == V.spp) {  // finish_pixel
-          const float v = V.spp == 1 ? sum : sum / spp;
-          const float kf = float(accum_id), k1 = float(accum_id + 1u);
-          mean = P.fr.accumulate ? (v + kf * mean) / k1 : v;
-          if (m2) sq = P.fr.accumulate ? (v * v + kf * sq) / k1 : v * v;
-          sample = 0;
-          sum = sum0;
-          ++accum_id;
-        }
-      }
-    }
-    if (d0 + 4 < draws) __syncthreads();
-  }
-  if (fold) {
-    *accum = mean;
-    if (m2) *m2 = sq;
-  }
+  team_quad(
+      P, V, bx, by, quad, frames,
+      [&](int w) -> FoldLds& { return *reinterpret_cast<FoldLds*>(s_wave[w].rec); },
+      [&](int f, int s, int px, int py, bool valid, uint32_t pixel, HitRec& h) {
+        const float4 o = trace_sample<MODE, DT, WIDE, LIT>(P, X, L, s_alpha, V, V.frame_id + uint32_t(f),
+                                                           s, px, py, valid, pixel, w2u, h);
+        wave_sync();
+        return o;
+      });
 }
 
 // Three waves per SIMD is what the LDS allows; stated, so that the register
@@ -949,20 +864,6 @@ __device__ __forceinline__ void team_quad(const RenderParams& P, const Ctx<DT>& 
   /* colours of a hit are looked up in the HBM copy of the tables */            \
   X.init(P, reinterpret_cast<const float4*>(P.tf.tab), s_ch);                     \
   [[maybe_unused]] WaveLds& L = s_wave[threadIdx.x >> 6];
-
-__device__ __forceinline__ ViewCtx frame_view(const RenderParams& P) {
-  ViewCtx V;
-  V.cam = &P.cam;
-  V.W = P.fr.width;
-  V.H = P.fr.height;
-  V.spp = P.fr.spp;
-  V.seed = P.fr.seed;
-  V.frame_id = P.fr.frame_id;
-  V.accum_id = P.fr.accum_id;
-  V.accum = P.fr.accum;
-  V.m2 = P.fr.m2;
-  return V;
-}
 
 // One view: workgroup i renders the pixel block at position block_slot(i) of
 // the frame's block order.
@@ -989,8 +890,8 @@ MDWT_WAVE_KERNEL void render_wave_team(RenderParams P) {
   const uint32_t slot_b = blockIdx.x / q, quad = blockIdx.x - slot_b * q;
   const uint32_t bxy = P.fr.block_order[slot_b];
   const ViewCtx V = frame_view(P);
-  team_quad<MODE, DT, WIDE, LIT>(P, X, s_wave, s_alpha, V, int(bxy & 0xffffu), int(bxy >> 16),
-                                 int(quad), P.fr.team_frames);
+  wave_team_quad<MODE, DT, WIDE, LIT>(P, X, s_wave, s_alpha, V, int(bxy & 0xffffu), int(bxy >> 16),
+                                      int(quad), P.fr.team_frames);
   if (P.fr.wave_cost && threadIdx.x == 0)
     P.fr.wave_cost[blockIdx.x] = uint32_t(wall_clock64() - t_begin);
 }

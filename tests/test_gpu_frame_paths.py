@@ -69,7 +69,8 @@ def test_shading_and_aov_on_both_schedules(capi, mode, channels, dtype):
 @pytest.mark.parametrize("mode,channels,dtype,shaded", [
     (0, 3, np.uint8, False), (0, 5, np.uint16, False), (1, 4, np.float16, False),
     (2, 4, np.uint8, False), (2, 10, np.float32, True), (3, 2, np.uint16, True),
-    (4, 4, np.uint8, False), (5, 1, np.float32, True)])
+    (4, 4, np.uint8, False), (5, 1, np.float32, True), (6, 2, np.uint16, False),
+    (7, 3, np.uint8, True), (8, 4, np.float32, False), (9, 5, np.float16, True)])
 def test_several_frames_in_one_launch(capi, mode, channels, dtype, shaded):
     """n frames in one call against n calls of one frame: around the launch's
     rounds of four draws and its 32 draws, with the auxiliary buffers ending
