@@ -349,8 +349,14 @@ hipError_t prepare(RenderFn f, size_t lds) {
 }
 }  // namespace
 
+// The marchers' transfer-function tables share the LDS with the fold (6 KiB):
+// several frames per launch where a CU holds two such workgroups, the one-frame
+// kernels above that (their tables may fill the LDS).
 bool several_frames_apply(const RenderParams& p, int mode, bool count) {
-  return !count && (mode >= 6 || (p.fr.schedule == 1 && wave_schedule_applies(p, mode, count)));
+  if (count) return false;
+  if (mode < 6) return p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
+  const size_t fixed = sizeof(ChanTf) * kMaxChannels + sizeof(FoldLds) * (kThreads / 64);
+  return 2 * (render_lds_bytes(p) + fixed) <= size_t(160) << 10;
 }
 
 hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s) {

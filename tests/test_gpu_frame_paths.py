@@ -148,3 +148,24 @@ def test_majorants_match_the_oracle(capi, texels, mode, conservative):
         out.append(r.read_majorants().view(np.uint32))
         r.close()
     np.testing.assert_array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("mode", [6, 7, 8, 9])
+@pytest.mark.parametrize("texels", [1568, 1572, 3404])
+def test_marchers_with_tables_up_to_the_lds(capi, mode, texels):
+    """Tables of three channels: the longest with which two workgroups of the
+    several-frame kernel fit a CU, the next, and the longest of the one-frame
+    kernels (160 KiB with the channel parameters), which the fold's LDS does not
+    fit beside."""
+    vols, _ = volume(3, np.uint8, dims=(19, 22, 17))
+    rng = np.random.default_rng(texels)
+    tfs = [rng.uniform(0, 1, (texels, 4)).astype(np.float32) for _ in vols]
+    out = []
+    for split in (False, True):
+        print(f"[paths] mode {mode} texels {texels} split {split}", flush=True)
+        r = renderer(capi, vols, tfs, mode, (43, 30), 1, 1, mc=(4, 5, 3), opacity=0.2)
+        for _ in range(8 if split else 1):
+            r.render(1 if split else 8)
+        out.append(r.read_accum().view(np.uint32))
+        r.close()
+    np.testing.assert_array_equal(*out)
