@@ -257,7 +257,7 @@ int mdwt_batch_read_view(mdwt_renderer* h, int view, float* rgba, float* m2);
  * Launch form 0: HIP events around its launch on its stream (so it includes
  * time shared with views on the other streams); form 1: from the launch's
  * first workgroup start to the view's last workgroup end (device wall
- * clock). MDWT_ERR_STATE before the first batched frame. */
+ * clock). Where a launch renders several frames, its time divided by them. MDWT_ERR_STATE before the first batched frame. */
 int mdwt_batch_view_times(mdwt_renderer* h, float* us);
 /* Autotuner: times `frames` frames (after one warm-up frame) for every
  * combination of macrocell size s (voxels per macrocell side; grid = dims /

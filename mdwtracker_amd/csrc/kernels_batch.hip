@@ -12,7 +12,8 @@
 // number of items.
 // Under the wave-coherent schedule, -m 0 to -m 5 views run wave_paths.hpp's
 // render_views_wave and (without shading) render_views_wave_persistent
-// instead, with the same items and ids.
+// instead, with the same items and ids; form 1's frames by render_wave_team,
+// several a launch.
 // No reference counterpart: the reference renders one camera per owlLaunch2D
 // (renderer.cpp:949).
 #include "mdwt_internal.hpp"
@@ -249,6 +250,8 @@ bool wave_persistent(const RenderParams& p, int mode) {
 }
 }  // namespace
 
+bool several_view_frames_apply(const RenderParams& p, int mode) { return wave_views(p, mode, false); }
+
 hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int dtype, int* out) {
   const bool wave = wave_persistent(p, mode);
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
@@ -276,12 +279,17 @@ hipError_t launch_views_persistent(const RenderParams& p, int mode, int dtype, i
 
 hipError_t launch_views(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s) {
   if (p.fr.n_items <= 0) return hipSuccess;
-  const bool wave = wave_views(p, mode, count);
+  const bool wave = wave_views(p, mode, count), team = p.fr.team_frames > 0;
+  if (team && !wave) return hipErrorInvalidValue;
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
-  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 1)
+  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, team ? 3 : 1)
                           : select_views(mode, dtype, count, is_lit(p), wide_views(p, dtype));
   const hipError_t e = prepare(f, lds);
   if (e != hipSuccess) return e;
+  if (team) {  // one workgroup per 8x8 quad
+    hipLaunchKernelGGL(f, dim3(unsigned(p.fr.n_items) * unsigned(p.fr.bw * p.fr.bh / 64)), dim3(256), lds, s, p);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(f, dim3(unsigned(p.fr.n_items)), dim3(unsigned(p.fr.bw * p.fr.bh)), lds, s, p);
   return hipGetLastError();
 }

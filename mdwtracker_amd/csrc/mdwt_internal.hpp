@@ -21,6 +21,8 @@ RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form
 // whether launch_render can render several frames (team_frames) in one launch:
 // the wave-coherent modes and the ray marchers
 bool several_frames_apply(const RenderParams& p, int mode, bool count);
+// the same of launch_views: the wave-coherent modes
+bool several_view_frames_apply(const RenderParams& p, int mode);
 RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int form);
 // dynamic LDS of a wave-coherent launch (transfer-function opacities)
 size_t wave_lds_bytes(const RenderParams& p);

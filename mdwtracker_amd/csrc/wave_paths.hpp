@@ -880,22 +880,6 @@ MDWT_WAVE_KERNEL void render_wave(RenderParams P) {
         uint32_t(wall_clock64() - t_begin);
 }
 
-// One view, P.fr.team_frames frames: workgroup i renders quad i % q of the
-// pixel block at position i / q of the block order (q quads per block).
-template <int MODE, int DT, bool WIDE, bool LIT>
-MDWT_WAVE_KERNEL void render_wave_team(RenderParams P) {
-  const uint64_t t_begin = P.fr.wave_cost ? wall_clock64() : 0ull;
-  MDWT_WAVE_PROLOGUE
-  const uint32_t q = uint32_t(P.fr.bw * P.fr.bh) / 64u;
-  const uint32_t slot_b = blockIdx.x / q, quad = blockIdx.x - slot_b * q;
-  const uint32_t bxy = P.fr.block_order[slot_b];
-  const ViewCtx V = frame_view(P);
-  wave_team_quad<MODE, DT, WIDE, LIT>(P, X, s_wave, s_alpha, V, int(bxy & 0xffffu), int(bxy >> 16),
-                                      int(quad), P.fr.team_frames);
-  if (P.fr.wave_cost && threadIdx.x == 0)
-    P.fr.wave_cost[blockIdx.x] = uint32_t(wall_clock64() - t_begin);
-}
-
 __device__ __forceinline__ ViewCtx batch_view(const RenderParams& P, uint32_t code,
                                               uint32_t frame_id, uint32_t accum_id) {
   const ViewParams* vp = P.fr.views + (code >> 20);
@@ -910,6 +894,42 @@ __device__ __forceinline__ ViewCtx batch_view(const RenderParams& P, uint32_t co
   V.accum = vp->accum;
   V.m2 = vp->m2;
   return V;
+}
+
+// P.fr.team_frames frames of one view or of every view of a batch: workgroup i
+// renders quad i % q of pixel block i / q of the block order or of the items (q
+// quads per block). A batch's item_ticks get the start of an item's first quad
+// and the latest end of its quads (stamps of earlier launches are smaller).
+// 24 views of 128^2 to 512^2 (-m 2, 4 x 128^3 f16), four frames in one launch against
+// four launches: 2.63 -> 2.51 ms at 1 to 4 samples, 1.11 -> 1.03 ms at one sample.
+template <int MODE, int DT, bool WIDE, bool LIT>
+MDWT_WAVE_KERNEL void render_wave_team(RenderParams P) {
+  const uint64_t t_begin = P.fr.wave_cost || P.fr.item_ticks ? wall_clock64() : 0ull;
+  MDWT_WAVE_PROLOGUE
+  const uint32_t q = uint32_t(P.fr.bw * P.fr.bh) / 64u;
+  const uint32_t slot_b = blockIdx.x / q, quad = blockIdx.x - slot_b * q;
+  ViewCtx V;
+  uint32_t bx, by;
+  if (P.fr.views) {
+    const uint32_t code = P.fr.items[slot_b];
+    V = batch_view(P, code, P.fr.frame_id, P.fr.accum_id);
+    bx = code & 0x3ffu;
+    by = (code >> 10) & 0x3ffu;
+  } else {
+    const uint32_t bxy = P.fr.block_order[slot_b];
+    V = frame_view(P);
+    bx = bxy & 0xffffu;
+    by = bxy >> 16;
+  }
+  wave_team_quad<MODE, DT, WIDE, LIT>(P, X, s_wave, s_alpha, V, int(bx), int(by), int(quad),
+                                      P.fr.team_frames);
+  if (threadIdx.x == 0) {
+    if (P.fr.wave_cost) P.fr.wave_cost[blockIdx.x] = uint32_t(wall_clock64() - t_begin);
+    if (P.fr.item_ticks) {
+      if (quad == 0) P.fr.item_ticks[2 * slot_b] = t_begin;
+      atomicMax(&P.fr.item_ticks[2 * slot_b + 1], static_cast<unsigned long long>(wall_clock64()));
+    }
+  }
 }
 
 // Batched views, launch form 1: workgroup i renders item i (view << 20 |

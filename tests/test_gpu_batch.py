@@ -324,3 +324,40 @@ def test_ten_channel_batch_equals_single_view_renders(capi, launch):
         np.testing.assert_array_equal(_bits(m_b), _bits(m_s))
         assert a_s[..., :3].max() > 0.0  # the views see the volume
     g.close()
+
+
+@pytest.mark.parametrize("launch", [0, 1])
+@pytest.mark.parametrize("mode,spps,frames,shaded,accumulate,block", [
+    (0, (4, 4, 8), 1, False, True, 256), (1, (1, 3, 2), 3, False, True, 64),
+    (2, (1, 2, 4), 13, False, True, 128), (2, (33, 1, 2), 5, True, True, 256),
+    (3, (2, 2, 2), 6, True, False, 256), (4, (1, 1, 1), 4, False, False, 64),
+    (5, (3, 1, 1), 2, False, True, 256), (8, (1, 2, 4), 5, False, True, 256)])
+def test_several_frames_in_one_launch(capi, scene, launch, mode, spps, frames, shaded, accumulate, block):
+    """n batched frames in one call against n calls of one frame of the
+    thread-per-pixel kernels, over views of uneven sizes and sample counts."""
+    views = _views(len(spps), seed=mode)
+    for v, spp in zip(views, spps):
+        v["spp"] = spp
+    out = []
+    for split in (False, True):
+        print(f"[batch] launch {launch} mode {mode} spps {spps} frames {frames} split {split}", flush=True)
+        g = capi.MdwtRenderer(0)
+        g.set_moments(True)
+        scenes.load_scene(g, scene, mode)
+        g.set_frame(8, 8, 1, accumulate, (0.1, 0.2, 0.3))
+        g.set_schedule(0 if split else 1)
+        g.set_block(block)
+        if shaded:
+            g.set_light((0.3, -1.0, 0.2), True, True)
+        g.batch_set_launch(launch)
+        g.batch_set_views(views)
+        for _ in range(2):
+            g.batch_reset()
+            for _ in range(frames if split else 1):
+                g.batch_render(1 if split else frames)
+        us = g.batch_view_times()
+        assert (us > 0).all() and (us < 1e6).all()
+        out.append([_bits(a) for i in range(len(views)) for a in g.batch_read_view(i, with_m2=True)])
+        g.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
