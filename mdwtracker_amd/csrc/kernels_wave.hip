@@ -48,7 +48,8 @@ RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form
 }
 
 size_t wave_lds_bytes(const RenderParams& p) {
-  static_assert(sizeof(WaveLds) % 16 == 0, "the opacity table follows the per-wave LDS");
+  static_assert(sizeof(WaveLds<kRecords>) % 16 == 0 && sizeof(WaveLds<kRecordsWide>) % 16 == 0,
+                "the opacity table follows the per-wave LDS");
   return size_t(p.vol.channels) * size_t(p.tf.stride) * sizeof(float);
 }
 

@@ -67,6 +67,13 @@ namespace mdwt {
 namespace {
 
 constexpr int kRecords = 412;  // records per wave and round
+// The same above four channels of -m 0 / 1 / 2. Their opacity tables come on top
+// of the waves' LDS (1 KiB per channel at 256 texels): with 290 records three
+// workgroups fit a CU up to twelve such channels, with 412 two fit. Eight frames
+// of 640x480 (128^3 f32 voxels) at 5 / 8 / 10 / 12 channels: 485 / 520 / 617 / 659 us with
+// 412, 396 / 417 / 484 / 503 us with 290; 400 records: 393 us at 5, unchanged above;
+// 322: 400 / 425 / 491 / 612. Ten channels of 256 x 256 x 64, 1024^2: 2.57 -> 1.92 ms.
+constexpr int kRecordsWide = 290;
 constexpr int kMaxAhead = 16;  // cells a ray walks ahead per round, at most (-m 0: 64 / C above 4 channels)
 constexpr int kStack = 128;    // the item stack: < 64 left + one channel's 64 pushes
 // Safety factor of the certain-exit test (see the enter phase): far above the
@@ -117,8 +124,10 @@ struct Draw {
 // round (the smallest key among its hits and the box ends that end it, see
 // event_key / clock_key) is an LDS atomic minimum, and -m 0's box ends set
 // bits of a word, so only events write: leaving a cell writes nothing.
+template <int RECORDS>
 struct WaveLds {
-  Record rec[kRecords];
+  static constexpr int kCapacity = RECORDS;
+  Record rec[RECORDS];
   Item stk[kStack];  // first steps (x = uniform) and null-collision tests (x = t)
   WaveRay ray[64];
   unsigned long long ev[64];   // per ray: first event key of the round
@@ -157,8 +166,8 @@ __device__ __forceinline__ uint64_t event_key(uint32_t visit, uint32_t flag, flo
 __device__ __forceinline__ uint64_t clock_key(uint32_t visit, uint32_t flag, float t, uint32_t ch) {
   return (uint64_t(visit) << 37) | (uint64_t(order_bits(t)) << 5) | (uint64_t(ch) << 1) | flag;
 }
-template <int MODE>
-__device__ __forceinline__ void on_hit(WaveLds& L, const Record& R, int c, float t) {
+template <int MODE, class Lds>
+__device__ __forceinline__ void on_hit(Lds& L, const Record& R, int c, float t) {
   if (MODE == 1) {
     atomicMin(&L.ev[R.vl >> kVisitBits], clock_key(R.vl & kVisitMask, 0u, t, uint32_t(c)));
     return;
@@ -166,8 +175,8 @@ __device__ __forceinline__ void on_hit(WaveLds& L, const Record& R, int c, float
   const uint32_t ch = MODE == 0 ? uint32_t(15 - c) : uint32_t(c);
   atomicMin(&L.ev[R.vl >> kVisitBits], event_key(R.vl & kVisitMask, 0u, t, ch));
 }
-template <int MODE>
-__device__ __forceinline__ void on_box_end(WaveLds& L, const Record& R, int c, int C, float t) {
+template <int MODE, class Lds>
+__device__ __forceinline__ void on_box_end(Lds& L, const Record& R, int c, int C, float t) {
   if (MODE == 1) {
     atomicMin(&L.ev[R.vl >> kVisitBits], clock_key(R.vl & kVisitMask, 1u, t, uint32_t(c)));
   } else if (MODE >= 3) {
@@ -224,8 +233,8 @@ __device__ __forceinline__ float alpha_lookup(const float* s_a, const ChanTf& t,
 // (visit, channel) stream. Returns true when the step needs another test (tn
 // inside the cell and before the box's end); otherwise its event, if any, is
 // recorded here.
-template <int MODE, int DT>
-__device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+template <int MODE, int DT, class Lds>
+__device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& X, Lds& L,
                                           const float* s_a, V3 w2u, const Draw& D, int c,
                                           const Record& R, const WaveRay& Y, uint32_t j, float t,
                                           float m, float& tn) {
@@ -307,8 +316,8 @@ __device__ __forceinline__ bool null_test(const RenderParams& P, const Ctx<DT>& 
 // its t. Full passes push a rejected step's successor back; the round's last
 // pass (DRAIN, fewer than 64 items) keeps every lane on its item until it is
 // settled.
-template <int MODE, int DT, bool DRAIN>
-__device__ __forceinline__ void item_pass(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+template <int MODE, int DT, bool DRAIN, class Lds>
+__device__ __forceinline__ void item_pass(const RenderParams& P, const Ctx<DT>& X, Lds& L,
                                           const float* s_a, uint32_t& n_items, V3 w2u,
                                           const Draw& D) {
   const int lane = threadIdx.x & 63;
@@ -455,8 +464,8 @@ struct CellWalk {
 // The first event of one sample's ray per lane: the tracking rounds of the
 // header comment. d, alive and L.ray[lane] hold the lane's ray; hit_c and hit_t
 // (grid units) are set where the result is true.
-template <int MODE, int DT, bool WIDE>
-__device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+template <int MODE, int DT, bool WIDE, class Lds>
+__device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>& X, Lds& L,
                                            const float* s_alpha, V3 w2u, const Draw& D, CellWalk& d,
                                            bool alive, int& hit_c, float& hit_t) {
   const int lane = threadIdx.x & 63;
@@ -469,7 +478,7 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
     const uint64_t live = __ballot(alive);
     if (live == 0ull) break;
     const uint32_t n_live = uint32_t(__popcll(live));
-    int K = int(uint32_t(kRecords) / n_live);
+    int K = int(uint32_t(Lds::kCapacity) / n_live);
     K = K > kMaxAhead ? kMaxAhead : K;
     if (MODE == 0 && WIDE && K > 64 / C) K = 64 / C;  // the end-of-box word's visits
     const uint32_t visit0 = visit;
@@ -693,8 +702,8 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
 // shadow rays, as render_block (render_paths.hpp) does them: the shadow ray of
 // every lane that hit runs through the same tracking rounds
 // (deviceCode.cu:383-403), on stream 1.
-template <int MODE, int DT, bool WIDE, bool LIT>
-__device__ __forceinline__ float4 trace_sample(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+template <int MODE, int DT, bool WIDE, bool LIT, class Lds>
+__device__ __forceinline__ float4 trace_sample(const RenderParams& P, const Ctx<DT>& X, Lds& L,
                                                const float* s_alpha, const ViewCtx& V,
                                                uint32_t frame_id, int s, int px, int py, bool valid,
                                                uint32_t pixel, V3 w2u, HitRec& h) {
@@ -797,8 +806,8 @@ __device__ __forceinline__ V3 world_to_unit(const RenderParams& P) {
 
 // The 8x8 pixel quad of this wave in pixel block (bx, by) of view V (a
 // workgroup's bw x bh block has one quad per wave), one frame.
-template <int MODE, int DT, bool WIDE, bool LIT>
-__device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>& X, WaveLds& L,
+template <int MODE, int DT, bool WIDE, bool LIT, class Lds>
+__device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>& X, Lds& L,
                                            const float* s_alpha, const ViewCtx& V, int bx, int by) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int qs = P.fr.bw == 16 ? 1 : 0;
@@ -824,12 +833,13 @@ __device__ __forceinline__ void wave_block(const RenderParams& P, const Ctx<DT>&
 
 // One 8x8 pixel quad, `frames` frames (team_quad): the contributions pass through
 // the waves' record lists, which are free after a draw.
-static_assert(sizeof(FoldLds) <= sizeof(Record) * kRecords, "folded through the record list");
-template <int MODE, int DT, bool WIDE, bool LIT>
-__device__ __forceinline__ void wave_team_quad(const RenderParams& P, const Ctx<DT>& X, WaveLds* s_wave,
+static_assert(sizeof(FoldLds) <= sizeof(Record) * kRecordsWide && kRecordsWide <= kRecords,
+              "folded through the record list");
+template <int MODE, int DT, bool WIDE, bool LIT, class Lds>
+__device__ __forceinline__ void wave_team_quad(const RenderParams& P, const Ctx<DT>& X, Lds* s_wave,
                                                const float* s_alpha, const ViewCtx& V, int bx, int by,
                                                int quad, int frames) {
-  WaveLds& L = s_wave[threadIdx.x >> 6];
+  Lds& L = s_wave[threadIdx.x >> 6];
   const V3 w2u = world_to_unit(P);
   team_quad(
       P, V, bx, by, quad, frames,
@@ -857,13 +867,13 @@ __device__ __forceinline__ void wave_team_quad(const RenderParams& P, const Ctx<
 #define MDWT_WAVE_PROLOGUE                                                        \
   extern __shared__ float s_alpha[];                                              \
   __shared__ ChanTf s_ch[kMaxChannels];                                           \
-  __shared__ WaveLds s_wave[kThreads / 64];                                       \
+  __shared__ WaveLds<WIDE ? kRecordsWide : kRecords> s_wave[kThreads / 64];       \
   load_alpha_lds(P, s_alpha, s_ch);                                               \
   __syncthreads();                                                                \
   Ctx<DT> X;                                                                      \
   /* colours of a hit are looked up in the HBM copy of the tables */            \
   X.init(P, reinterpret_cast<const float4*>(P.tf.tab), s_ch);                     \
-  [[maybe_unused]] WaveLds& L = s_wave[threadIdx.x >> 6];
+  [[maybe_unused]] auto& L = s_wave[threadIdx.x >> 6];
 
 // One view: workgroup i renders the pixel block at position block_slot(i) of
 // the frame's block order.
