@@ -169,3 +169,27 @@ def test_marchers_with_tables_up_to_the_lds(capi, mode, texels):
         out.append(r.read_accum().view(np.uint32))
         r.close()
     np.testing.assert_array_equal(*out)
+
+
+@pytest.mark.parametrize("size,block", [
+    ((8, 8), 64), ((16, 8), 128), ((512, 512), 64), ((520, 512), 64), ((1024, 512), 128),
+    ((1024, 528), 128), ((1024, 1024), 256), ((1040, 1024), 256)])
+def test_cost_order_is_a_permutation(capi, size, block):
+    """Frames of one block up to just past 4096, of 64, 128 and 256 pixels: in
+    cost order every block is still rendered once (the images of Hilbert order)."""
+    vols, tfs = volume(2, np.uint8, dims=(19, 22, 17))
+    out = []
+    for order in (1, 2):
+        print(f"[paths] tile order {order} {size} block {block}", flush=True)
+        r = renderer(capi, vols, tfs, 2, size, 1, 1, mc=(4, 5, 3))
+        r.set_block(block)
+        r.set_tile_order(order)
+        images = []
+        for _ in range(4):
+            r.reset_accumulation()
+            r.render(1)
+            images.append(r.read_accum().view(np.uint32))
+        r.close()
+        out.append(images)
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
