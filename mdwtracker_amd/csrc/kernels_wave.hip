@@ -39,9 +39,12 @@ RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form
   if (is_shaded(p)) return select_wave_lit_kernel(p, mode, dtype, form);
   if (mode == 0)
     return p.vol.channels > 4 ? wave_fn<0, true>(dtype, form) : wave_fn<0, false>(dtype, form);
-  if (mode == 3) return wave_fn<3, false>(dtype, form);
-  if (mode == 4) return wave_fn<4, false>(dtype, form);
-  if (mode == 5) return wave_fn<5, false>(dtype, form);
+  if (mode == 3)
+    return p.vol.channels > 4 ? wave_fn<3, true>(dtype, form) : wave_fn<3, false>(dtype, form);
+  if (mode == 4)
+    return p.vol.channels > 4 ? wave_fn<4, true>(dtype, form) : wave_fn<4, false>(dtype, form);
+  if (mode == 5)
+    return p.vol.channels > 4 ? wave_fn<5, true>(dtype, form) : wave_fn<5, false>(dtype, form);
   if (mode == 1)
     return p.vol.channels > 4 ? wave_fn<1, true>(dtype, form) : wave_fn<1, false>(dtype, form);
   return p.vol.channels > 4 ? wave_fn<2, true>(dtype, form) : wave_fn<2, false>(dtype, form);

@@ -40,9 +40,9 @@ RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int 
     case 0: return wide ? lit_fn<0, true>(dtype, form) : lit_fn<0, false>(dtype, form);
     case 1: return wide ? lit_fn<1, true>(dtype, form) : lit_fn<1, false>(dtype, form);
     case 2: return wide ? lit_fn<2, true>(dtype, form) : lit_fn<2, false>(dtype, form);
-    case 3: return lit_fn<3, false>(dtype, form);
-    case 4: return lit_fn<4, false>(dtype, form);
-    default: return lit_fn<5, false>(dtype, form);
+    case 3: return wide ? lit_fn<3, true>(dtype, form) : lit_fn<3, false>(dtype, form);
+    case 4: return wide ? lit_fn<4, true>(dtype, form) : lit_fn<4, false>(dtype, form);
+    default: return wide ? lit_fn<5, true>(dtype, form) : lit_fn<5, false>(dtype, form);
   }
 }
 

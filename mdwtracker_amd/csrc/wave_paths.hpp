@@ -67,12 +67,14 @@ namespace mdwt {
 namespace {
 
 constexpr int kRecords = 412;  // records per wave and round
-// The same above four channels of -m 0 / 1 / 2. Their opacity tables come on top
+// The same above four channels. Their opacity tables come on top
 // of the waves' LDS (1 KiB per channel at 256 texels): with 290 records three
 // workgroups fit a CU up to twelve such channels, with 412 two fit. Eight frames
 // of 640x480 (128^3 f32 voxels) at 5 / 8 / 10 / 12 channels: 485 / 520 / 617 / 659 us with
 // 412, 396 / 417 / 484 / 503 us with 290; 400 records: 393 us at 5, unchanged above;
 // 322: 400 / 425 / 491 / 612. Ten channels of 256 x 256 x 64, 1024^2: 2.57 -> 1.92 ms.
+// -m 3 / 4 / 5 at ten: 1082 / 1279 / 1287 -> 849 / 1069 / 1077 us; on three channels (801x603,
+// cells of 4 voxels) 290 records were 7 % slower, so up to four keep 412.
 constexpr int kRecordsWide = 290;
 constexpr int kMaxAhead = 16;  // cells a ray walks ahead per round, at most (-m 0: 64 / C above 4 channels)
 constexpr int kStack = 128;    // the item stack: < 64 left + one channel's 64 pushes
@@ -516,12 +518,13 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
     // pass it with a few instructions; the rest are computed exactly, in
     // full batches, from the first-step stack.
     uint32_t n_items = 0u;
-    const int groups = WIDE ? (C + 3) >> 2 : 1;  // channels in groups of 4: one Philox block each
+    constexpr bool kGroups = WIDE && MODE < 3;
+    const int groups = kGroups ? (C + 3) >> 2 : 1;  // channels in groups of 4: one Philox block each
     // -m 3 / 4 / 5 (one summed majorant per cell): each batch's record and
     // majorant are read one batch ahead, so their latency overlaps the batch
     // before (records do not change during the round). 3 % faster there; the
     // same for the per-channel majorants of -m 0 / 1 / 2 measured 1 % slower.
-    constexpr bool kAhead = !WIDE && MODE >= 3;
+    constexpr bool kAhead = MODE >= 3;
     Record r_nx = {0u, 0.f, 0.f, 0u};
     float m_nx = 0.f;
     auto fetch_next = [&](const uint32_t i) {
@@ -600,7 +603,7 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
           }
         }
       };
-      if (WIDE) {
+      if (kGroups) {
         for (int g = 0; g < groups; ++g) enter_group(g);
       } else {
         enter_group(0);
@@ -697,8 +700,9 @@ __device__ __forceinline__ bool track_rays(const RenderParams& P, const Ctx<DT>&
 // view V): the camera ray tracked to its first event, shaded. The lane's
 // contribution to its pixel's sums is returned (composite_sample on empty
 // sums); h is the hit for the auxiliary buffers. WIDE: more than four channels
-// (-m 2), drawn in groups of four; a separate instantiation, since the group
-// loop's code in the four-channel kernel cost it 3%. LIT: gradient shading and
+// (shorter rounds, and -m 0 / 1 / 2 draw them in groups of four); a separate
+// instantiation, since the group loop's code in the four-channel kernel cost it
+// 3%. LIT: gradient shading and
 // shadow rays, as render_block (render_paths.hpp) does them: the shadow ray of
 // every lane that hit runs through the same tracking rounds
 // (deviceCode.cu:383-403), on stream 1.
