@@ -439,7 +439,7 @@ def main() -> int:
                 "measured_read_bytes": READ_STREAM_BYTES,
                 "measured_copy_gbps": round(copy_bw, 1),
                 "frac_of_measured": round(achieved / bw, 5) if bw > 0 else None,
-                "kernel": ((f"render_wave<{args.mode},{VOXEL_NAMES[str(scene.volumes[0].dtype)]}>")
+                "kernel": ((f"render_wave{'_team' if args.steps >= 4 else ''}<{args.mode},{VOXEL_NAMES[str(scene.volumes[0].dtype)]}>")
                            if args.schedule == 1 and args.mode <= 5 else
                            f"render_kernel<{args.mode},{VOXEL_NAMES[str(scene.volumes[0].dtype)]}>")}
     if traffic_src:
