@@ -36,7 +36,7 @@ COMMON = [
 ]
 
 SOURCES = ["kernels_build.hip", "kernels_render.hip", "kernels_batch.hip", "kernels_wave.hip",
-           "kernels_wave_lit.hip",
+           "kernels_wave_sum.hip", "kernels_wave_lit.hip", "kernels_wave_lit_sum.hip",
            "kernels_denoise.hip", "mdwt_api.cpp", "denoise_api.cpp",
            "host_copy.hip"]
 

@@ -2,7 +2,7 @@
 // pinned ring, with the host side of the copy spread over a few threads.
 //
 // The runtime copies pageable memory with one thread: 18 GB/s from the device
-// and 38 GB/s to it on the target boxes, where the link does 57 GB/s; a 16.8 MB
+// and 38 GB/s to it on an MI355X host whose link does 57 GB/s; a 16.8 MB
 // image took 960 us of an 8.2 ms render, and a denoiser inference of 0.6 ms of
 // kernels took 3 ms. Here each chunk's transfer overlaps the other chunks' host
 // copies.

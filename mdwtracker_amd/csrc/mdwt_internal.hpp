@@ -23,7 +23,10 @@ RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form
 bool several_frames_apply(const RenderParams& p, int mode, bool count);
 // the same of launch_views: the wave-coherent modes
 bool several_view_frames_apply(const RenderParams& p, int mode);
+// its parts: shaded -m 0 / 1 / 2, and -m 3 / 4 / 5 plain and shaded
 RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int form);
+RenderFn select_wave_sum_kernel(const RenderParams& p, int mode, int dtype, int form);
+RenderFn select_wave_lit_sum_kernel(const RenderParams& p, int mode, int dtype, int form);
 // dynamic LDS of a wave-coherent launch (transfer-function opacities)
 size_t wave_lds_bytes(const RenderParams& p);
 

@@ -1,5 +1,6 @@
 // Device code of wave-coherent Woodcock tracking, shared by the plain kernels
-// (kernels_wave.hip) and the lit ones (kernels_wave_lit.hip): the tracking
+// (kernels_wave.hip, kernels_wave_sum.hip) and the lit ones
+// (kernels_wave_lit.hip, kernels_wave_lit_sum.hip): the tracking
 // modes on up to twelve channels, -m 0 (N-DDA), -m 1 (one clock per channel), -m 2 (syncDDA), -m 3
 // (cumulative majorant) and -m 4 / 5 (blend tracking) (frame-kernel schedule 1).
 //
@@ -986,6 +987,31 @@ MDWT_WAVE_KERNEL void render_views_wave_persistent(RenderParams P) {
   }
 }
 #undef MDWT_WAVE_PROLOGUE
+
+// The kernel of a mode for launch form `form` (select_wave_kernel; the persistent
+// form has no shaded instance).
+template <int MODE, int DT, bool WIDE, bool LIT>
+RenderFn wave_fn_form(int form) {
+  if (form == 0) return render_wave<MODE, DT, WIDE, LIT>;
+  if (form == 1) return render_views_wave<MODE, DT, WIDE, LIT>;
+  if constexpr (!LIT)
+    if (form == 2) return render_views_wave_persistent<MODE, DT, WIDE>;
+  return render_wave_team<MODE, DT, WIDE, LIT>;
+}
+template <int MODE, bool WIDE, bool LIT>
+RenderFn wave_fn_dt(int dtype, int form) {
+  switch (dtype) {
+    case MDWT_DT_U8: return wave_fn_form<MODE, MDWT_DT_U8, WIDE, LIT>(form);
+    case MDWT_DT_U16: return wave_fn_form<MODE, MDWT_DT_U16, WIDE, LIT>(form);
+    case MDWT_DT_F16: return wave_fn_form<MODE, MDWT_DT_F16, WIDE, LIT>(form);
+    default: return wave_fn_form<MODE, MDWT_DT_F32, WIDE, LIT>(form);
+  }
+}
+template <int MODE, bool LIT>
+RenderFn wave_fn(const RenderParams& p, int dtype, int form) {
+  return p.vol.channels > 4 ? wave_fn_dt<MODE, true, LIT>(dtype, form)
+                            : wave_fn_dt<MODE, false, LIT>(dtype, form);
+}
 
 }  // namespace
 }  // namespace mdwt
