@@ -250,7 +250,10 @@ bool wave_persistent(const RenderParams& p, int mode) {
 }
 }  // namespace
 
-bool several_view_frames_apply(const RenderParams& p, int mode) { return wave_views(p, mode, false); }
+bool several_view_frames_apply(const RenderParams& p, int mode) {
+  return wave_views(p, mode, false) &&
+         grid_fits(uint64_t(p.fr.n_items) * unsigned(p.fr.bw * p.fr.bh / 64), kThreads);
+}
 
 hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int dtype, int* out) {
   const bool wave = wave_persistent(p, mode);
@@ -280,7 +283,7 @@ hipError_t launch_views_persistent(const RenderParams& p, int mode, int dtype, i
 hipError_t launch_views(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s) {
   if (p.fr.n_items <= 0) return hipSuccess;
   const bool wave = wave_views(p, mode, count), team = p.fr.team_frames > 0;
-  if (team && !wave) return hipErrorInvalidValue;
+  if (team && (count || !several_view_frames_apply(p, mode))) return hipErrorInvalidValue;
   const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
   const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, team ? 3 : 1)
                           : select_views(mode, dtype, count, is_lit(p), wide_views(p, dtype));

@@ -353,7 +353,7 @@ hipError_t prepare(RenderFn f, size_t lds) {
 // several frames per launch where a CU holds two such workgroups, the one-frame
 // kernels above that (their tables may fill the LDS).
 bool several_frames_apply(const RenderParams& p, int mode, bool count) {
-  if (count) return false;
+  if (count || !grid_fits(uint64_t(p.fr.n_blocks) * unsigned(p.fr.bw * p.fr.bh / 64), kThreads)) return false;
   if (mode < 6) return p.fr.schedule == 1 && wave_schedule_applies(p, mode, count);
   const size_t fixed = sizeof(ChanTf) * kMaxChannels + sizeof(FoldLds) * (kThreads / 64);
   return 2 * (render_lds_bytes(p) + fixed) <= size_t(160) << 10;

@@ -18,10 +18,15 @@ inline bool is_shaded(const RenderParams& p) { return p.fr.sh.shadows != 0 || p.
 // one view in one launch
 bool wave_schedule_applies(const RenderParams& p, int mode, bool count);
 RenderFn select_wave_kernel(const RenderParams& p, int mode, int dtype, int form);
+// whether HIP takes a launch of `blocks` workgroups of `threads` threads along x:
+// it supports fewer than 2^32 threads. The several-frame kernels have a
+// workgroup of 256 threads per 64 pixels, four times the one-frame kernels'
+// threads, and pass it at 2^30 pixels.
+inline bool grid_fits(uint64_t blocks, uint64_t threads) { return blocks * threads < (uint64_t(1) << 32); }
 // whether launch_render can render several frames (team_frames) in one launch:
-// the wave-coherent modes and the ray marchers
+// the wave-coherent modes and the ray marchers, where the grid fits
 bool several_frames_apply(const RenderParams& p, int mode, bool count);
-// the same of launch_views: the wave-coherent modes
+// the same of launch_views: the wave-coherent modes, where the grid fits
 bool several_view_frames_apply(const RenderParams& p, int mode);
 // its parts: shaded -m 0 / 1 / 2, and -m 3 / 4 / 5 plain and shaded
 RenderFn select_wave_lit_kernel(const RenderParams& p, int mode, int dtype, int form);

@@ -1,0 +1,64 @@
+"""Which launches the dispatch chooses at the limits of its arguments, checked
+on the host: a program linked against libmdwt.so asks the library's own rules."""
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+PKG = ROOT / "mdwtracker_amd"
+
+PROLOGUE = r"""
+#include <cstdio>
+#include <cstring>
+#include "mdwt_internal.hpp"
+using namespace mdwt;
+static int bad = 0;
+#define EXPECT(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); ++bad; } } while (0)
+static RenderParams params(int blocks, int items, int bw, int bh) {
+  RenderParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.vol.channels = 4;
+  p.tf.stride = 64;
+  for (int& m : p.mc) m = 8;
+  p.fr.schedule = 1;
+  p.fr.n_blocks = blocks;
+  p.fr.n_items = items;
+  p.fr.bw = bw;
+  p.fr.bh = bh;
+  return p;
+}
+"""
+
+
+def run(tmp_path, body):
+    if not (PKG / "libmdwt.so").exists():
+        pytest.skip("libmdwt.so is not built")
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    src.write_text(PROLOGUE + "int main() {\n" + body + '\n  if (!bad) std::printf("ok\\n");\n  return bad;\n}\n')
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                        f"-I{ROOT / 'include'}", f"-I{PKG / 'csrc'}", str(src), str(PKG / "libmdwt.so"),
+                        f"-Wl,-rpath,{PKG}", "-L/opt/rocm/lib", "-Wl,-rpath,/opt/rocm/lib", "-lamdhip64",
+                        "-o", str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout + r.stderr
+
+
+def test_several_frames_only_where_the_grid_fits(tmp_path):
+    """A workgroup of 256 threads per 8x8 pixels: HIP takes fewer than 2^32
+    threads, so frames of 2^30 pixels and batches of as many go frame by frame
+    (one thread per pixel), the next smaller ones several frames at a time."""
+    run(tmp_path, r"""
+  const struct { int bw, bh; } shapes[] = {{8, 8}, {16, 8}, {16, 16}};
+  for (const auto& s : shapes) {
+    const int q = s.bw * s.bh / 64, limit = (1 << 24) / q;  // blocks of 2^30 pixels
+    for (int mode = 0; mode < 10; ++mode) {
+      EXPECT(!several_frames_apply(params(limit, 0, s.bw, s.bh), mode, false));
+      EXPECT(several_frames_apply(params(limit - 1, 0, s.bw, s.bh), mode, false));
+      EXPECT(!several_frames_apply(params(1, 0, s.bw, s.bh), mode, true));  // the counting pass
+      EXPECT(!several_view_frames_apply(params(0, limit, s.bw, s.bh), mode));
+      EXPECT(!several_view_frames_apply(params(0, 2 * limit, s.bw, s.bh), mode));
+      EXPECT(several_view_frames_apply(params(0, limit - 1, s.bw, s.bh), mode) == (mode <= 5));
+    }
+  }""")
