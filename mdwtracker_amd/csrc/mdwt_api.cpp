@@ -626,17 +626,13 @@ mdwt::RenderParams render_params(const mdwt_renderer* h) {
 }
 
 // Frames of the next launch when `left` are to be rendered: several by the
-// team kernel (see team_quad in render_paths.hpp), whose four waves take four
-// draws (samples) at a time, or 0 for one frame by the one-frame kernels. Only
-// whole rounds of four draws: in a partial one, waves hold their workgroup's
-// LDS and do nothing. About 32 draws: longer launches gained under 1 %.
-constexpr int kTeamDraws = 32;
+// team kernel (see team_quad in render_paths.hpp), or 0 for one frame by the
+// one-frame kernels.
 int team_frames(const mdwt_renderer* h, const mdwt::RenderParams& p, int left) {
   if (!mdwt::several_frames_apply(p, h->mode, false)) return 0;
   // the auxiliary buffers stop at their own frame count
   if (p.fr.aov && h->aov_frames) left = std::min(left, int(uint32_t(h->aov_frames) - h->accum_id));
-  const int spp = p.fr.spp, step = spp % 4 == 0 ? 1 : (spp % 2 == 0 ? 2 : 4);
-  return std::min(left, std::max(step, kTeamDraws / spp)) / step * step;
+  return mdwt::frames_per_launch(left, p.fr.spp);
 }
 
 // One frame launch (the counting pass always runs the thread-per-pixel kernel),
@@ -1733,7 +1729,7 @@ int team_view_frames(const mdwt_renderer* h, const mdwt::RenderParams& p, int le
   if (!mdwt::several_view_frames_apply(p, h->mode)) return 0;
   int top = 1;
   for (const auto& s : h->spp_pixels) top = std::max(top, s.first);
-  for (int n = std::min(left, std::max(4, kTeamDraws / top)); n > 0; --n) {
+  for (int n = std::min(left, std::max(4, mdwt::kTeamDraws / top)); n > 0; --n) {
     double used = 0.0, slots = 0.0;
     for (const auto& s : h->spp_pixels) {
       const int draws = n * s.first;

@@ -26,6 +26,19 @@ inline bool grid_fits(uint64_t blocks, uint64_t threads) { return blocks * threa
 // whether launch_render can render several frames (team_frames) in one launch:
 // the wave-coherent modes and the ray marchers, where the grid fits
 bool several_frames_apply(const RenderParams& p, int mode, bool count);
+// Frames of a several-frame launch when `left` are to be rendered, or 0 for one
+// frame by the one-frame kernels. The team kernel's four waves take four draws
+// (samples) at a time: only whole rounds of four draws, since in a partial one
+// waves hold their workgroup's LDS and do nothing. About 32 draws: longer
+// launches gained under 1 %. The draws of a launch stay below 2^30 (the kernel
+// counts them in 32 bits).
+constexpr int kTeamDraws = 32;
+inline int frames_per_launch(int left, int spp) {
+  if (spp >= 1 << 28) return 0;
+  const int step = spp % 4 == 0 ? 1 : (spp % 2 == 0 ? 2 : 4), most = kTeamDraws / spp;
+  const int n = most > step ? most : step;
+  return (left < n ? left : n) / step * step;
+}
 // the same of launch_views: the wave-coherent modes, where the grid fits
 bool several_view_frames_apply(const RenderParams& p, int mode);
 // its parts: shaded -m 0 / 1 / 2, and -m 3 / 4 / 5 plain and shaded

@@ -62,3 +62,17 @@ def test_several_frames_only_where_the_grid_fits(tmp_path):
       EXPECT(several_view_frames_apply(params(0, limit - 1, s.bw, s.bh), mode) == (mode <= 5));
     }
   }""")
+
+
+def test_draws_of_a_launch_fit_32_bits(tmp_path):
+    """Any sample count: whole rounds of four draws, at least one round or about
+    32 draws, and never more draws than the kernels' 32-bit count holds."""
+    run(tmp_path, r"""
+  for (int64_t spp : {1ll, 2ll, 3ll, 4ll, 5ll, 6ll, 8ll, 31ll, 32ll, 33ll, 1000ll, (1ll << 28) - 1, 1ll << 28,
+                      (1ll << 29) + 1, (1ll << 30) - 2, (1ll << 30) + 1, (1ll << 31) - 4, (1ll << 31) - 1})
+    for (int left : {0, 1, 2, 3, 4, 5, 7, 32, 33, 100, 2147483647}) {
+      const int64_t n = frames_per_launch(left, int(spp));
+      EXPECT(n >= 0 && n <= left && n * spp % 4 == 0 && n * spp < (1ll << 31));
+      EXPECT(n * spp <= 32 || n <= 4);
+      if (left >= 4 && spp <= 1000) EXPECT(n > 0);
+    }""")
