@@ -49,14 +49,17 @@ class Lane {
   static std::unique_ptr<Lane> make(int device) {
     std::unique_ptr<Lane> l(new (std::nothrow) Lane(device));
     if (!l) return nullptr;
-    if (hipHostMalloc(reinterpret_cast<void**>(&l->ring_), kChunk * kSlots, hipHostMallocPortable) !=
-        hipSuccess) {
+    // Kernels and host threads take turns on a slot: coherent memory, so that
+    // each sees the other's writes whatever the runtime's default, and events that
+    // release to the system, since a host thread reads what lies before one.
+    if (hipHostMalloc(reinterpret_cast<void**>(&l->ring_), kChunk * kSlots,
+                      hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
       l->ring_ = nullptr;
       (void)hipGetLastError();
       return nullptr;
     }
     for (auto& e : l->ev_)
-      if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
         e = nullptr;
         (void)hipGetLastError();
         return nullptr;
