@@ -138,10 +138,15 @@ class Lane {
   // the transfer of chunk c and the event behind it; marks the slot as chunk c's
   void issue(size_t c) {
     const size_t k = c % kSlots;
-    uint8_t* slot = ring_ + k * kChunk;
-    hipLaunchKernelGGL(move_kernel, dim3(256), dim3(256), 0, stream_, to_host_ ? dev_ + c * kChunk : slot,
-                       to_host_ ? slot : dev_ + c * kChunk, uint32_t(size(c)));
-    hipError_t e = hipGetLastError();
+    uint8_t *slot = ring_ + k * kChunk, *dev = dev_ + c * kChunk;
+    const uint8_t* src = to_host_ ? dev : slot;
+    uint8_t* dst = to_host_ ? slot : dev;
+    uint32_t n = uint32_t(size(c));
+    void* args[] = {&src, &dst, &n};
+    // the launch's own status: hipGetLastError would give the error of any
+    // earlier call of this thread, and the copy would fail with it
+    hipError_t e = hipLaunchKernel(reinterpret_cast<const void*>(move_kernel), dim3(256), dim3(256), args, 0,
+                                   stream_);
     if (e == hipSuccess) e = hipEventRecord(ev_[k], stream_);
     if (e != hipSuccess) fail(e);
     used_[k] = true;

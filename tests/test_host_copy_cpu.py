@@ -247,3 +247,15 @@ def test_what_kernels_write_is_visible_to_the_host(run):
   EXPECT(fake::event_flags & hipEventReleaseToSystem);
   EXPECT(fake::event_flags & hipEventDisableTiming);
   host_copy_release();""")
+
+
+def test_an_earlier_error_of_the_thread_is_not_the_copys(run):
+    """An error that an earlier call of the calling thread left behind (the
+    runtime keeps it until it is asked for)."""
+    run(r"""
+  host_copy_acquire();
+  fake::Stream s;
+  fake::last = hipErrorOutOfMemory;
+  round_trip(kRing + 1, 1, 0, &s);
+  EXPECT(hipGetLastError() == hipErrorOutOfMemory);
+  host_copy_release();""")
