@@ -1,6 +1,6 @@
 // See host_copy.hpp. A lane is a pinned ring of kSlots chunks, an event per slot
 // and kWorkers threads; a call takes a free lane of its device (or makes one, up
-// to kMaxLanes; past that, or where pinned memory is not to be had, it copies
+// to kMaxLanes per device; past that, or where pinned memory is not to be had, it copies
 // as the runtime does), so calls of several threads, handles and streams run
 // side by side and share nothing but the list of free lanes.
 #include "host_copy.hpp"
@@ -28,7 +28,7 @@ constexpr size_t kChunk = size_t(2) << 20;
 constexpr int kSlots = 8;                     // 16 MiB per lane
 constexpr size_t kPiece = size_t(256) << 10;  // bytes a thread copies at a time
 constexpr int kWorkers = 3;                   // beside the calling thread
-constexpr size_t kMaxLanes = 4;
+constexpr size_t kMaxLanes = 4;               // per device
 // below this, waking the workers costs more than they save
 constexpr size_t kMinBytes = size_t(512) << 10;
 
@@ -79,6 +79,8 @@ class Lane {
     }
     cv_.notify_all();
     for (auto& t : threads_) t.join();
+    int current = device_;
+    (void)hipGetDevice(&current);
     (void)hipSetDevice(device_);
     for (auto& e : ev_)
       if (e) {
@@ -86,6 +88,7 @@ class Lane {
         (void)hipEventDestroy(e);
       }
     if (ring_) (void)hipHostFree(ring_);
+    (void)hipSetDevice(current);
   }
   int device() const { return device_; }
 
@@ -233,7 +236,7 @@ class Lane {
 struct Pool {
   std::mutex mu;
   int handles = 0;
-  size_t lanes = 0;  // made, free or in use
+  std::vector<size_t> lanes;  // by device: made, free or in use
   std::vector<std::unique_ptr<Lane>> free;
 };
 Pool& pool() {
@@ -252,23 +255,29 @@ std::unique_ptr<Lane> take(int device) {
         p.free.pop_back();
         return got;
       }
-    if (p.lanes >= kMaxLanes) return nullptr;
-    ++p.lanes;
+    try {
+      if (p.lanes.size() <= size_t(device)) p.lanes.resize(size_t(device) + 1, 0);
+    } catch (const std::bad_alloc&) {
+      return nullptr;
+    }
+    if (p.lanes[size_t(device)] >= kMaxLanes) return nullptr;
+    ++p.lanes[size_t(device)];
   }
   std::unique_ptr<Lane> l = Lane::make(device);
   if (!l) {
     std::lock_guard<std::mutex> lock(p.mu);
-    --p.lanes;
+    --p.lanes[size_t(device)];
   }
   return l;
 }
 void give(std::unique_ptr<Lane> l) {
   Pool& p = pool();
   std::lock_guard<std::mutex> lock(p.mu);
+  const size_t device = size_t(l->device());
   try {
     p.free.push_back(std::move(l));
   } catch (const std::bad_alloc&) {
-    --p.lanes;
+    --p.lanes[device];
   }
 }
 
@@ -302,7 +311,7 @@ void host_copy_release() {
     std::lock_guard<std::mutex> lock(p.mu);
     if (--p.handles > 0) return;
     gone.swap(p.free);
-    p.lanes -= gone.size();
+    for (const auto& l : gone) --p.lanes[size_t(l->device())];
   }
 }
 

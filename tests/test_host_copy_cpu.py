@@ -85,6 +85,7 @@ typedef fake::Stream* hipStream_t;
 typedef fake::Event* hipEvent_t;
 inline hipError_t hipGetLastError() { hipError_t e = fake::last; fake::last = hipSuccess; return e; }
 inline hipError_t hipSetDevice(int d) { fake::device = d; return hipSuccess; }
+inline hipError_t hipGetDevice(int* d) { *d = fake::device; return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
   std::lock_guard<std::mutex> l(fake::mu);
   fake::host_flags = flags;
@@ -259,3 +260,24 @@ def test_an_earlier_error_of_the_thread_is_not_the_copys(run):
   round_trip(kRing + 1, 1, 0, &s);
   EXPECT(hipGetLastError() == hipErrorOutOfMemory);
   host_copy_release();""")
+
+
+def test_every_device_gets_rings(run):
+    """One thread that goes over several devices, twice: each keeps a ring of its
+    own, however many others there are, and the current device stays."""
+    run(r"""
+  host_copy_acquire();
+  fake::Stream s;
+  for (int round = 0; round < 2; ++round)
+    for (int d = 0; d < 7; ++d) {
+      hipSetDevice(d);
+      const int before = fake::launches[d];
+      round_trip(kRing, 1, d, &s);
+      EXPECT(fake::launches[d] == before + 2 * kSlots && fake::copies[d] == 0);
+      EXPECT(fake::rings[d] == 1);
+      EXPECT(fake::device == d);
+    }
+  hipSetDevice(3);
+  host_copy_release();
+  EXPECT(fake::device == 3);
+  for (const auto& r : fake::rings) EXPECT(r.second == 0);""")
