@@ -1,9 +1,11 @@
 // See host_copy.hpp. A lane is a pinned ring of kSlots chunks, an event per slot
-// and kWorkers threads; a call takes a free lane of its device (or makes one, up
+// and up to kWorkers threads; a call takes a free lane of its device (or makes one, up
 // to kMaxLanes per device; past that, or where pinned memory is not to be had, it copies
 // as the runtime does), so calls of several threads, handles and streams run
 // side by side and share nothing but the list of free lanes.
 #include "host_copy.hpp"
+
+#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
@@ -27,7 +29,7 @@ namespace {
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr int kSlots = 8;                     // 16 MiB per lane
 constexpr size_t kPiece = size_t(256) << 10;  // bytes a thread copies at a time
-constexpr int kWorkers = 3;                   // beside the calling thread
+constexpr int kWorkers = 3;                   // beside the calling thread, at most
 constexpr size_t kMaxLanes = 4;               // per device
 // below this, waking the workers costs more than they save
 constexpr size_t kMinBytes = size_t(512) << 10;
@@ -64,8 +66,13 @@ class Lane {
         (void)hipGetLastError();
         return nullptr;
       }
+    // a thread per core that this process may use: with fewer cores than threads
+    // the copies would take them from each other while they wait for transfers
+    cpu_set_t cores;
+    const int n = sched_getaffinity(0, sizeof(cores), &cores) == 0 ? CPU_COUNT(&cores) : kWorkers + 1;
+    const int workers = std::min(kWorkers, n - 1);
     try {
-      for (int i = 0; i < kWorkers; ++i) l->threads_.emplace_back([p = l.get()] { p->worker(); });
+      for (int i = 0; i < workers; ++i) l->threads_.emplace_back([p = l.get()] { p->worker(); });
     } catch (const std::system_error&) {
       // fewer workers: the calling thread does the rest
     } catch (const std::bad_alloc&) {

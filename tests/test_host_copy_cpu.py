@@ -2,6 +2,7 @@
 small stand-in of the HIP runtime (streams as threads, events as marks on them,
 the copy kernel run as written), so that what it asks of the runtime and the order
 of its transfers can be checked without a GPU."""
+import os
 import subprocess
 from pathlib import Path
 
@@ -281,3 +282,23 @@ def test_every_device_gets_rings(run):
   host_copy_release();
   EXPECT(fake::device == 3);
   for (const auto& r : fake::rings) EXPECT(r.second == 0);""")
+
+
+@pytest.mark.parametrize("cores", [1, 2, 3, 4, 6])
+def test_no_more_threads_than_cores(run, cores):
+    """The calling thread and its helpers, on a process of few cores."""
+    if len(os.sched_getaffinity(0)) < cores:
+        pytest.skip("fewer cores here")
+    run(r"""
+  cpu_set_t all, some;
+  sched_getaffinity(0, sizeof(all), &all);
+  CPU_ZERO(&some);
+  for (int i = 0, n = 0; i < CPU_SETSIZE && n < %d; ++i)
+    if (CPU_ISSET(i, &all)) CPU_SET(i, &some), ++n;
+  sched_setaffinity(0, sizeof(some), &some);
+  host_copy_acquire();
+  fake::Stream s;
+  round_trip(kRing + 100, 1, 0, &s);
+  EXPECT(threads_now() == 1 + 1 + std::min(3, %d - 1));  // main, the stream, the helpers
+  host_copy_release();
+  EXPECT(threads_now() == 2);""" % (cores, cores))
