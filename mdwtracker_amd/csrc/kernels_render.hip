@@ -427,9 +427,11 @@ hipError_t launch_rgba8(const void* accum, uint32_t* out, int n, hipStream_t s) 
 }
 
 hipError_t launch_pack_aov(const float* aov, int row, int nv, size_t n, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(pack_aov_kernel, dim3(unsigned((n * size_t(nv) + 255) / 256)), dim3(256), 0, s, aov,
-                     row, nv, n, out);
-  return hipGetLastError();
+  if (n == 0 || n > pack_aov_pixels(nv)) return hipErrorInvalidValue;
+  void* args[] = {&aov, &row, &nv, &n, &out};
+  // (the launch's own status: a read-back does not fail with the thread's last error)
+  return hipLaunchKernel(reinterpret_cast<const void*>(pack_aov_kernel), dim3(unsigned((n * size_t(nv) + 255) / 256)),
+                         dim3(256), args, 0, s);
 }
 
 hipError_t launch_read(const void* src, size_t n16, float* sums, hipStream_t s) {

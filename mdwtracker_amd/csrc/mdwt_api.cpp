@@ -387,17 +387,20 @@ void free_frame(mdwt_renderer* h) {
 }
 
 // Device scratch of at least `bytes` for a read-back's conversion, kept until
-// the frame size changes.
-int read_scratch(mdwt_renderer* h, size_t bytes, void** out) {
+// the frame size changes; nullptr where the memory is not there (a smaller one
+// stays).
+void* read_scratch(mdwt_renderer* h, size_t bytes) {
   if (bytes > h->read_bytes) {
+    void* d = nullptr;
+    if (hipMalloc(&d, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
     if (h->d_read) (void)hipFree(h->d_read);
-    h->d_read = nullptr;
-    h->read_bytes = 0;
-    HIPCHK(h, hipMalloc(&h->d_read, bytes));
+    h->d_read = d;
     h->read_bytes = bytes;
   }
-  *out = h->d_read;
-  return MDWT_OK;
+  return h->d_read;
 }
 
 // Block order of one image (nbx x nby blocks of bw x bh pixels): row-major,
@@ -441,8 +444,7 @@ int alloc_frame(mdwt_renderer* h) {
   }
   h->fb_pixels = n;
   // the RGBA8 frame buffer
-  void* fb = nullptr;
-  if (const int rc = read_scratch(h, n * sizeof(uint32_t), &fb)) return rc;
+  if (!read_scratch(h, n * sizeof(uint32_t))) return fail(h, MDWT_ERR_HIP, "device memory of the frame buffer");
   if (h->aov_on) {
     const size_t na = size_t(mdwt::aov_groups(h->C)) * n;
     HIPCHK(h, hipMalloc(&h->d_aov, na * sizeof(Float4)));
@@ -1148,9 +1150,8 @@ int mdwt_read_fb(mdwt_renderer* h, uint32_t* rgba8) {
   if (!h->inited) return fail(h, MDWT_ERR_STATE, "renderer not initialized");
   if (!rgba8) return fail(h, MDWT_ERR_ARG, "null output");
   HIPCHK(h, hipSetDevice(h->device));
-  void* d = nullptr;
-  const int rc = read_scratch(h, h->fb_pixels * sizeof(uint32_t), &d);
-  if (rc != MDWT_OK) return rc;
+  void* d = read_scratch(h, h->fb_pixels * sizeof(uint32_t));
+  if (!d) return fail(h, MDWT_ERR_HIP, "read_fb: no device memory for the RGBA8 image");
   HIPCHK(h, mdwt::launch_rgba8(h->d_accum, static_cast<uint32_t*>(d), int(h->fb_pixels), h->stream));
   HIPCHK(h, mdwt::copy_to_host(rgba8, d, h->fb_pixels * sizeof(uint32_t), h->device, h->stream));
   return MDWT_OK;
@@ -2170,17 +2171,29 @@ int mdwt_read_aov(mdwt_renderer* h, float* out) {
   if (!h->aov_on || !h->d_aov) return fail(h, MDWT_ERR_STATE, "auxiliary buffers are off");
   HIPCHK(h, hipSetDevice(h->device));
   const int row = 4 * mdwt::aov_groups(h->C), nv = 2 + h->C;
-  const size_t bytes = h->fb_pixels * size_t(nv) * sizeof(float);
-  const void* src = h->d_aov;
-  if (row != nv) {  // the padding is dropped on the device
-    void* d = nullptr;
-    const int rc = read_scratch(h, bytes, &d);
-    if (rc != MDWT_OK) return rc;
-    HIPCHK(h, mdwt::launch_pack_aov(reinterpret_cast<const float*>(h->d_aov), row, nv, h->fb_pixels,
-                                    static_cast<float*>(d), h->stream));
-    src = d;
+  const float* src = reinterpret_cast<const float*>(h->d_aov);
+  if (row == nv) {
+    HIPCHK(h, mdwt::copy_to_host(out, src, h->fb_pixels * size_t(nv) * sizeof(float), h->device, h->stream));
+    return MDWT_OK;
   }
-  HIPCHK(h, mdwt::copy_to_host(out, src, bytes, h->device, h->stream));
+  // the padding is dropped on the device, a piece of the image at a time; by the
+  // host where there is no memory for a piece
+  const size_t most = mdwt::pack_aov_pixels(nv);
+  float* d = static_cast<float*>(read_scratch(h, std::min(h->fb_pixels, most) * size_t(nv) * sizeof(float)));
+  std::vector<float> rows(d ? 0 : std::min(h->fb_pixels, most) * size_t(row));
+  for (size_t at = 0; at < h->fb_pixels; at += most) {
+    const size_t n = std::min(most, h->fb_pixels - at);
+    float* to = out + at * size_t(nv);
+    if (d) {
+      HIPCHK(h, mdwt::launch_pack_aov(src + at * size_t(row), row, nv, n, d, h->stream));
+      HIPCHK(h, mdwt::copy_to_host(to, d, n * size_t(nv) * sizeof(float), h->device, h->stream));
+    } else {
+      HIPCHK(h, mdwt::copy_to_host(rows.data(), src + at * size_t(row), n * size_t(row) * sizeof(float), h->device,
+                                   h->stream));
+      for (size_t p = 0; p < n; ++p)
+        std::memcpy(to + size_t(nv) * p, rows.data() + size_t(row) * p, size_t(nv) * sizeof(float));
+    }
+  }
   return MDWT_OK;
 }
 

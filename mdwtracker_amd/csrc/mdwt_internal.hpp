@@ -54,7 +54,10 @@ hipError_t launch_majorants(const MajorantParams& p, hipStream_t s);
 // (the block at position b); tmp: nb entries
 hipError_t launch_cost_order(uint32_t* order, const uint32_t* ticks, uint32_t* tmp, int nb, int wpb,
                              hipStream_t s);
-// out[p][0 .. nv) = aov[p][0 .. nv) of rows of `row` floats, n pixels
+// out[p][0 .. nv) = aov[p][0 .. nv) of rows of `row` floats, n pixels: at most
+// pack_aov_pixels(nv), 64 MiB of output (a thread per value stays far below the
+// threads that HIP takes, and the scratch small beside the image)
+inline size_t pack_aov_pixels(int nv) { return (size_t(64) << 20) / (size_t(nv) * sizeof(float)); }
 hipError_t launch_pack_aov(const float* aov, int row, int nv, size_t n, float* out, hipStream_t s);
 // v.bricks (brick_stride bytes per channel) = v.vol in 4 x 4 x 4 bricks
 hipError_t launch_bricks(const VolumeParams& v, int dtype, hipStream_t s);

@@ -66,3 +66,24 @@ def test_batch_of_2_30_pixels(capi, launch):
         assert want[..., :3].std() > 0.01
         np.testing.assert_array_equal(g.batch_read_view(i).view(np.uint32), want.view(np.uint32))
     g.close()
+
+
+@pytest.mark.parametrize("channels,size", [(1, (2365, 2365)), (5, (1549, 1547)), (12, (1095, 1095)), (12, (1094, 1095))])
+def test_auxiliary_buffers_of_more_than_a_piece(capi, channels, size):
+    """Around the 64 MiB piece of the packed read-back, with the buffers' rows
+    padded: a pixel misses exactly where the image shows the background."""
+    print(f"[limits] aov {channels} channels {size}", flush=True)
+    bg = (0.3137, 0.41, 0.77)
+    r = _renderer(capi, mode=2, channels=channels)
+    r.set_aov(True)
+    r.set_frame(size[0], size[1], 1, True, bg)
+    r.set_camera((0.5, 0.5, 0.05), (0.5, 0.5, 1.0), (0.0, 1.0, 0.0), 60.0)  # inside: every ray is in the volume
+    r.render(1)
+    img, aov = r.read_accum(), r.read_aov()
+    r.close()
+    miss = (img[..., :3] == np.float32(bg)).all(-1)
+    assert 0.0 < miss.mean() < 1.0 and not miss[-1].all()
+    np.testing.assert_array_equal(aov[..., 1], miss.astype(np.float32))
+    np.testing.assert_array_equal(aov[..., 1:].sum(-1), np.ones(miss.shape, np.float32))
+    # the first free flight may have no length: a hit at 0, with odds of about 1e-7 a step
+    assert (aov[..., 0][miss] == 0).all() and (aov[..., 0][~miss] > 0).mean() > 0.9999

@@ -76,3 +76,16 @@ def test_draws_of_a_launch_fit_32_bits(tmp_path):
       EXPECT(n * spp <= 32 || n <= 4);
       if (left >= 4 && spp <= 1000) EXPECT(n > 0);
     }""")
+
+
+def test_auxiliary_buffers_are_packed_in_pieces_that_fit(tmp_path):
+    """A thread per value of a piece, for every channel count; the launcher takes
+    no larger piece (a frame of 2^30 pixels has up to 14 values each)."""
+    run(tmp_path, r"""
+  for (int c = 1; c <= kMaxChannels; ++c) {
+    const size_t n = pack_aov_pixels(2 + c);
+    EXPECT(n > 0 && grid_fits((n * (2 + c) + 255) / 256, 256));
+    const int row = 4 * aov_groups(c);
+    EXPECT(launch_pack_aov(nullptr, row, 2 + c, n + 1, nullptr, nullptr) == hipErrorInvalidValue);
+    EXPECT(launch_pack_aov(nullptr, row, 2 + c, size_t(1) << 30, nullptr, nullptr) == hipErrorInvalidValue);
+  }""")
