@@ -443,8 +443,6 @@ int alloc_frame(mdwt_renderer* h) {
     HIPCHK(h, hipMemsetAsync(h->d_m2, 0, n * sizeof(Float4), h->stream));
   }
   h->fb_pixels = n;
-  // the RGBA8 frame buffer
-  if (!read_scratch(h, n * sizeof(uint32_t))) return fail(h, MDWT_ERR_HIP, "device memory of the frame buffer");
   if (h->aov_on) {
     const size_t na = size_t(mdwt::aov_groups(h->C)) * n;
     HIPCHK(h, hipMalloc(&h->d_aov, na * sizeof(Float4)));
@@ -459,6 +457,9 @@ int alloc_frame(mdwt_renderer* h) {
                            hipMemcpyHostToDevice, h->stream));
   HIPCHK(h, hipMalloc(&h->d_order_tmp, order.size() * sizeof(uint32_t)));
   HIPCHK(h, hipMalloc(&h->d_wave_cost, 4 * order.size() * sizeof(uint32_t)));
+  // the RGBA8 frame buffer; where there is no memory for it now, mdwt_read_fb
+  // asks again
+  (void)read_scratch(h, n * sizeof(uint32_t));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->cost_ready = false;
   h->need_resort = true;

@@ -1,0 +1,98 @@
+"""Device memory that is short: what a handle keeps for speed alone makes room.
+Most of the card is taken by one allocation of the test's own, freed after it."""
+import ctypes
+from contextlib import contextmanager
+
+import numpy as np
+import pytest
+
+from mdwtracker_amd import scenes
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def capi():
+    from mdwtracker_amd import capi
+    return capi
+
+
+@pytest.fixture(scope="module")
+def hip(capi):
+    return ctypes.CDLL("libamdhip64.so.7")  # the runtime that libmdwt.so has loaded
+
+
+def _memory(hip):
+    """(free, total) bytes of the device"""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value, total.value
+
+
+def _take(hip, left):
+    """Allocations that leave `left` bytes of the device free (in a few steps: the
+    runtime counts more as free at first than it has)."""
+    taken = []
+    for _ in range(4):
+        n = _memory(hip)[0] - left
+        if n < 8 * MIB:
+            break
+        p = ctypes.c_void_p()
+        assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(n)) == 0
+        taken.append(p)
+    return taken
+
+
+@pytest.fixture(scope="module", autouse=True)
+def most_of_the_card(hip):
+    taken = _take(hip, 48 << 30)
+    yield
+    for p in taken:
+        assert hip.hipFree(p) == 0
+
+
+@contextmanager
+def _only(hip, left):
+    taken = _take(hip, left)
+    try:
+        print(f"[memory] free {_memory(hip)[0] >> 20} MiB", flush=True)
+        assert abs(_memory(hip)[0] - left) < 16 * MIB
+        yield
+    finally:
+        for p in taken:
+            assert hip.hipFree(p) == 0
+
+
+def _renderer(capi, mode, dims=(64, 48, 40), size=(96, 64)):
+    """Two u8 channels of `dims` voxels: their joint copy has 4 bytes a voxel."""
+    rng = np.random.default_rng(9)
+    r = capi.MdwtRenderer(0)
+    for _ in range(2):
+        block = scenes.blob_volume_u8(16, 5, rng)
+        reps = [-(-n // 16) for n in dims[::-1]]
+        r.push_channel(np.ascontiguousarray(np.tile(block, reps)[:dims[2], :dims[1], :dims[0]]))
+    r.init(mode, (8, 8, 8), True)
+    for c in range(2):
+        r.set_tf(c, scenes.piecewise_tf(6, rng, 0.3 * c, clear_first=True), 0.2, (0.0, 1.0))
+    r.set_frame(size[0], size[1], 1, True, (0.2, 0.4, 0.6))
+    r.set_seed(5)
+    r.render(1)  # what the runtime allocates at a first launch is there
+    r.reset_accumulation()
+    return r
+
+
+def test_frame_without_room_for_its_8_bit_image(capi, hip):
+    """A frame whose accumulator fits beside nothing else: rendered and read as
+    floats; the 8-bit image is refused, and read once there is memory."""
+    r = _renderer(capi, 2)
+    with _only(hip, 1024 * MIB + 128 * MIB):
+        r.set_frame(8192, 8192, 1, True, (0.2, 0.4, 0.6))  # 1 GiB, and 256 MiB as RGBA8
+        r.render(1)
+        a = r.read_accum()
+        with pytest.raises(Exception, match="RGBA8"):
+            r.read_fb()
+    v = np.clip(np.trunc(np.clip(a * np.float32(256), -1, 256)), 0, 255).astype(np.uint32)
+    np.testing.assert_array_equal(v[..., 0] | (v[..., 1] << 8) | (v[..., 2] << 16) | (v[..., 3] << 24), r.read_fb())
+    r.close()
