@@ -76,7 +76,9 @@ struct mdwt_denoiser {
 
 namespace {
 
+// (as the renderer's: an error of the runtime is reported once)
 int fail(mdwt_denoiser* d, int code, const std::string& m) {
+  if (code == MDWT_ERR_HIP || code == MDWT_ERR_OOM) (void)hipGetLastError();
   d->err = m;
   return code;
 }

@@ -189,7 +189,10 @@ namespace {
 void free_batch(mdwt_renderer* h);
 int reorder(mdwt_renderer* h);
 
+// An error of the runtime is reported once: it keeps the last one of a thread
+// until asked, and the next launch would fail with it.
 int fail(mdwt_renderer* h, int code, const std::string& msg) {
+  if (code == MDWT_ERR_HIP || code == MDWT_ERR_OOM) (void)hipGetLastError();
   h->err = msg;
   return code;
 }
@@ -641,6 +644,8 @@ int team_frames(const mdwt_renderer* h, const mdwt::RenderParams& p, int left) {
 // One frame launch (the counting pass always runs the thread-per-pixel kernel),
 // or of several (*frames, at most `left`) by the team kernel.
 int launch_frame(mdwt_renderer* h, bool count, int left = 1, int* frames = nullptr) {
+  if (!h->d_accum || !h->d_order || !h->d_wave_cost)
+    return fail(h, MDWT_ERR_STATE, "no frame buffers (the last allocation of a frame failed)");
   mdwt::RenderParams p = render_params(h);
   if (count) p.fr.wave_cost = nullptr;
   p.fr.team_frames = count ? 0 : team_frames(h, p, left);

@@ -96,3 +96,20 @@ def test_frame_without_room_for_its_8_bit_image(capi, hip):
     v = np.clip(np.trunc(np.clip(a * np.float32(256), -1, 256)), 0, 255).astype(np.uint32)
     np.testing.assert_array_equal(v[..., 0] | (v[..., 1] << 8) | (v[..., 2] << 16) | (v[..., 3] << 24), r.read_fb())
     r.close()
+
+
+def test_a_frame_that_was_not_allocated_is_an_error(capi, hip):
+    """A frame that does not fit is refused, and so is rendering until one does."""
+    r = _renderer(capi, 2)
+    r.render(1)
+    want = r.read_accum()
+    with _only(hip, 512 * MIB):
+        with pytest.raises(Exception):
+            r.set_frame(8192, 8192, 1, True, (0.2, 0.4, 0.6))
+        for _ in range(2):
+            with pytest.raises(Exception):
+                r.render(1)
+    r.set_frame(96, 64, 1, True, (0.2, 0.4, 0.6))
+    r.render(1)
+    assert r.read_accum().shape == want.shape
+    r.close()
