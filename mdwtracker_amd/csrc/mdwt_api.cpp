@@ -212,6 +212,25 @@ void reset_acc(mdwt_renderer* h) {
       return fail((h), MDWT_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+// The joint copy of the volume given back; the kernels read the channels' own
+// bricks without it (the same images, slower).
+void release_joint(mdwt_renderer* h) {
+  if (!h->d_joint) return;
+  if (h->stream) (void)hipStreamSynchronize(h->stream);
+  (void)hipFree(h->d_joint);
+  h->d_joint = nullptr;
+}
+
+// Device memory of the handle; where it is short, the joint copy makes room.
+template <class T>
+hipError_t device_alloc(mdwt_renderer* h, T** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !h->d_joint) return e;
+  (void)hipGetLastError();
+  release_joint(h);
+  return hipMalloc(p, bytes);
+}
+
 size_t bytes_per_voxel(int dt) { return dt == MDWT_U8 ? 1 : (dt == MDWT_F32 ? 4 : 2); }
 
 float half_to_float(uint16_t h) {
@@ -395,7 +414,7 @@ void free_frame(mdwt_renderer* h) {
 void* read_scratch(mdwt_renderer* h, size_t bytes) {
   if (bytes > h->read_bytes) {
     void* d = nullptr;
-    if (hipMalloc(&d, bytes) != hipSuccess) {
+    if (device_alloc(h, &d, bytes) != hipSuccess) {
       (void)hipGetLastError();
       return nullptr;
     }
@@ -439,27 +458,27 @@ std::vector<uint32_t> block_order(int nbx, int nby, int bw, int bh, int tile, bo
 int alloc_frame(mdwt_renderer* h) {
   free_frame(h);
   const size_t n = size_t(h->W) * h->H;
-  HIPCHK(h, hipMalloc(&h->d_accum, n * sizeof(Float4)));
+  HIPCHK(h, device_alloc(h, &h->d_accum, n * sizeof(Float4)));
   HIPCHK(h, hipMemsetAsync(h->d_accum, 0, n * sizeof(Float4), h->stream));
   if (h->moments) {
-    HIPCHK(h, hipMalloc(&h->d_m2, n * sizeof(Float4)));
+    HIPCHK(h, device_alloc(h, &h->d_m2, n * sizeof(Float4)));
     HIPCHK(h, hipMemsetAsync(h->d_m2, 0, n * sizeof(Float4), h->stream));
   }
   h->fb_pixels = n;
   if (h->aov_on) {
     const size_t na = size_t(mdwt::aov_groups(h->C)) * n;
-    HIPCHK(h, hipMalloc(&h->d_aov, na * sizeof(Float4)));
+    HIPCHK(h, device_alloc(h, &h->d_aov, na * sizeof(Float4)));
     HIPCHK(h, hipMemsetAsync(h->d_aov, 0, na * sizeof(Float4), h->stream));
   }
   const int bw = h->bw, bh = h->bh;
   const int nbx = (h->W + bw - 1) / bw, nby = (h->H + bh - 1) / bh;
   std::vector<uint32_t> order = block_order(nbx, nby, bw, bh, h->tile, h->order_mode >= 1);
   h->n_blocks = int(order.size());
-  HIPCHK(h, hipMalloc(&h->d_order, order.size() * sizeof(uint32_t)));
+  HIPCHK(h, device_alloc(h, &h->d_order, order.size() * sizeof(uint32_t)));
   HIPCHK(h, hipMemcpyAsync(h->d_order, order.data(), order.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipMalloc(&h->d_order_tmp, order.size() * sizeof(uint32_t)));
-  HIPCHK(h, hipMalloc(&h->d_wave_cost, 4 * order.size() * sizeof(uint32_t)));
+  HIPCHK(h, device_alloc(h, &h->d_order_tmp, order.size() * sizeof(uint32_t)));
+  HIPCHK(h, device_alloc(h, &h->d_wave_cost, 4 * order.size() * sizeof(uint32_t)));
   // the RGBA8 frame buffer; where there is no memory for it now, mdwt_read_fb
   // asks again
   (void)read_scratch(h, n * sizeof(uint32_t));
@@ -504,7 +523,7 @@ int rebuild_majorants(mdwt_renderer* h) {
   if (texels > h->d_tf_texels) {
     if (h->d_tf) (void)hipFree(h->d_tf);
     h->d_tf = nullptr;
-    HIPCHK(h, hipMalloc(&h->d_tf, texels * sizeof(Float4)));
+    HIPCHK(h, device_alloc(h, &h->d_tf, texels * sizeof(Float4)));
     h->d_tf_texels = texels;
   }
   h->tf_stride = stride;
@@ -566,21 +585,34 @@ int make_bricks(mdwt_renderer* h) {
   return MDWT_OK;
 }
 
-// Make the joint copy for -m 3 to -m 8 (which read every channel at a
-// position) on two channels or more. Where the memory for it is not there, the
-// kernels read the channels' own bricks.
-int make_joint(mdwt_renderer* h) {
-  if (h->joint_tried || h->mode < 3 || h->mode > 8 || h->C < 2) return MDWT_OK;
+// The joint copy for -m 3 to -m 8 (which read every channel at a position) on
+// two channels or more: made when the mode first needs it, given back when the
+// mode leaves them. It is as large as the bricks (two channels: twice) and
+// optional, so an eighth of the device's memory is left for what is allocated
+// later: this handle's frames and views, which take the copy back where they
+// fall short (device_alloc), and other handles and libraries, which cannot.
+int fit_joint(mdwt_renderer* h) {
+  if (h->mode < 3 || h->mode > 8 || h->C < 2) {
+    release_joint(h);
+    h->joint_tried = false;
+    return MDWT_OK;
+  }
+  if (h->joint_tried) return MDWT_OK;
   h->joint_tried = true;
   const size_t per = size_t((h->dims[0] + 3) / 4) * size_t((h->dims[1] + 3) / 4) *
                      size_t((h->dims[2] + 3) / 4) * 64u * 4u * bytes_per_voxel(h->dtype);
   h->joint_stride = (per + 255) & ~size_t(255);
-  if (hipMalloc(&h->d_joint, h->joint_stride * size_t((h->C + 3) / 4)) != hipSuccess) {
+  const size_t bytes = h->joint_stride * size_t((h->C + 3) / 4);
+  size_t left = 0, total = 0;
+  if (hipMemGetInfo(&left, &total) != hipSuccess || left < bytes + total / 8 ||
+      hipMalloc(&h->d_joint, bytes) != hipSuccess) {
     (void)hipGetLastError();
     h->d_joint = nullptr;
     return MDWT_OK;
   }
-  HIPCHK(h, mdwt::launch_joint(volume_params(h), h->dtype, h->stream));
+  const hipError_t e = mdwt::launch_joint(volume_params(h), h->dtype, h->stream);
+  if (e != hipSuccess) release_joint(h);
+  HIPCHK(h, e);
   return MDWT_OK;
 }
 
@@ -670,11 +702,11 @@ int build_range_grid(mdwt_renderer* h, const std::vector<int>& wx, const std::ve
   win.insert(win.end(), wx.begin(), wx.end());
   win.insert(win.end(), wy.begin(), wy.end());
   win.insert(win.end(), wz.begin(), wz.end());
-  HIPCHK(h, hipMalloc(&h->d_win, win.size() * sizeof(int)));
+  HIPCHK(h, device_alloc(h, &h->d_win, win.size() * sizeof(int)));
   HIPCHK(h, hipMemcpyAsync(h->d_win, win.data(), win.size() * sizeof(int), hipMemcpyHostToDevice,
                            h->stream));
-  HIPCHK(h, hipMalloc(&h->d_ranges, n_cells * h->C * 2 * sizeof(float)));
-  HIPCHK(h, hipMalloc(&h->d_maj, n_cells * h->C * sizeof(float)));
+  HIPCHK(h, device_alloc(h, &h->d_ranges, n_cells * h->C * 2 * sizeof(float)));
+  HIPCHK(h, device_alloc(h, &h->d_maj, n_cells * h->C * sizeof(float)));
   HIPCHK(h, hipMemsetAsync(h->d_maj, 0, n_cells * h->C * sizeof(float), h->stream));
   mdwt::RangeParams rp{};
   rp.vol = h->d_vol;
@@ -881,8 +913,8 @@ int mdwt_init(mdwt_renderer* h, int mode, const int mc[3], int auto_camera) {
                                    h->device, h->stream));
   int rc0 = build_range_grid(h, wx, wy, wz);
   if (rc0 != MDWT_OK) return rc0;
-  if ((rc0 = make_bricks(h)) != MDWT_OK || (rc0 = make_joint(h)) != MDWT_OK) return rc0;
-  HIPCHK(h, hipMalloc(&h->d_counters, 4 * sizeof(unsigned long long)));
+  if ((rc0 = make_bricks(h)) != MDWT_OK || (rc0 = fit_joint(h)) != MDWT_OK) return rc0;
+  HIPCHK(h, device_alloc(h, &h->d_counters, 4 * sizeof(unsigned long long)));
   HIPCHK(h, hipDeviceGetAttribute(&h->cu_count, hipDeviceAttributeMultiprocessorCount, h->device));
   // this device's copy of the allocation-free read's staging array
   HIPCHK(h, mdwt::fb_scratch_setup(h->device));
@@ -911,7 +943,7 @@ int mdwt_set_mode(mdwt_renderer* h, int mode) {
   HIPCHK(h, hipSetDevice(h->device));
   h->mode = mode;
   reset_acc(h);
-  const int rc = make_joint(h);
+  const int rc = fit_joint(h);
   return rc != MDWT_OK ? rc : rebuild_majorants(h);
 }
 
@@ -1253,11 +1285,11 @@ int mdwt_trace_cells(mdwt_renderer* h, const float* org, const float* dir, int n
   const size_t nc = size_t(n) * std::max(max_cells, 1);
   float *d_org = nullptr, *d_dir = nullptr, *d_t = nullptr;
   int *d_cells = nullptr, *d_cnt = nullptr;
-  hipError_t e = hipMalloc(&d_org, size_t(n) * 12);
-  if (e == hipSuccess) e = hipMalloc(&d_dir, size_t(n) * 12);
-  if (e == hipSuccess) e = hipMalloc(&d_t, nc * 8);
-  if (e == hipSuccess) e = hipMalloc(&d_cells, nc * 4);
-  if (e == hipSuccess) e = hipMalloc(&d_cnt, size_t(n) * 4);
+  hipError_t e = device_alloc(h, &d_org, size_t(n) * 12);
+  if (e == hipSuccess) e = device_alloc(h, &d_dir, size_t(n) * 12);
+  if (e == hipSuccess) e = device_alloc(h, &d_t, nc * 8);
+  if (e == hipSuccess) e = device_alloc(h, &d_cells, nc * 4);
+  if (e == hipSuccess) e = device_alloc(h, &d_cnt, size_t(n) * 4);
   if (e == hipSuccess) e = hipMemcpy(d_org, org, size_t(n) * 12, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(d_dir, dir, size_t(n) * 12, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
@@ -1284,8 +1316,8 @@ int mdwt_gen_rays(mdwt_renderer* h, uint32_t frame, uint32_t sample, float* org,
   HIPCHK(h, hipSetDevice(h->device));
   const size_t n = size_t(h->W) * h->H;
   float *d_org = nullptr, *d_dir = nullptr;
-  hipError_t e = hipMalloc(&d_org, n * 12);
-  if (e == hipSuccess) e = hipMalloc(&d_dir, n * 12);
+  hipError_t e = device_alloc(h, &d_org, n * 12);
+  if (e == hipSuccess) e = device_alloc(h, &d_dir, n * 12);
   if (e == hipSuccess)
     e = mdwt::launch_gen_rays(h->cam, h->W, h->H, h->seed, frame, sample, h->jitter2d ? 1 : 0,
                               d_org, d_dir, h->stream);
@@ -1308,10 +1340,10 @@ int mdwt_clip_rays(mdwt_renderer* h, const float* org, const float* dir, int n, 
   HIPCHK(h, hipSetDevice(h->device));
   float *d_org = nullptr, *d_dir = nullptr, *d_t = nullptr;
   int* d_hit = nullptr;
-  hipError_t e = hipMalloc(&d_org, size_t(n) * 12);
-  if (e == hipSuccess) e = hipMalloc(&d_dir, size_t(n) * 12);
-  if (e == hipSuccess) e = hipMalloc(&d_t, size_t(n) * 8);
-  if (e == hipSuccess) e = hipMalloc(&d_hit, size_t(n) * 4);
+  hipError_t e = device_alloc(h, &d_org, size_t(n) * 12);
+  if (e == hipSuccess) e = device_alloc(h, &d_dir, size_t(n) * 12);
+  if (e == hipSuccess) e = device_alloc(h, &d_t, size_t(n) * 8);
+  if (e == hipSuccess) e = device_alloc(h, &d_hit, size_t(n) * 4);
   if (e == hipSuccess) e = hipMemcpy(d_org, org, size_t(n) * 12, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(d_dir, dir, size_t(n) * 12, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = mdwt::launch_clip(volume_params(h), d_org, d_dir, n, d_t, d_hit, h->stream);
@@ -1397,7 +1429,7 @@ int mdwt_set_moments(mdwt_renderer* h, int on) {
     for (auto& v : h->views) {
       const size_t bytes = size_t(v.width) * v.height * sizeof(Float4);
       if (want && !v.m2) {
-        if (hipMalloc(&v.m2, bytes) != hipSuccess) {
+        if (device_alloc(h, &v.m2, bytes) != hipSuccess) {
           v.m2 = nullptr;
           return fail(h, MDWT_ERR_OOM, "view second moments");
         }
@@ -1428,8 +1460,8 @@ int mdwt_stream_read(mdwt_renderer* h, uint64_t bytes, int iters, float* gbps) {
   const size_t n16 = size_t(bytes / 16);
   const unsigned grid = mdwt::kReadGrid;
   void *a = nullptr, *sums = nullptr;
-  if (hipMalloc(&a, n16 * 16) != hipSuccess) return fail(h, MDWT_ERR_OOM, "read buffer");
-  if (hipMalloc(&sums, size_t(grid) * sizeof(float)) != hipSuccess) {
+  if (device_alloc(h, &a, n16 * 16) != hipSuccess) return fail(h, MDWT_ERR_OOM, "read buffer");
+  if (device_alloc(h, &sums, size_t(grid) * sizeof(float)) != hipSuccess) {
     (void)hipFree(a);
     return fail(h, MDWT_ERR_OOM, "read partial sums");
   }
@@ -1462,8 +1494,8 @@ int mdwt_stream_copy(mdwt_renderer* h, uint64_t bytes, int iters, float* gbps) {
   HIPCHK(h, hipSetDevice(h->device));
   const size_t n16 = size_t(bytes / 16);
   void *a = nullptr, *b = nullptr;
-  if (hipMalloc(&a, n16 * 16) != hipSuccess) return fail(h, MDWT_ERR_OOM, "copy buffer");
-  if (hipMalloc(&b, n16 * 16) != hipSuccess) {
+  if (device_alloc(h, &a, n16 * 16) != hipSuccess) return fail(h, MDWT_ERR_OOM, "copy buffer");
+  if (device_alloc(h, &b, n16 * 16) != hipSuccess) {
     (void)hipFree(a);
     return fail(h, MDWT_ERR_OOM, "copy buffer");
   }
@@ -1546,7 +1578,7 @@ int build_view_orders(mdwt_renderer* h) {
     const auto& vw = h->views[i];
     const int nbx = (vw.width + h->bw - 1) / h->bw, nby = (vw.height + h->bh - 1) / h->bh;
     const std::vector<uint32_t> order = block_order(nbx, nby, h->bw, h->bh, h->tile, true);
-    HIPCHK(h, hipMalloc(&h->view_order[i], order.size() * sizeof(uint32_t)));
+    HIPCHK(h, device_alloc(h, &h->view_order[i], order.size() * sizeof(uint32_t)));
     HIPCHK(h, hipMemcpy(h->view_order[i], order.data(), order.size() * sizeof(uint32_t),
                         hipMemcpyHostToDevice));
     h->view_blocks[i] = int(order.size());
@@ -1578,9 +1610,9 @@ int build_items(mdwt_renderer* h) {
   h->d_items = nullptr;
   h->d_pitems = nullptr;
   h->d_item_ticks = nullptr;
-  HIPCHK(h, hipMalloc(&h->d_items, items.size() * sizeof(uint32_t)));
-  HIPCHK(h, hipMalloc(&h->d_pitems, items.size() * sizeof(uint32_t)));
-  HIPCHK(h, hipMalloc(&h->d_item_ticks, 2 * items.size() * sizeof(unsigned long long)));
+  HIPCHK(h, device_alloc(h, &h->d_items, items.size() * sizeof(uint32_t)));
+  HIPCHK(h, device_alloc(h, &h->d_pitems, items.size() * sizeof(uint32_t)));
+  HIPCHK(h, device_alloc(h, &h->d_item_ticks, 2 * items.size() * sizeof(unsigned long long)));
   HIPCHK(h, hipMemcpy(h->d_items, items.data(), items.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(h->d_pitems, items.data(), items.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
   HIPCHK(h, hipMemset(h->d_item_ticks, 0, 2 * items.size() * sizeof(unsigned long long)));
@@ -1979,8 +2011,8 @@ int mdwt_batch_set_views(mdwt_renderer* h, const mdwt_view* views, int n) {
     vp.spp = v.spp;
     vp.seed = v.seed;
     const size_t bytes = size_t(v.width) * v.height * sizeof(Float4);
-    if (hipMalloc(&vp.accum, bytes) != hipSuccess ||
-        (h->moments && hipMalloc(&vp.m2, bytes) != hipSuccess)) {
+    if (device_alloc(h, &vp.accum, bytes) != hipSuccess ||
+        (h->moments && device_alloc(h, &vp.m2, bytes) != hipSuccess)) {
       h->views.push_back(vp);
       free_batch(h);
       return fail(h, MDWT_ERR_OOM, "view accumulators");
@@ -1998,10 +2030,10 @@ int mdwt_batch_set_views(mdwt_renderer* h, const mdwt_view* views, int n) {
     else
       at->second += px;
   }
-  HIPCHK(h, hipMalloc(&h->d_views, h->views.size() * sizeof(mdwt::ViewParams)));
+  HIPCHK(h, device_alloc(h, &h->d_views, h->views.size() * sizeof(mdwt::ViewParams)));
   HIPCHK(h, hipMemcpy(h->d_views, h->views.data(), h->views.size() * sizeof(mdwt::ViewParams),
                       hipMemcpyHostToDevice));
-  HIPCHK(h, hipMalloc(&h->d_work, 4 * sizeof(unsigned)));
+  HIPCHK(h, device_alloc(h, &h->d_work, 4 * sizeof(unsigned)));
   const unsigned zero[4] = {0, 0, 0, 0};
   HIPCHK(h, hipMemcpy(h->d_work, zero, sizeof(zero), hipMemcpyHostToDevice));
   h->batch_frame = h->batch_accum = 0;

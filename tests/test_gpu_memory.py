@@ -113,3 +113,79 @@ def test_a_frame_that_was_not_allocated_is_an_error(capi, hip):
     r.render(1)
     assert r.read_accum().shape == want.shape
     r.close()
+
+
+def test_joint_copy_goes_with_the_modes_that_read_it(capi, hip):
+    dims = (512, 512, 256)
+    joint = 4 * dims[0] * dims[1] * dims[2]  # 256 MiB
+    r = _renderer(capi, 2, dims)
+    base = _memory(hip)[0]
+    for mode, has in ((3, True), (8, True), (9, False), (4, True), (1, False)):
+        r.set_mode(mode)
+        assert abs(base - _memory(hip)[0] - has * joint) < 16 * MIB, mode
+    r.close()
+
+
+@pytest.mark.parametrize("mode", [3, 5, 7])
+def test_joint_copy_leaves_a_reserve(capi, hip, mode):
+    """Not made where less than an eighth of the device would be left; the same
+    images from the channels' own bricks."""
+    dims = (512, 512, 256)
+    r = _renderer(capi, 2, dims)
+    r.set_mode(mode)
+    r.render(3)
+    want = r.read_accum()
+    r.close()
+    r = _renderer(capi, 2, dims)
+    with _only(hip, _memory(hip)[1] // 8 + 128 * MIB):
+        base = _memory(hip)[0]
+        r.set_mode(mode)
+        assert abs(base - _memory(hip)[0]) < 16 * MIB
+        r.render(3)
+        got = r.read_accum()
+    assert want[..., :3].std() > 0.01
+    np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32))
+    r.close()
+
+
+@pytest.mark.parametrize("views", [False, True])
+def test_joint_copy_makes_room(capi, hip, views):
+    """A frame, or views, that fit only where the joint copy was (1.5 GiB), with the
+    images of a handle that has both; a graph captured with it is not replayed."""
+    dims = (1024, 768, 512)
+    joint = 4 * dims[0] * dims[1] * dims[2]
+    view = {"from": (0.5, 0.6, 2.4), "at": (0.5, 0.5, 0.5), "up": (0.0, 1.0, 0.0), "fovy": 45.0, "width": 8192,
+            "height": 8192, "spp": 1, "seed": 3}
+    small = dict(view, width=96, height=64)
+    out = []
+    for short in (False, True):
+        r = _renderer(capi, 3, dims)
+        r.batch_set_launch(2)
+        r.batch_set_views([small])
+        r.batch_render(2)  # captures the graph
+        base = _memory(hip)[0]
+        if short:
+            with _only(hip, 640 * MIB):
+                if views:
+                    r.batch_set_views([small, view])
+                else:
+                    r.set_frame(8192, 8192, 1, True, (0.2, 0.4, 0.6))
+                # the copy went, 1 GiB of accumulators came (and up to 256 MiB of RGBA8)
+                assert _memory(hip)[0] > 640 * MIB + joint - 1024 * MIB - 300 * MIB
+                r.batch_render(2)
+                if not views:
+                    r.render(1)
+        else:
+            if views:
+                r.batch_set_views([small, view])
+            else:
+                r.set_frame(8192, 8192, 1, True, (0.2, 0.4, 0.6))
+            assert base - _memory(hip)[0] > 1024 * MIB
+            r.batch_render(2)
+            if not views:
+                r.render(1)
+        out.append([r.batch_read_view(0)] + [r.batch_read_view(1) if views else r.read_accum()])
+        r.close()
+    for a, b in zip(*out):
+        assert a[..., :3].std() > 0.01
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
