@@ -255,26 +255,29 @@ bool several_view_frames_apply(const RenderParams& p, int mode) {
          grid_fits(uint64_t(p.fr.n_items) * unsigned(p.fr.bw * p.fr.bh / 64), kThreads);
 }
 
-hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int dtype, int* out) {
+PersistentKernel persistent_kernel(const RenderParams& p, int mode, int dtype) {
+  PersistentKernel k;
   const bool wave = wave_persistent(p, mode);
-  const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
-  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 2)
-                          : select_persistent(mode, dtype, is_lit(p), wide_views(p, dtype));
-  const hipError_t e = prepare(f, lds);
+  k.lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
+  k.fn = wave ? select_wave_kernel(p, mode, dtype, 2)
+              : select_persistent(mode, dtype, is_lit(p), wide_views(p, dtype));
+  k.threads = p.fr.bw * p.fr.bh;
+  return k;
+}
+
+hipError_t persistent_blocks_per_cu(const PersistentKernel& k, int* out) {
+  const hipError_t e = prepare(k.fn, k.lds);
   if (e != hipSuccess) return e;
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(out, f, p.fr.bw * p.fr.bh, lds);
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(out, k.fn, k.threads, k.lds);
 }
 
 hipError_t launch_views_persistent(const RenderParams& p, int mode, int dtype, int grid,
                                    hipStream_t s) {
   if (p.fr.n_items <= 0 || grid <= 0 || !p.fr.work) return hipErrorInvalidValue;
-  const bool wave = wave_persistent(p, mode);
-  const size_t lds = wave ? wave_lds_bytes(p) : render_lds_bytes(p);
-  const RenderFn f = wave ? select_wave_kernel(p, mode, dtype, 2)
-                          : select_persistent(mode, dtype, is_lit(p), wide_views(p, dtype));
-  hipError_t e = prepare(f, lds);
+  const PersistentKernel k = persistent_kernel(p, mode, dtype);
+  hipError_t e = prepare(k.fn, k.lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(f, dim3(unsigned(grid)), dim3(unsigned(p.fr.bw * p.fr.bh)), lds, s, p);
+  hipLaunchKernelGGL(k.fn, dim3(unsigned(grid)), dim3(unsigned(k.threads)), k.lds, s, p);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   hipLaunchKernelGGL(views_advance_kernel, dim3(1), dim3(64), 0, s, p.fr.work, p.fr.accumulate);
   return hipGetLastError();

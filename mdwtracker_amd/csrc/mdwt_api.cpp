@@ -165,7 +165,8 @@ struct mdwt_renderer {
   std::vector<unsigned long long> pitem_ticks;
   bool pitems_measured = false;
   uint32_t batch_frame = 0, batch_accum = 0;
-  int batch_grid = 0, batch_grid_key = -1;  // resident grid of launch form 2
+  int batch_grid = 0;  // resident grid of launch form 2, of this kernel
+  mdwt::PersistentKernel batch_grid_of;
   hipGraph_t graph = nullptr;               // launch form 2: one captured frame
   hipGraphExec_t graph_exec = nullptr;
   bool graph_valid = false;
@@ -1837,17 +1838,15 @@ int deal_by_cost(mdwt_renderer* h, int G) {
   return MDWT_OK;
 }
 
-// resident workgroups of the persistent launch (cached per kernel choice),
-// at most one per item
+// resident workgroups of the persistent launch (kept while its kernel is the
+// same), at most one per item
 int persistent_grid(mdwt_renderer* h, const mdwt::RenderParams& p, int* grid) {
-  const bool lit = p.fr.sh.shadows || p.fr.sh.gradient || p.fr.aov != nullptr;
-  const int key = int(mdwt::render_lds_bytes(p)) * 64 + h->mode * 16 + h->bw * h->bh / 64 * 2 +
-                  (lit ? 1 << 30 : 0);
-  if (key != h->batch_grid_key) {
+  const mdwt::PersistentKernel k = mdwt::persistent_kernel(p, h->mode, h->dtype);
+  if (!(k == h->batch_grid_of)) {
     int per_cu = 0;
-    HIPCHK(h, mdwt::views_persistent_blocks_per_cu(p, h->mode, h->dtype, &per_cu));
+    HIPCHK(h, mdwt::persistent_blocks_per_cu(k, &per_cu));
     h->batch_grid = std::max(1, per_cu) * h->cu_count;
-    h->batch_grid_key = key;
+    h->batch_grid_of = k;
   }
   *grid = std::min(h->batch_grid, std::max(1, p.fr.n_items));
   return MDWT_OK;

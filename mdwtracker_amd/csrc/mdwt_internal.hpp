@@ -70,8 +70,18 @@ hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count,
 // graph captures for one frame
 hipError_t launch_views_persistent(const RenderParams& p, int mode, int dtype, int grid,
                                    hipStream_t s);
-// resident workgroups per CU of that persistent kernel
-hipError_t views_persistent_blocks_per_cu(const RenderParams& p, int mode, int dtype, int* out);
+// the kernel that it launches for p (the schedule, mode, shading, channels and
+// block shape choose it), and its resident workgroups per CU
+struct PersistentKernel {
+  RenderFn fn = nullptr;
+  size_t lds = 0;
+  int threads = 0;
+  bool operator==(const PersistentKernel& o) const {
+    return fn == o.fn && lds == o.lds && threads == o.threads;
+  }
+};
+PersistentKernel persistent_kernel(const RenderParams& p, int mode, int dtype);
+hipError_t persistent_blocks_per_cu(const PersistentKernel& k, int* out);
 // batched views in one launch: one workgroup per item of p.fr.items (view,
 // pixel block), frame and accumulation ids from p.fr.frame_id / accum_id
 hipError_t launch_views(const RenderParams& p, int mode, int dtype, bool count, hipStream_t s);

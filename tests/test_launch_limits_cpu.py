@@ -89,3 +89,28 @@ def test_auxiliary_buffers_are_packed_in_pieces_that_fit(tmp_path):
     EXPECT(launch_pack_aov(nullptr, row, 2 + c, n + 1, nullptr, nullptr) == hipErrorInvalidValue);
     EXPECT(launch_pack_aov(nullptr, row, 2 + c, size_t(1) << 30, nullptr, nullptr) == hipErrorInvalidValue);
   }""")
+
+
+def test_persistent_grid_belongs_to_the_kernel(tmp_path):
+    """The resident grid of launch form 2 is kept for one kernel: whatever changes
+    the kernel, its tables or its workgroup (the schedule too) is another."""
+    run(tmp_path, r"""
+  for (int mode = 0; mode < 10; ++mode)
+    for (int dtype = 0; dtype < 4; ++dtype) {
+      RenderParams a = params(0, 100, 16, 16), b = a;
+      const PersistentKernel k = persistent_kernel(a, mode, dtype);
+      EXPECT(k.fn && k == persistent_kernel(b, mode, dtype));
+      b.fr.schedule = 0;
+      EXPECT((k == persistent_kernel(b, mode, dtype)) == (mode > 5));
+      b = a;
+      b.fr.sh.shadows = 1;
+      EXPECT(!(k == persistent_kernel(b, mode, dtype)) || mode == 9);
+      b = a;
+      b.fr.bh = 8;
+      EXPECT(!(k == persistent_kernel(b, mode, dtype)));
+      b = a;
+      b.tf.stride = 128;
+      EXPECT(!(k == persistent_kernel(b, mode, dtype)));
+      EXPECT(!(k == persistent_kernel(a, (mode + 1) % 10, dtype)));
+      EXPECT(!(k == persistent_kernel(a, mode, (dtype + 1) % 4)));
+    }""")
