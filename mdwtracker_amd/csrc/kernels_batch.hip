@@ -229,6 +229,7 @@ bool is_lit(const RenderParams& p) {
 }
 
 hipError_t prepare(RenderFn f, size_t lds) {
+  if (!f) return hipErrorInvalidValue;
   if (lds <= 65536) return hipSuccess;
   return hipFuncSetAttribute(reinterpret_cast<const void*>(f),
                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));

@@ -340,6 +340,7 @@ bool six_waves(const RenderParams& p, int dtype) {
 }
 // Kernels whose static plus dynamic LDS passes 64 KiB must say so first.
 hipError_t prepare(RenderFn f, size_t lds) {
+  if (!f) return hipErrorInvalidValue;
   hipFuncAttributes a{};
   hipError_t e = hipFuncGetAttributes(&a, reinterpret_cast<const void*>(f));
   if (e != hipSuccess) return e;

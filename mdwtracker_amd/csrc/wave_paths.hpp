@@ -988,15 +988,16 @@ MDWT_WAVE_KERNEL void render_views_wave_persistent(RenderParams P) {
 }
 #undef MDWT_WAVE_PROLOGUE
 
-// The kernel of a mode for launch form `form` (select_wave_kernel; the persistent
-// form has no shaded instance).
+// The kernel of a mode for launch form `form` (select_wave_kernel), nullptr for a
+// form that has none (the persistent form has no shaded instance).
 template <int MODE, int DT, bool WIDE, bool LIT>
 RenderFn wave_fn_form(int form) {
   if (form == 0) return render_wave<MODE, DT, WIDE, LIT>;
   if (form == 1) return render_views_wave<MODE, DT, WIDE, LIT>;
+  if (form == 3) return render_wave_team<MODE, DT, WIDE, LIT>;
   if constexpr (!LIT)
     if (form == 2) return render_views_wave_persistent<MODE, DT, WIDE>;
-  return render_wave_team<MODE, DT, WIDE, LIT>;
+  return nullptr;
 }
 template <int MODE, bool WIDE, bool LIT>
 RenderFn wave_fn_dt(int dtype, int form) {

@@ -114,3 +114,28 @@ def test_persistent_grid_belongs_to_the_kernel(tmp_path):
       EXPECT(!(k == persistent_kernel(a, (mode + 1) % 10, dtype)));
       EXPECT(!(k == persistent_kernel(a, mode, (dtype + 1) % 4)));
     }""")
+
+
+def test_no_kernel_for_a_form_that_has_none(tmp_path):
+    """The persistent form has no shaded instance, and there are four forms; what
+    has no kernel is not launched."""
+    run(tmp_path, r"""
+  for (int mode = 0; mode < 6; ++mode)
+    for (int dtype = 0; dtype < 4; ++dtype)
+      for (int channels : {4, 10})
+        for (int shaded = 0; shaded < 2; ++shaded) {
+          RenderParams p = params(1, 1, 16, 16);
+          p.vol.channels = channels;
+          p.fr.sh.gradient = shaded;
+          RenderFn seen[4];
+          for (int form = 0; form < 4; ++form) {
+            seen[form] = select_wave_kernel(p, mode, dtype, form);
+            EXPECT((seen[form] != nullptr) == !(shaded && form == 2));
+            for (int k = 0; k < form; ++k) EXPECT(seen[form] != seen[k]);
+          }
+          EXPECT(!select_wave_kernel(p, mode, dtype, -1) && !select_wave_kernel(p, mode, dtype, 4));
+          EXPECT(persistent_kernel(p, mode, dtype).fn);
+        }
+  PersistentKernel none;
+  int n = 0;
+  EXPECT(persistent_blocks_per_cu(none, &n) == hipErrorInvalidValue);""")
