@@ -170,7 +170,8 @@ struct mdwt_renderer {
   hipGraph_t graph = nullptr;               // launch form 2: one captured frame
   hipGraphExec_t graph_exec = nullptr;
   bool graph_valid = false;
-  mdwt::RenderParams graph_params;  // what the captured graph launches
+  mdwt::RenderParams graph_params;  // what the captured graph launches, with this kernel
+  mdwt::PersistentKernel graph_kernel;
   int graph_grid = 0;
   // per-view launches (the batch path in use): each view's block order and
   // block count, events around each view's launch, the last frame's times
@@ -1861,7 +1862,9 @@ int batch_render_persistent(mdwt_renderer* h, int n_frames, float* ms_out) {
   int grid = 0;
   int rc = persistent_grid(h, p, &grid);
   if (rc != MDWT_OK) return rc;
-  if (!h->graph_valid || grid != h->graph_grid ||
+  // (the mode is in the kernel, not in the parameters)
+  const mdwt::PersistentKernel kernel = mdwt::persistent_kernel(p, h->mode, h->dtype);
+  if (!h->graph_valid || grid != h->graph_grid || !(kernel == h->graph_kernel) ||
       std::memcmp(&p, &h->graph_params, sizeof(p)) != 0) {
     if (h->graph_exec) (void)hipGraphExecDestroy(h->graph_exec);
     if (h->graph) (void)hipGraphDestroy(h->graph);
@@ -1880,6 +1883,7 @@ int batch_render_persistent(mdwt_renderer* h, int n_frames, float* ms_out) {
     h->graph = g;
     HIPCHK(h, hipGraphInstantiate(&h->graph_exec, h->graph, nullptr, nullptr, 0));
     h->graph_params = p;
+    h->graph_kernel = kernel;
     h->graph_grid = grid;
     h->graph_valid = true;
   }
