@@ -273,7 +273,29 @@ struct Ctx {
     }
   }
 
+  // The value of one channel that is the same for the whole wave (NaN outside the
+  // unit cube), as in the thread-per-pixel kernels' channel loops: the channel's
+  // base is scalar. corners(), whose offsets count from the array's base, costs
+  // them an addition per voxel, a second address path and its registers (-m 9,
+  // 300 x 200, 128^3 u8: 640 -> 720 us on four channels; shaded batched views in
+  // launch form 2 fell from three waves per SIMD to two). All eight loads are
+  // issued before the first value is used (see trilinear).
   __device__ __forceinline__ float sample(V3 p, int c) const {
+    if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
+      return qnan();
+    const Foot f = foot(p);
+    const uint8_t* base = bricks + size_t(c) * brick_stride;
+    uint32_t w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = fetch_bits<DT>(base, f.i[i]);
+    asm("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]));
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = voxel_value<DT>(w[i]);
+    return lerp8(v, f.fx, f.fy, f.fz, true);
+  }
+  // the same of a channel that differs between lanes
+  __device__ __forceinline__ float sample_lane(V3 p, int c) const {
     if (p.x < 0.0f || p.x > 1.0f || p.y < 0.0f || p.y > 1.0f || p.z < 0.0f || p.z > 1.0f)
       return qnan();
     return trilinear(corners(p, c));
@@ -295,8 +317,7 @@ struct Ctx {
   }
   // full transferFunction (deviceCode.cu:27-42) for the blend and marcher
   // modes; f is never NaN here (callers test the unit cube or the sample)
-  __device__ __forceinline__ float4 tf_rgba(float f, int c) const {
-    const ChanTf t = chtf[c];
+  __device__ __forceinline__ float4 tf_rgba(float f, const ChanTf& t) const {
     if (f < t.dlo || f > t.dhi) return make_float4(1.f, 0.f, 1.f, 0.f);
     const float r1 = (f - t.dlo) * t.idw;
     const float r2 = (r1 - t.xlo) * t.ixw;
@@ -327,8 +348,8 @@ struct Ctx {
         div = 2.0f * eps;
       }
       float r;
-      const float v1 = tf_alpha(sample(v3(p1[0], p1[1], p1[2]), c), c, r);
-      const float v2 = tf_alpha(sample(v3(p2[0], p2[1], p2[2]), c), c, r);
+      const float v1 = tf_alpha(sample_lane(v3(p1[0], p1[1], p1[2]), c), c, r);
+      const float v2 = tf_alpha(sample_lane(v3(p2[0], p2[1], p2[2]), c), c, r);
       g[i] = (v2 - v1) / div;
     }
     return v3(g[0], g[1], g[2]);

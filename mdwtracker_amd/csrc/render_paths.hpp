@@ -310,7 +310,7 @@ __device__ void trace_multi(const Ctx<DT>& X, const GridRay& g, float prd_t1, Rn
         float th, rand;
         rng.vc_pair(visit, uint32_t(sel), j, th, rand);
         const float thr = th * mj;
-        const float value = X.sample(xT, sel);
+        const float value = X.sample_lane(xT, sel);
         cnt.samples++;
         if (!(value != value)) {
           float r2;
@@ -529,12 +529,19 @@ __device__ void march_comp(const Ctx<DT>& X, V3 org, V3 dir0, V3 w2u, float prd_
   for (int n = 0; n < kMaxChannels; ++n) {
     float a = 0.0f, r = 0.f, g = 0.f, b = 0.f;
     if (n < X.C) {
+      // The channel's parameters are read once, for its own loop. (An opaque index:
+      // otherwise the compiler reads all twelve channels' before the first, 100 VGPRs
+      // that keep the kernel at two waves per SIMD: 2.80 -> 2.01 ms at 1920 x 1080, four
+      // 128^3 u8 channels.)
+      int c = n;
+      asm volatile("" : "+s"(c));
+      const ChanTf tf = X.chtf[c];
       for (float t = prd_t0; (t < prd_t1) && (a < 0.99f); t += dt) {
         const V3 posTex = pos * w2u;
-        const float v = X.sample(posTex, n);
+        const float v = X.sample(posTex, c);
         float4 sc = make_float4(0.f, 0.f, 0.f, 0.f);
         if (!(v != v)) {
-          sc = X.tf_rgba(v, n);
+          sc = X.tf_rgba(v, tf);
           cnt.samples++;
         }
         const float k = 1.f - a;

@@ -413,8 +413,8 @@ __device__ __forceinline__ V3 opacity_gradient(const Ctx<DT>& X, const float* s_
     if (!low) p1[i] = pc[i] - eps;
     if (!high) p2[i] = pc[i] + eps;
     const float div = low || high ? eps : 2.0f * eps;
-    const float v1 = alpha_lookup(s_a, tf, X.sample(v3(p1[0], p1[1], p1[2]), c));
-    const float v2 = alpha_lookup(s_a, tf, X.sample(v3(p2[0], p2[1], p2[2]), c));
+    const float v1 = alpha_lookup(s_a, tf, X.sample_lane(v3(p1[0], p1[1], p1[2]), c));
+    const float v2 = alpha_lookup(s_a, tf, X.sample_lane(v3(p2[0], p2[1], p2[2]), c));
     g[i] = (v2 - v1) / div;
   }
   return v3(g[0], g[1], g[2]);
@@ -779,7 +779,7 @@ __device__ __forceinline__ float4 trace_sample(const RenderParams& P, const Ctx<
         h.b = sb.z;
       } else {
         float r2;
-        (void)X.tf_alpha(X.sample(xT, hit_c), hit_c, r2);
+        (void)X.tf_alpha(X.sample_lane(xT, hit_c), hit_c, r2);
         X.tf_rgb(r2, hit_c, h);
         h.channel = hit_c;
       }
