@@ -105,8 +105,12 @@ __device__ __forceinline__ void render_views_persistent_body(const RenderParams&
 
 // Occupancy targets as for the single-view frame kernel (kernels_render.hip):
 // six waves per SIMD for -m 0 / -m 2 without lighting on at most four
-// channels of 1- or 2-byte voxels (wide), a stated three for blend tracking,
-// the natural budget otherwise.
+// channels of 1- or 2-byte voxels (wide), a stated three for -m 3 / 4 / 5, four for
+// the marchers -m 6 / 7 / 8 (three on f32), the natural budget otherwise. A batch
+// fills the chip, so the marchers have no second instance for small frames. 16
+// views of 128^2 to 512^2, 128^3 voxels, at the natural budgets and so: -m 8 on two
+// f32 channels 5.80 -> 4.44 ms; launch form 2, shaded, -m 3 on two f16 channels 1.05 ->
+// 0.90 ms, -m 5 on ten 7.1 -> 5.2 ms.
 template <int MODE, int DT, bool COUNT, bool LIT>
 __global__ __launch_bounds__(256) void render_views_kernel(RenderParams P) {
   render_views_body<MODE, DT, COUNT, LIT>(P);
@@ -117,7 +121,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void r
   render_views_body<MODE, DT, COUNT, false>(P);
 }
 template <int MODE, int DT, bool COUNT, bool LIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) void render_views_kernel_w3(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_views_kernel_w3(
+    RenderParams P) {
+  render_views_body<MODE, DT, COUNT, LIT>(P);
+}
+template <int MODE, int DT, bool COUNT, bool LIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_views_kernel_w4(
     RenderParams P) {
   render_views_body<MODE, DT, COUNT, LIT>(P);
 }
@@ -131,8 +140,13 @@ render_views_persistent_w6(RenderParams P) {
   render_views_persistent_body<MODE, DT, false>(P);
 }
 template <int MODE, int DT, bool LIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void
 render_views_persistent_w3(RenderParams P) {
+  render_views_persistent_body<MODE, DT, LIT>(P);
+}
+template <int MODE, int DT, bool LIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void
+render_views_persistent_w4(RenderParams P) {
   render_views_persistent_body<MODE, DT, LIT>(P);
 }
 template <int MODE, int DT, bool LIT>
@@ -140,8 +154,10 @@ RenderFn persistent_fn(bool wide) {
   if constexpr ((MODE == 0 || MODE == 2) && !LIT) {
     if (wide) return render_views_persistent_w6<MODE, DT>;
     return render_views_persistent<MODE, DT, LIT>;
-  } else if constexpr (MODE == 4 || MODE == 5) {
+  } else if constexpr (MODE >= 3 && MODE <= 8 && (MODE <= 5 || DT == MDWT_DT_F32)) {
     return render_views_persistent_w3<MODE, DT, LIT>;
+  } else if constexpr (MODE >= 6 && MODE <= 8) {
+    return render_views_persistent_w4<MODE, DT, LIT>;
   } else {
     return render_views_persistent<MODE, DT, LIT>;
   }
@@ -187,8 +203,10 @@ RenderFn views_fn(bool wide) {
   if constexpr ((MODE == 0 || MODE == 2) && !LIT) {
     if (wide) return render_views_kernel_w6<MODE, DT, COUNT>;
     return render_views_kernel<MODE, DT, COUNT, LIT>;
-  } else if constexpr (MODE == 4 || MODE == 5) {
+  } else if constexpr (MODE >= 3 && MODE <= 8 && (MODE <= 5 || DT == MDWT_DT_F32)) {
     return render_views_kernel_w3<MODE, DT, COUNT, LIT>;
+  } else if constexpr (MODE >= 6 && MODE <= 8) {
+    return render_views_kernel_w4<MODE, DT, COUNT, LIT>;
   } else {
     return render_views_kernel<MODE, DT, COUNT, LIT>;
   }

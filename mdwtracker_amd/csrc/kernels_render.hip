@@ -68,8 +68,8 @@ __global__ __launch_bounds__(256) void render_kernel(RenderParams P) {
 // compiler spills the rest to scratch): more waves hide the latency of the
 // sample's dependent loads and the cell walk better than the spills cost
 // (-m 2 0.334 -> 0.317 ms, -m 0 0.370 -> 0.345 ms per 1024^2 frame on four
-// 256^3 u8 channels). -m 3 and the lit kernels spill too much and stay at
-// their natural budget.
+// 256^3 u8 channels). The lit kernels spill too much and stay at their natural
+// budget.
 template <int MODE, int DT, bool COUNT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void render_kernel_w6(
     RenderParams P) {
@@ -263,26 +263,42 @@ __global__ __launch_bounds__(256) void read_kernel(const float4* __restrict__ sr
   if (threadIdx.x == 0) sums[blockIdx.x] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
 }
 
-// Blend tracking (-m 4 / 5) needs more than 128 VGPRs, so it runs at three
-// waves per SIMD whatever it is given. Without that stated, the scheduler
-// squeezed it towards four waves by issuing the blended sample's voxel loads
-// one or two at a time with a full wait in between (0.41 -> 0.9 ms per frame
-// from an unrelated four-register change); with the target stated it keeps
-// them in flight together.
+// -m 3 to -m 8 read every channel at a position, a joint voxel of each corner at
+// a time; the marchers have two steps' voxels in flight. At their natural budget
+// they take 170 to 213 VGPRs and run at two waves per SIMD, so the occupancy is
+// stated. -m 3 / 4 / 5: three waves (-m 4, 1024^2, 128^3 f16: 145 -> 105 us on one
+// channel, 197 -> 149 us on two). The marchers: four on 1- and 2-byte voxels, three on
+// f32, as in the several-frame kernels (-m 8, 1024 x 768, 96^3: 994 -> 699 us on two
+// f16 channels, 1045 -> 738 us on four, 1010 -> 769 us on two of f32). A frame that
+// three waves per SIMD hold gains nothing from the fourth's budget and pays its
+// spills, on 2-byte voxels 2 to 6 % (512 x 384, the largest, -m 6 on two f16
+// channels: 335 against 327 us; 640 x 480: 391 against 400 us): three waves there.
 template <int MODE, int DT, bool COUNT, bool LIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 3))) void render_kernel_w3(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void render_kernel_w3(
+    RenderParams P) {
+  render_body<MODE, DT, COUNT, LIT>(P);
+}
+template <int MODE, int DT, bool COUNT, bool LIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void render_kernel_w4(
     RenderParams P) {
   render_body<MODE, DT, COUNT, LIT>(P);
 }
 
 // wide: the six-wave entry for -m 0 / -m 2 without lighting (see
-// render_kernel_w6; chosen per launch by six_waves()).
+// render_kernel_w6) and the four-wave one for the marchers on 2-byte voxels;
+// chosen per launch by wide_kernel().
 template <int MODE, int DT, bool COUNT, bool LIT>
 RenderFn static_fn(bool wide) {
   if constexpr ((MODE == 0 || MODE == 2) && !LIT) {
     if (wide) return render_kernel_w6<MODE, DT, COUNT>;
     return render_kernel<MODE, DT, COUNT, LIT>;
-  } else if constexpr (MODE == 4 || MODE == 5) {
+  } else if constexpr (MODE >= 6 && MODE <= 8 && DT == MDWT_DT_U8) {
+    return render_kernel_w4<MODE, DT, COUNT, LIT>;
+  } else if constexpr (MODE >= 6 && MODE <= 8 && DT != MDWT_DT_F32 && !COUNT) {
+    if (wide) return render_kernel_w4<MODE, DT, COUNT, LIT>;
+    if constexpr (LIT) return render_kernel<MODE, DT, COUNT, LIT>;
+    return render_kernel_w3<MODE, DT, COUNT, LIT>;
+  } else if constexpr (MODE >= 3 && MODE <= 8) {
     return render_kernel_w3<MODE, DT, COUNT, LIT>;
   } else {
     return render_kernel<MODE, DT, COUNT, LIT>;
@@ -338,6 +354,11 @@ bool is_lit(const RenderParams& p) {
 bool six_waves(const RenderParams& p, int dtype) {
   return p.vol.channels <= 4 && (dtype == MDWT_DT_U8 || dtype == MDWT_DT_U16);
 }
+bool wide_kernel(const RenderParams& p, int mode, int dtype) {
+  if (mode < 6) return six_waves(p, dtype);
+  constexpr int kSimds = 4 * 256;  // of 256 CUs
+  return p.fr.n_blocks > (is_lit(p) ? 2 : 3) * kSimds / (p.fr.bw * p.fr.bh / 64);
+}
 // Kernels whose static plus dynamic LDS passes 64 KiB must say so first.
 hipError_t prepare(RenderFn f, size_t lds) {
   if (!f) return hipErrorInvalidValue;
@@ -368,7 +389,7 @@ hipError_t launch_render(const RenderParams& p, int mode, int dtype, bool count,
   if (team && !several_frames_apply(p, mode, count)) return hipErrorInvalidValue;
   const RenderFn f = wave   ? select_wave_kernel(p, mode, dtype, team ? 3 : 0)
                      : team ? select_march_team(mode, dtype, is_shaded(p))
-                            : select_render(mode, dtype, count, lit, six_waves(p, dtype));
+                            : select_render(mode, dtype, count, lit, wide_kernel(p, mode, dtype));
   const hipError_t e = prepare(f, lds);
   if (e != hipSuccess) return e;
   if (team) {  // one workgroup per 8x8 quad

@@ -421,11 +421,21 @@ __device__ void trace_blend(const Ctx<DT>& X, const GridRay& g, float prd_t1, Rn
           cnt.rejections++;
           return;
         }
-        const float4 s = blend_channels<MODE, DT>(X, xT);
+        // the blended opacity, the largest in both blends (0 outside the unit
+        // cube, where the values are NaN); the colour only at the hit
+        float top = 0.0f;
+        auto all = X.all_channels(xT);
+        X.each(all, [&](int c, float value) {
+          float r2;
+          const float a = X.tf_alpha(value, c, r2);
+          if (a > top) top = a;
+          return true;
+        });
         cnt.samples++;
         const float th = rng.pair_thr();
         u = rng.pair_dist();
-        if (s.w > 0.0f && th * majorant < s.w) {
+        if (top > 0.0f && th * majorant < top) {
+          const float4 s = blend_channels<MODE, DT>(X, xT);
           h.missed = false;
           h.tHit = tWorld;
           h.channel = 0;
