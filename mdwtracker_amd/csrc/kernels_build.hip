@@ -292,11 +292,24 @@ __global__ __launch_bounds__(256) void range_pencil_kernel(RangeParams P) {
 
 // Majorants. A cell's majorant in a channel is the largest of the opacities at
 // the texels its value range covers, so the opacity of every texel is computed
-// once per workgroup into LDS and kMajLanes lanes take the maximum over the
-// cell's texels (a maximum does not depend on the order). One lane per cell,
-// with a lookup and a division per texel, took 42 us on 55 k cells of three
-// channels and 121 us on 512 cells of four.
+// once per workgroup into LDS, and a maximum over texels does not depend on the
+// order. (With a lookup and a division per texel and one lane per cell, 55 k cells
+// of three channels took 42 us and 512 cells of four 121 us.)
+//
+// SPREAD: a group of kMajLanes lanes per entry takes its texels side by side.
+// Otherwise a lane per entry: it takes a short range alone, and its group takes the
+// longer ones together, one after another. A rebuild (the whole call) of one slider's
+// change, smooth data: 64^3 cells of four channels, 64 texels: 91 us spread, 24 with a
+// lane each (33 with one lane and a lookup per texel); 128^3 cells, 16 texels: 572 and
+// 58 us (76); 38^3 cells, 256 texels: 37 and 46 us (53); 24^3 cells, 2048 texels, one
+// channel of noise: 39 and 118 us (430).
 constexpr int kMajLanes = 16;
+// A lane each wins from about 64 k entries on; below, with long tables, the entries
+// alone leave the chip idle. The shorter the table, the less there is to spread: with
+// 64 texels the two meet between 14 and 33 k entries (four channels' sums: 22.5 us
+// spread against 25.5 at 13.8 k, 27.1 against 21.9 at 32.8 k), with 16 or fewer below 14 k
+// (18.0 against 17.2).
+inline int spread_entries(int texels) { return texels <= 32 ? 4096 : (texels <= 128 ? 16384 : 65536); }
 
 // maximum over the kMajLanes lanes of a group
 __device__ __forceinline__ float group_max(float m) {
@@ -304,13 +317,39 @@ __device__ __forceinline__ float group_max(float m) {
   for (int o = kMajLanes / 2; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
   return m;
 }
+// maximum (at least 0) of table[at + i], i = i0 .. i1: SPREAD for the group's one
+// interval, otherwise for every lane's own (all lanes of the group call it)
+template <bool SPREAD>
+__device__ __forceinline__ float interval_max(const float* table, int at, int i0, int i1) {
+  const int sub = threadIdx.x % kMajLanes, first = (threadIdx.x & 63) - sub;
+  float m = 0.f;
+  if (SPREAD) {
+    for (int i = i0 + sub; i <= i1; i += kMajLanes) m = fmaxf(m, table[at + i]);
+    return group_max(m);
+  }
+  const bool wide = i1 - i0 >= kMajLanes;
+  if (!wide)
+    for (int i = i0; i <= i1; ++i) m = fmaxf(m, table[at + i]);
+  uint32_t todo = uint32_t(__ballot(wide) >> first) & ((1u << kMajLanes) - 1u);
+  while (todo) {  // the same for the lanes of a group
+    const int l = __builtin_ctz(todo);
+    todo &= todo - 1u;
+    const int j0 = __shfl(i0, first + l, 64), j1 = __shfl(i1, first + l, 64), t = __shfl(at, first + l, 64);
+    float x = 0.f;
+    for (int i = j0 + sub; i <= j1; i += kMajLanes) x = fmaxf(x, table[t + i]);
+    x = group_max(x);
+    if (sub == l) m = x;
+  }
+  return m;
+}
 
 // Per-channel majorant of one cell, renderer.cu:159-203 (the texel-interval
-// max plus the two extra lerp lookups at addr + 0.5). at_texel[i]: the channel's
-// opacity looked up at texel i, (i + 0.5) / n.
-__device__ __forceinline__ float channel_majorant(const float* at_texel, const float4* tab, int n,
+// max plus the two extra lerp lookups at addr + 0.5). at_texel[at + i]: the channel's
+// opacity looked up at texel i, (i + 0.5) / n; 0 without any (an empty range).
+template <bool SPREAD>
+__device__ __forceinline__ float channel_majorant(const float* at_texel, int at, const float4* tab, int n,
                                                   float os, float xlo, float xhi, float vlo, float vhi,
-                                                  float mn, float mx, int sub) {
+                                                  float mn, float mx, bool any) {
   const float remappedMin1 = (mn - vlo) / (vhi - vlo);
   const float remappedMin = (remappedMin1 - xlo) / (xhi - xlo);
   const float remappedMax1 = (mx - vlo) / (vhi - vlo);
@@ -319,9 +358,8 @@ __device__ __forceinline__ float channel_majorant(const float* at_texel, const f
   const float addr2 = remappedMax * float(n);
   const int addrMin = clamp_index(fminf(floorf(addr1), floorf(addr2)), n);
   const int addrMax = clamp_index(fmaxf(ceilf(addr1), ceilf(addr2)), n);
-  float m = 0.f;
-  for (int i = addrMin + sub; i <= addrMax; i += kMajLanes) m = fmaxf(m, at_texel[i]);
-  m = group_max(m);
+  float m = interval_max<SPREAD>(at_texel, at, addrMin, any ? addrMax : addrMin - 1);
+  if (!any) return 0.f;
   float d = tf_lerp_alpha(tab, n, (addr1 + 0.5f) / float(n)) * os;
   m = fmaxf(m, d);
   d = tf_lerp_alpha(tab, n, (addr2 + 0.5f) / float(n)) * os;
@@ -335,25 +373,27 @@ __device__ __forceinline__ float channel_majorant(const float* at_texel, const f
 // lookup interval is widened by 2^-12 (1 + |r|) on each side, which covers the
 // render's remap by reciprocals against the divisions here, and the maximum
 // is scaled by 1 + 2^-20 for the lerp's rounding. A lookup at u reads
-// texels floor(u n - 0.5) and the next one, clamped to the table. texel[i]: the
+// texels floor(u n - 0.5) and the next one, clamped to the table. texel[at + i]: the
 // channel's stored opacity.
-__device__ __forceinline__ float channel_majorant_conservative(const float* texel, int n, float os,
+template <bool SPREAD>
+__device__ __forceinline__ float channel_majorant_conservative(const float* texel, int at, int n, float os,
                                                                float xlo, float xhi, float vlo,
-                                                               float vhi, float mn, float mx, int sub) {
+                                                               float vhi, float mn, float mx, bool any) {
   const float r1 = ((mn - vlo) / (vhi - vlo) - xlo) / (xhi - xlo);
   const float r2 = ((mx - vlo) / (vhi - vlo) - xlo) / (xhi - xlo);
   const float a = fminf(r1, r2), b = fmaxf(r1, r2);
   const float lo = a - 0x1p-12f * (1.0f + fabsf(a)), hi = b + 0x1p-12f * (1.0f + fabsf(b));
   const int i0 = clamp_index(floorf(lo * float(n) - 0.5f), n);
   const int i1 = clamp_index_plus1(floorf(hi * float(n) - 0.5f), n);
-  float m = 0.f;
-  for (int i = i0 + sub; i <= i1; i += kMajLanes) m = fmaxf(m, texel[i]);
-  return group_max(m) * os * (1.0f + 0x1p-20f);
+  const float m = interval_max<SPREAD>(texel, at, i0, any ? i1 : i0 - 1);
+  return any ? m * os * (1.0f + 0x1p-20f) : 0.f;
 }
 
 // renderer.cu:206-274: modes 0-2 keep one majorant per (cell, channel)
 // (renderer.cu:159-203), modes 3-9 their sum per cell (renderer.cu:111-157).
-// A group of kMajLanes lanes per entry; workgroups stride over the entries.
+// A group of kMajLanes lanes (SPREAD) or a lane per entry; workgroups stride over
+// the entries.
+template <bool SPREAD>
 __global__ __launch_bounds__(256) void majorant_kernel(MajorantParams P) {
   extern __shared__ float s_texel[];  // [channel][stride]
   const int C = P.channels, stride = P.tf.stride;
@@ -369,27 +409,29 @@ __global__ __launch_bounds__(256) void majorant_kernel(MajorantParams P) {
     s_texel[k] = v;
   }
   __syncthreads();
-  const int sub = threadIdx.x % kMajLanes;
-  auto majorant = [&](const float2 r, int c) {
-    if (r.y < r.x) return 0.f;
+  auto majorant = [&](const float2 r, int c, bool any) {
+    any = any && !(r.y < r.x);
+    const int at = c * stride;
     return P.conservative
-               ? channel_majorant_conservative(s_texel + c * stride, P.tf.n[c], P.tf.opacity[c],
-                                               P.tf.xf_lo[c], P.tf.xf_hi[c], P.tf.dom_lo[c],
-                                               P.tf.dom_hi[c], r.x, r.y, sub)
-               : channel_majorant(s_texel + c * stride, tab + size_t(c) * stride, P.tf.n[c],
-                                  P.tf.opacity[c], P.tf.xf_lo[c], P.tf.xf_hi[c], P.tf.dom_lo[c],
-                                  P.tf.dom_hi[c], r.x, r.y, sub);
+               ? channel_majorant_conservative<SPREAD>(s_texel, at, P.tf.n[c], P.tf.opacity[c], P.tf.xf_lo[c],
+                                                       P.tf.xf_hi[c], P.tf.dom_lo[c], P.tf.dom_hi[c], r.x, r.y, any)
+               : channel_majorant<SPREAD>(s_texel, at, tab + size_t(c) * stride, P.tf.n[c], P.tf.opacity[c],
+                                          P.tf.xf_lo[c], P.tf.xf_hi[c], P.tf.dom_lo[c], P.tf.dom_hi[c], r.x, r.y,
+                                          any);
   };
   const int entries = P.mode <= 2 ? P.n_cells * C : P.n_cells;
-  const int step = int(gridDim.x) * (256 / kMajLanes);
-  for (int i = int(blockIdx.x) * (256 / kMajLanes) + int(threadIdx.x) / kMajLanes; i < entries; i += step) {
+  constexpr int kLanes = SPREAD ? kMajLanes : 1, kPer = 256 / kLanes;
+  const int own = int(threadIdx.x) / kLanes;
+  for (int i0 = int(blockIdx.x) * kPer; i0 < entries; i0 += int(gridDim.x) * kPer) {
+    const bool any = i0 + own < entries;
+    const int i = any ? i0 + own : 0;
     float m = 0.f;
     if (P.mode <= 2) {
-      m = majorant(rg[i], i % C);
+      m = majorant(rg[i], i % C, any);
     } else {
-      for (int c = 0; c < C; ++c) m += majorant(rg[size_t(i) * C + c], c);
+      for (int c = 0; c < C; ++c) m += majorant(rg[size_t(i) * C + c], c, any);
     }
-    if (sub == 0) P.maj[i] = m;
+    if (any && threadIdx.x % kLanes == 0) P.maj[i] = m;
   }
 }
 
@@ -611,10 +653,12 @@ hipError_t launch_joint(const VolumeParams& v, int dtype, hipStream_t s) {
 
 hipError_t launch_majorants(const MajorantParams& p, hipStream_t s) {
   const int work = p.mode <= 2 ? p.n_cells * p.channels : p.n_cells;
-  const int per = 256 / kMajLanes, blocks = std::min((work + per - 1) / per, 2048);
+  const bool spread = work <= spread_entries(p.tf.stride);
+  const int per = spread ? 256 / kMajLanes : 256, blocks = std::min((work + per - 1) / per, 2048);
   // at most kMaxTexelsLds floats (40 KiB)
   const size_t lds = size_t(p.channels) * size_t(p.tf.stride) * sizeof(float);
-  hipLaunchKernelGGL(majorant_kernel, dim3(unsigned(blocks)), dim3(256), lds, s, p);
+  hipLaunchKernelGGL(spread ? majorant_kernel<true> : majorant_kernel<false>, dim3(unsigned(blocks)), dim3(256), lds,
+                     s, p);
   return hipGetLastError();
 }
 
