@@ -297,10 +297,9 @@ hipError_t copy(bool to_host, void* host, void* dev, size_t bytes, int device, h
       return e;
     }
   }
-  hipError_t e = to_host ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s)
-                         : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  return e;
+  if (!to_host) return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+  const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
+  return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
 
 }  // namespace
