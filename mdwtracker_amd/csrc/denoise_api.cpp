@@ -113,7 +113,8 @@ constexpr float kInitSigma = 1.5f;
 // floats of partial weight gradients (48 MiB): at least 9 * cout * cin + cout of
 // every layer, and room for enough workgroups to fill the GPU
 constexpr size_t kWgradPart = size_t(12) << 20;
-// pixels of one training batch on the device (3 GB); larger batches go in parts
+// pixels of one training batch on the device (968 bytes each: about 1 GB); larger
+// batches go in parts, of one image at least
 constexpr size_t kTrainPixels = size_t(1) << 20;
 
 int setup(mdwt_denoiser* d, uint32_t seed) {

@@ -13,8 +13,13 @@
 
 namespace mdwt {
 
-// A handle that copies holds a reference while it lives; the rings and their
-// threads are given back with the last one.
+// Kernels and host threads take turns on a ring's slots, each after the other's
+// event: the memory is coherent and the events release to the system, and the
+// protocol needs both. A lane is one ring with its events and threads; a device has
+// at most four.
+//
+// A handle that copies holds a reference while it lives; the lanes are given back with
+// the last one.
 void host_copy_acquire();
 void host_copy_release();
 

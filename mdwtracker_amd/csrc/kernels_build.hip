@@ -37,7 +37,7 @@ __host__ __device__ constexpr int voxel_bytes() {
   return DT == MDWT_DT_U8 ? 1 : DT == MDWT_DT_F32 ? 4 : 2;
 }
 // Voxel e of a little-endian dword holding 4 / voxel_bytes voxels, as
-// fetch_raw would convert it.
+// voxel_value would convert it.
 template <int DT>
 __device__ __forceinline__ float word_voxel(uint32_t w, int e) {
   if constexpr (DT == MDWT_DT_U8) return float((w >> (8 * e)) & 0xffu);

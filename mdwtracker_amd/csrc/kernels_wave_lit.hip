@@ -7,7 +7,7 @@
 // 1024^2 on four 256^3 u8 channels with both (-m 2), a frame was 745 us on the
 // thread-per-pixel kernel (23% of lanes active) and is about 250 us here. The
 // denoiser's buffers need no instance of their own: a wave writes them after
-// the sample is composited (64 frames of 512^2: 9.2 -> 3.6 ms; plain frames
+// the sample is composited (64 frames of 512^2: 9.9 -> 4.4 ms; plain frames
 // unchanged).
 #include "wave_paths.hpp"
 

@@ -140,9 +140,10 @@ struct WaveLds {
 __device__ __forceinline__ uint32_t lane_rank(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
 }
-// Orders the wave's LDS accesses across a phase boundary (lanes read what
-// other lanes of the same wave wrote; the waves of a workgroup never share
-// LDS, so no workgroup barrier is needed or allowed: they loop independently).
+// Orders the wave's LDS accesses across a phase boundary: lanes read what other
+// lanes of the same wave wrote. Within a draw the waves of a workgroup share no LDS
+// and loop independently, so no workgroup barrier is needed or allowed there; only
+// the several-frame kernels exchange between draws, at team_quad's own barriers.
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -864,8 +865,8 @@ __device__ __forceinline__ void wave_team_quad(const RenderParams& P, const Ctx<
 #define MDWT_WAVE_KERNEL \
   __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 
-// Per-workgroup set-up: the opacity table and channel parameters in LDS (the
-// only workgroup barrier: the waves run independently from here) and the
+// Per-workgroup set-up: the opacity table and channel parameters in LDS (behind a
+// workgroup barrier; the waves trace independently from here) and the
 // per-wave LDS. The per-wave LDS is static, sized for a 256-thread block (with
 // a dynamic array behind the opacity table the frame ran 15% slower); smaller
 // blocks leave part of it unused.
